@@ -71,6 +71,7 @@ struct C2SBuffers {
     void * conv2;     // [8 rows, out] (bf16 only; fp32 writes y directly)
     float * skip;     // [8 rows, C / 8]
     int64_t * m_dev;  // child count
+    int64_t * info;   // child_lists: list starts and child count
     void * c2s_ws;
     MapBuffers map1;
     MapBuffers map2;
@@ -86,12 +87,14 @@ C2SBuffers carve_c2s(Carver & c, int dtype, int64_t rows, int channels, int out_
     C2SBuffers b{};
     b.pred = static_cast<float *>(c.take(r * 8 * 4));
     b.norm = c.take(r * C * e);
-    b.packed = c.take(r * 8 * O * e);
+    // The packed children, or (one at a time) the lists of the kept ones.
+    b.packed = c.take(std::max(r * 8 * O * e, child_lists_bytes(static_cast<int64_t>(r), 1)));
     b.hidden = c.take(8 * r * O * e);
     b.hnorm = c.take(8 * r * O * e);
     b.conv2 = dtype == PXS_BF16 ? c.take(8 * r * O * e) : nullptr;
     b.skip = static_cast<float *>(c.take(8 * r * (C / 8) * 4));
     b.m_dev = static_cast<int64_t *>(c.take(sizeof(int64_t)));
+    b.info = static_cast<int64_t *>(c.take(10 * sizeof(int64_t)));
     b.c2s_ws = c.take(pxs_channel_to_spatial_workspace_bytes(rows, 2));
     if (own_in) b.map1 = carve_map(c, rows);
     if (own_out) b.map2 = carve_map(c, 8 * std::max<int64_t>(rows, 1));
@@ -279,19 +282,38 @@ static int resblock_c2s(int dtype, const int32_t * coords, int64_t rows, const f
                            b.norm, stream));
     PXS_TRY(pxs_activation(dtype, b.norm, rows * channels, PXS_ACT_SILU, stream));
     if (!in_map) PXS_TRY(build_map(coords, rows, map1, stream));
-    PXS_TRY(pxs_subm_conv3d(dtype, b.norm, rows, channels, w->conv1_weight, w->conv1_bias,
-                            packed_ch, map1.nbr, map1.masks, b.packed, stream));
-    PXS_TRY(pxs_channel_to_spatial(dtype, coords, rows, b.packed, packed_ch, 2, selected,
-                                   out_coords, b.hidden, b.m_dev, b.c2s_ws, stream));
-    // The skip path subdivides the fp32 input with the same selection; its
-    // coordinates are identical, so they land in out_coords again.
-    PXS_TRY(pxs_channel_to_spatial(PXS_F32, coords, rows, x, channels, 2, selected, out_coords,
-                                   b.skip, b.m_dev, b.c2s_ws, stream));
+    // With a subdivision, about half the children are dropped: the bf16
+    // convolution then runs over the kept ones only, once their count is known.
+    const int group = selected && dtype == PXS_BF16
+                          ? child_conv_group(channels, out_channels, w->conv1_weight)
+                          : 0;
     int64_t m = 8 * rows;
-    if (selected) {
-        PXS_TRY(check_hip(hipMemcpyAsync(&m, b.m_dev, sizeof(m), hipMemcpyDeviceToHost, s),
+    if (group > 0) {
+        PXS_TRY(pxs_channel_to_spatial(PXS_F32, coords, rows, x, channels, 2, selected, out_coords,
+                                       b.skip, b.m_dev, b.c2s_ws, stream));
+        const void * entries = nullptr;
+        PXS_TRY(child_lists(selected, rows, group, b.c2s_ws, b.m_dev, b.packed, &entries, b.info, s));
+        int64_t info[10];
+        PXS_TRY(check_hip(hipMemcpyAsync(info, b.info, sizeof(info), hipMemcpyDeviceToHost, s),
                           "pxs_resblock_c2s: read child count"));
         PXS_TRY(check_hip(hipStreamSynchronize(s), "pxs_resblock_c2s: read child count"));
+        m = info[9];
+        PXS_TRY(child_conv(b.norm, rows, channels, w->conv1_weight, w->conv1_bias, out_channels,
+                           group, map1.nbr, map1.masks, entries, info, b.hidden, s));
+    } else {
+        PXS_TRY(pxs_subm_conv3d(dtype, b.norm, rows, channels, w->conv1_weight, w->conv1_bias,
+                                packed_ch, map1.nbr, map1.masks, b.packed, stream));
+        PXS_TRY(pxs_channel_to_spatial(dtype, coords, rows, b.packed, packed_ch, 2, selected,
+                                       out_coords, b.hidden, b.m_dev, b.c2s_ws, stream));
+        // The skip path subdivides the fp32 input with the same selection;
+        // its coordinates are identical, so they land in out_coords again.
+        PXS_TRY(pxs_channel_to_spatial(PXS_F32, coords, rows, x, channels, 2, selected, out_coords,
+                                       b.skip, b.m_dev, b.c2s_ws, stream));
+        if (selected) {
+            PXS_TRY(check_hip(hipMemcpyAsync(&m, b.m_dev, sizeof(m), hipMemcpyDeviceToHost, s),
+                              "pxs_resblock_c2s: read child count"));
+            PXS_TRY(check_hip(hipStreamSynchronize(s), "pxs_resblock_c2s: read child count"));
+        }
     }
     *rows_out = m;
     if (m == 0) return PXS_OK;

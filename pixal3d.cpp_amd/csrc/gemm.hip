@@ -22,6 +22,7 @@
 #include "s2emit.h"
 #include "scan.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace pxs {
@@ -546,14 +547,73 @@ __device__ __forceinline__ void spin_until(const uint32_t * flag, uint32_t gen, 
     atomicOr(error, 1u);
 }
 
+// SubMConv3d of a channel-to-spatial up-block, kept children only
+// (child_conv).  The children c = g * group .. of list g share its output
+// columns [c * out, (c + 1) * out); the list holds the parent rows that keep
+// at least one of them, and a tile covers up to BM consecutive list entries of
+// one list, so the columns of dropped children cost nothing where a list's
+// parents all drop them.  Kept children's features go straight to their rows
+// of the subdivided tensor.
+struct ChildArgs {
+    const int4 * entries;  // (parent row, first child's output row, kept children, 0)
+    int lists;             // 8 / group
+    int group;             // children per list
+    int out;               // columns per child
+    int start[9];          // list g is entries[start[g], start[g + 1])
+    int tile[9];           // first row tile of list g
+};
+
+// Store epilogue of child_conv through LDS, as gemm_epilogue_staged, with
+// each 16-byte piece (8 columns, all of one child) going to its child's row
+// if the parent keeps that child.
+template <int BM, int BN, int TI, int TJ, int WM, int WN, int NT>
+__device__ __forceinline__ void child_epilogue(const GemmArgs & a, const ChildArgs & c, int list,
+                                               const int4 * rows, const f32x16 (&acc)[TI][TJ],
+                                               char * stage, int live, int n0, int row0, int wm,
+                                               int wn, int h, int r, int tid) {
+    constexpr int kPitch = BN * 2 + 16;
+    const int cols = c.group * c.out;
+    const int col0 = list * cols;
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            const int cl = wn * WN + j * 32 + r;
+            const float b = (a.bias && n0 + cl < cols) ? a.bias[col0 + n0 + cl] : 0.0f;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int rl = row0 + wm * WM + i * 32 + 8 * (v >> 2) + 4 * h + (v & 3);
+                *reinterpret_cast<uint16_t *>(stage + rl * kPitch + cl * 2) = f32_to_bf16(acc[i][j][v] + b);
+            }
+        }
+    barrier_no_fence();
+    uint16_t * y = static_cast<uint16_t *>(a.y);
+    for (int q = tid; q < BM * (BN / 8); q += NT) {
+        const int rl = q / (BN / 8), piece = q % (BN / 8);
+        const int col = n0 + piece * 8;
+        if (rl >= live || col >= cols) continue;
+        const int4 e = rows[rl];
+        const int sub = col / c.out;
+        const uint32_t bit = 1u << (list * c.group + sub);
+        const uint32_t kept = static_cast<uint32_t>(e.z);
+        if (!(kept & bit)) continue;
+        const int64_t row = e.y + __popc(kept & (bit - 1u));
+        *reinterpret_cast<uint4 *>(y + row * c.out + (col - sub * c.out)) =
+            *reinterpret_cast<const uint4 *>(stage + rl * kPitch + piece * 16);
+    }
+}
+
 // NW waves per workgroup in KSPLIT groups; the waves of a group form a
 // WAVES_M x (NW / KSPLIT / WAVES_M) grid, each owning a block of the output
 // tile.  With KSPLIT = 2 the two groups take alternate 16-element K steps
 // of every stage and add their partial sums once at the end: 8 waves of
 // 64x64 blocks read each LDS fragment for two MFMAs instead of 1.5.
-template <typename T, int BM, int BN, int EPI, int NSTAGE, int NW, int WAVES_M, int KSPLIT, bool SYNC>
+// CHILD: the tile's rows are entries of a child list (ChildArgs) instead of
+// consecutive output rows.
+template <typename T, int BM, int BN, int EPI, int NSTAGE, int NW, int WAVES_M, int KSPLIT, bool SYNC,
+          bool CHILD = false>
 __device__ __forceinline__ void gemm_lds_tile(const GemmArgs & a, int logical, const TileSync & sync,
-                                              char * smem) {
+                                              char * smem, const ChildArgs * child = nullptr) {
     constexpr int kVec = Mfma<T>::kVec;
     constexpr int kChunk = Mfma<T>::kChunk;
     constexpr int kThreads = NW * 64;
@@ -582,9 +642,28 @@ __device__ __forceinline__ void gemm_lds_tile(const GemmArgs & a, int logical, c
     const int wm = wl / WAVES_N, wn = wl % WAVES_N;
     const int h = lane >> 5, r = lane & 31;
 
-    const int tiles_n = (a.cout + BN - 1) / BN;
-    const int64_t p0 = static_cast<int64_t>(logical / tiles_n) * BM;
+    // Columns of this tile's product, the first of them in W and bias, and
+    // the end of its rows.
+    int cols = a.cout, col0 = 0, list = 0;
+    if constexpr (CHILD) cols = child->group * child->out;
+    const int tiles_n = (cols + BN - 1) / BN;
+    int64_t p0 = static_cast<int64_t>(logical / tiles_n) * BM, p_end = a.m;
     const int n0 = (logical % tiles_n) * BN;
+    [[maybe_unused]] __shared__ int4 child_rows[CHILD ? BM : 1];
+    if constexpr (CHILD) {
+        const int rt = logical / tiles_n;
+        while (list + 1 < child->lists && rt >= child->tile[list + 1]) ++list;
+        p0 = child->start[list] + static_cast<int64_t>(rt - child->tile[list]) * BM;
+        p_end = child->start[list + 1];
+        col0 = list * cols;
+        for (int row = tid; row < BM; row += kThreads)
+            if (p0 + row < p_end) child_rows[row] = child->entries[p0 + row];
+    }
+    // Output row (of the convolution over the parents) of tile row `row`.
+    auto row_of = [&](int row) -> int64_t {
+        if constexpr (CHILD) return child_rows[row].x;
+        return p0 + row;
+    };
     const T * __restrict__ x = static_cast<const T *>(a.x);
     const T * __restrict__ w = static_cast<const T *>(a.w);
 
@@ -609,7 +688,7 @@ __device__ __forceinline__ void gemm_lds_tile(const GemmArgs & a, int logical, c
         for (int e = tid; e < a.noff * BM; e += kThreads) {
             const int k = e / BM, row = e % BM;
             int32_t src = -1;
-            if (p0 + row < a.m) {
+            if (p0 + row < p_end) {
                 const int32_t * q = a.rowmap + k * a.ld_map + p0 + row;
                 int32_t s;
                 if constexpr (SYNC) {
@@ -628,8 +707,8 @@ __device__ __forceinline__ void gemm_lds_tile(const GemmArgs & a, int logical, c
     } else {
         uint32_t local = 0;
         for (int row = tid; row < BM; row += kThreads) {
-            if (p0 + row >= a.m) break;
-            const int64_t p = p0 + row;
+            if (p0 + row >= p_end) break;
+            const int64_t p = row_of(row);
             if (a.masks) {
                 local |= a.masks[p];
             } else if (a.rowmap) {
@@ -659,8 +738,8 @@ __device__ __forceinline__ void gemm_lds_tile(const GemmArgs & a, int logical, c
     for (int e = tid; !full_table && e < kcount * BM; e += kThreads) {
         const int i = e / BM, row = e % BM;
         int32_t src = -1;
-        if (p0 + row < a.m) {
-            const int64_t p = p0 + row;
+        if (p0 + row < p_end) {
+            const int64_t p = row_of(row);
             const int64_t s = a.rowmap ? static_cast<int64_t>(a.rowmap[koff[i] * a.ld_map + p]) : p;
             src = (s >= 0 && s < a.rows_in) ? static_cast<int32_t>(s) : -1;
         }
@@ -724,8 +803,8 @@ __device__ __forceinline__ void gemm_lds_tile(const GemmArgs & a, int logical, c
     for (int j = 0; j < BI; ++j) {
         const int row = (wave * BI + j) * 8 + lrow;
         b_piece[j] = lslot ^ swz(row);
-        b_ok[j] = n0 + row < a.cout;
-        b_off[j] = static_cast<int64_t>(n0 + row) * a.cin + b_piece[j] * kVec;
+        b_ok[j] = n0 + row < cols;
+        b_off[j] = static_cast<int64_t>(col0 + n0 + row) * a.cin + b_piece[j] * kVec;
     }
 
     auto issue = [&](int s) {
@@ -864,7 +943,15 @@ __device__ __forceinline__ void gemm_lds_tile(const GemmArgs & a, int logical, c
     const bool staged = kStageable && a.cout % 8 == 0 && a.ldy % 8 == 0 &&
                         (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
     if constexpr (KSPLIT == 1) {
-        if (kStageable && staged) {
+        if constexpr (CHILD) {
+            // The staged tile may reach into the source table, which no wave
+            // reads any more.
+            static_assert(BM * kStagedPitch <= lds_gemm_bytes<BM, BN, NSTAGE>(27), "staged tile");
+            barrier_no_fence();
+            child_epilogue<BM, BN, TI, TJ, WM, WN, kThreads>(
+                a, *child, list, child_rows, acc, smem,
+                static_cast<int>(min<int64_t>(BM, p_end - p0)), n0, 0, wm, wn, h, r, tid);
+        } else if (kStageable && staged) {
             barrier_no_fence();  // every wave is done reading the stage buffers
             if (SYNC && coherent_y)
                 gemm_epilogue_staged<BM, BN, TI, TJ, WM, WN, kThreads, true>(a, acc, smem, p0, n0, 0, wm, wn,
@@ -917,7 +1004,12 @@ __device__ __forceinline__ void gemm_lds_tile(const GemmArgs & a, int logical, c
                             fin[i][pass * TJP + j][v] =
                                 acc[KEEP + i][pass * TJP + j][v] + xch[slot(1 - kg, i, j, v)];
             }
-            if (kStageable && staged) {
+            if constexpr (CHILD) {
+                barrier_no_fence();  // the partner's sums are read: the exchange area is free
+                child_epilogue<BM, BN, HI, TJ, WM, WN, kThreads>(
+                    a, *child, list, child_rows, fin, smem,
+                    static_cast<int>(min<int64_t>(BM, p_end - p0)), n0, KEEP * 32, wm, wn, h, r, tid);
+            } else if (kStageable && staged) {
                 // A producer of the chained launch writes whole 16-byte
                 // pieces device-coherently (2-byte write-through stores would
                 // each go to memory on their own).
@@ -964,6 +1056,14 @@ gather_gemm_lds_kernel(GemmArgs a) {
     }
     gemm_lds_tile<T, BM, BN, EPI, NSTAGE, NW, WAVES_M, KSPLIT, false>(
         a, remap_xcd(blockIdx.x, tiles), TileSync{}, smem);
+}
+
+template <int BM, int BN, int NW, int WAVES_M, int KSPLIT>
+__global__ void __launch_bounds__(NW * 64)
+child_conv_kernel(GemmArgs a, ChildArgs c) {
+    extern __shared__ __align__(16) char smem[];
+    gemm_lds_tile<uint16_t, BM, BN, kEpiStore, 2, NW, WAVES_M, KSPLIT, false, true>(
+        a, remap_xcd(blockIdx.x, gridDim.x), TileSync{}, smem, &c);
 }
 
 // One U-Net level in one launch (pxs_unet_s2_level): workgroups [0, tiles_a)
@@ -1816,6 +1916,27 @@ int launch_lds_tile(const GemmArgs & args, hipStream_t stream) {
     return check_launch("gather GEMM (LDS pipeline)");
 }
 
+template <int BM, int BN, int NW, int WAVES_M, int KSPLIT>
+int launch_child_conv(const GemmArgs & args, ChildArgs c, hipStream_t stream) {
+    constexpr int smem = lds_gemm_bytes<BM, BN, 2>(27);
+    static bool configured = false;
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(
+            reinterpret_cast<const void *>(&child_conv_kernel<BM, BN, NW, WAVES_M, KSPLIT>),
+            hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+        if (e != hipSuccess) return check_hip(e, "hipFuncSetAttribute(child_conv)");
+        configured = true;
+    }
+    c.tile[0] = 0;
+    for (int g = 0; g < c.lists; ++g) c.tile[g + 1] = c.tile[g] + (c.start[g + 1] - c.start[g] + BM - 1) / BM;
+    const int64_t blocks = static_cast<int64_t>(c.tile[c.lists]) * ((c.group * c.out + BN - 1) / BN);
+    if (blocks > INT32_MAX) return fail(PXS_ERR_ARG, "gather GEMM grid too large");
+    if (blocks == 0) return PXS_OK;
+    hipLaunchKernelGGL((child_conv_kernel<BM, BN, NW, WAVES_M, KSPLIT>),
+                       dim3(static_cast<unsigned>(blocks)), dim3(NW * 64), smem, stream, args, c);
+    return check_launch("child convolution");
+}
+
 // The chained level runs the default bf16 tile of both convolutions
 // (128 x 128, 2 stages, 8 waves in two K groups), the one dispatch picks for
 // them.
@@ -2157,6 +2278,55 @@ int linear_rows(int dtype, const void * x, int64_t rows, int cin, const void * w
     a.cout = cout; a.m = rows; a.rowmap = nullptr; a.ld_map = 0; a.noff = 1; a.masks = nullptr;
     a.y = y; a.ldy = cout; a.act = act;
     return run_gemm(dtype, a, kEpiStore, s);
+}
+
+// Children per list: as many as fill 256 columns, which a tile's gathered
+// rows then feed at once.  Measured over the decoder's up-blocks (10,624 to
+// 662k parents, 47-54% of the children kept; child_conv against all children
+// on 256 x 256 tiles and the copy of the kept ones): 512 columns a child, one
+// per list, 1.12 against 2.34 ms; 256, one per list, 1.2 ms less; 128, two per
+// list, 1.0 ms less (one per list on 128 x 128 tiles the same); 64, four per
+// list, 0.9 ms less (two per list on 128 x 128 tiles the same, one per list
+// on 128 x 64 tiles 0.5 ms less).  Widths that leave a quarter or more of a
+// 64-column step empty, or are narrower than 64, stay on the all-children
+// convolution.
+int child_conv_group(int channels, int out, const void * weight) {
+    if (channels % 8 != 0 || out % 64 != 0 || !aligned16(weight)) return 0;
+    return out > 128 ? 1 : (out == 128 ? 2 : 4);
+}
+
+int child_conv(const void * x, int64_t n, int channels, const void * weight, const float * bias,
+               int out, int group, const int32_t * nbr, const uint32_t * masks,
+               const void * entries, const int64_t * start, void * y, hipStream_t s) {
+    GemmArgs a{};
+    a.x = x; a.rows_in = n; a.ldx = channels; a.cin = channels; a.w = weight; a.bias = bias;
+    a.cout = 8 * out; a.m = n; a.rowmap = nbr; a.ld_map = n; a.noff = 27; a.masks = masks;
+    a.y = y; a.ldy = out; a.act = PXS_ACT_NONE; a.vec_ok = 1;
+    ChildArgs c{};
+    c.entries = static_cast<const int4 *>(entries);
+    c.lists = 8 / group;
+    c.group = group;
+    c.out = out;
+    for (int g = 0; g <= c.lists; ++g) c.start[g] = static_cast<int>(start[g]);
+    // The tile that gives the shortest last round: tiles per CU (rounded up)
+    // times the tile's time, in 256 x 256 tiles.  192 x 256 and 256 x 256
+    // tiles run at the same rate (46k rows of 512 columns: 1.12 ms on
+    // 496 of the former, 1.50 on 368 of the latter, 256 CUs; with 174k rows of
+    // 256 columns both 1.1 ms), the smaller ones at 0.78 of it.
+    const int cols = group * out;
+    auto cost = [&](int bm, int bn, double time) {
+        int64_t tiles = 0;
+        for (int g = 0; g < c.lists; ++g) tiles += (c.start[g + 1] - c.start[g] + bm - 1) / bm;
+        tiles *= (cols + bn - 1) / bn;
+        return static_cast<double>((tiles + 255) / 256) * time;
+    };
+    const double t256 = cost(256, 256, 1.0), t192 = cost(192, 256, 0.75);
+    const double t128 = cost(128, 256, 0.5 / 0.78), tsq = cost(128, 128, 0.25 / 0.78);
+    const double best = std::min(std::min(t256, t192), std::min(t128, tsq));
+    if (t256 <= best) return launch_child_conv<256, 256, 16, 4, 1>(a, c, s);
+    if (t192 <= best) return launch_child_conv<192, 256, 8, 2, 1>(a, c, s);
+    if (t128 <= best) return launch_child_conv<128, 256, 8, 2, 1>(a, c, s);
+    return launch_child_conv<128, 128, 8, 2, 2>(a, c, s);
 }
 
 } // namespace pxs

@@ -36,6 +36,26 @@ int dense_linear_gate(int dtype, const void * x, int64_t rows, int cin, const vo
                       const float * block_mod, const float * time_mod, int gate_offset,
                       float * residual, hipStream_t s, bool * done);
 
+// The C -> 8 out SubMConv3d of a channel-to-spatial up-block with a
+// subdivision, bf16, computed for the kept children only and written straight
+// to their rows (csrc/gemm.hip; the lists come from csrc/topology.hip).
+//   child_conv_group: children per list for these widths, 0 when the
+//     convolution should be run over all children instead.
+//   child_lists: after pxs_channel_to_spatial (factor 2) with the same
+//     subdivision and workspace.  *entries (in ws, child_lists_bytes) lists
+//     per group of children the rows that keep any of them; info (device, 10
+//     values) = start of each list, end of the last, and at [9] the child
+//     count m.
+//   child_conv: start = info on the host; y [m, out].
+int child_conv_group(int channels, int out, const void * weight);
+size_t child_lists_bytes(int64_t n, int group);
+int child_lists(const float * subdivision, int64_t n, int group, const void * c2s_ws,
+                const int64_t * m_dev, void * ws, const void ** entries, int64_t * info,
+                hipStream_t s);
+int child_conv(const void * x, int64_t n, int channels, const void * weight, const float * bias,
+               int out, int group, const int32_t * nbr, const uint32_t * masks,
+               const void * entries, const int64_t * start, void * y, hipStream_t s);
+
 #define PXS_CHECK(expr, code, msg)            \
     do {                                      \
         if (!(expr)) return ::pxs::fail((code), (msg)); \

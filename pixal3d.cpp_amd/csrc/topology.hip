@@ -7,6 +7,7 @@
 
 #include "pxs_common.h"
 #include "s2emit.h"
+#include "carve.h"
 #include "scan.h"
 
 #include <algorithm>
@@ -1120,7 +1121,110 @@ __global__ void c2s_feats_kernel(const T * __restrict__ x, int channels, int cc,
     }
 }
 
+// ---- lists of the rows that keep a child, per group of children ----------------
+// One row per thread, kListRows per workgroup; counts[g * blocks + block], so
+// their prefix sums place list g after list g - 1 and rows ascending in it.
+constexpr int kListRows = 1024;
+
+__device__ __forceinline__ uint32_t kept_children(const float * __restrict__ sub, int64_t p) {
+    uint32_t kept = 0;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) kept |= sub[p * 8 + c] > 0.0f ? 1u << c : 0u;
+    return kept;
+}
+
+__global__ void __launch_bounds__(kListRows)
+child_count_kernel(const float * __restrict__ sub, int64_t n, int group, int32_t * __restrict__ counts) {
+    __shared__ int total[8];
+    const int tid = threadIdx.x, lists = 8 / group;
+    const int64_t p = static_cast<int64_t>(blockIdx.x) * kListRows + tid;
+    if (tid < 8) total[tid] = 0;
+    __syncthreads();
+    const uint32_t kept = p < n ? kept_children(sub, p) : 0u;
+    const uint32_t bits = (1u << group) - 1u;
+    for (int g = 0; g < lists; ++g) {
+        const int c = __popcll(__ballot((kept >> (g * group)) & bits));
+        if ((tid & 63) == 0 && c) atomicAdd(&total[g], c);
+    }
+    __syncthreads();
+    if (tid < lists) counts[static_cast<int64_t>(tid) * gridDim.x + blockIdx.x] = total[tid];
+}
+
+__global__ void __launch_bounds__(kListRows)
+child_list_kernel(const float * __restrict__ sub, int64_t n, int group,
+                  const int64_t * __restrict__ first_child, const int64_t * __restrict__ m_dev,
+                  const int64_t * __restrict__ start, int4 * __restrict__ entries,
+                  int64_t * __restrict__ info) {
+    __shared__ int wave_count[8][kListRows / 64];
+    const int tid = threadIdx.x, wave = tid >> 6, lists = 8 / group;
+    const int64_t p = static_cast<int64_t>(blockIdx.x) * kListRows + tid;
+    const uint32_t kept = p < n ? kept_children(sub, p) : 0u;
+    const uint32_t bits = (1u << group) - 1u;
+    for (int g = 0; g < lists; ++g) {
+        const int c = __popcll(__ballot((kept >> (g * group)) & bits));
+        if ((tid & 63) == 0) wave_count[g][wave] = c;
+    }
+    __syncthreads();
+    const int first = kept ? static_cast<int>(first_child[p]) : 0;
+    for (int g = 0; g < lists; ++g) {
+        const bool in = ((kept >> (g * group)) & bits) != 0;
+        const uint64_t lanes = __ballot(in);
+        if (!in) continue;
+        int64_t at = start[static_cast<int64_t>(g) * gridDim.x + blockIdx.x] +
+                     __popcll(lanes & ((1ull << (tid & 63)) - 1ull));
+        for (int w = 0; w < wave; ++w) at += wave_count[g][w];
+        entries[at] = make_int4(static_cast<int>(p), first, static_cast<int>(kept), 0);
+    }
+    if (blockIdx.x == 0) {
+        // start[lists * blocks] is the end of the last list
+        if (tid <= lists) info[tid] = start[static_cast<int64_t>(tid) * gridDim.x];
+        if (tid == 9) info[9] = *m_dev;
+    }
+}
+
+// Workspace of child_lists: entries, then the counts' prefix sums, the counts
+// and the scan's scratch.
+struct ChildListBuffers {
+    int4 * entries;
+    int64_t * start;
+    int32_t * counts;
+    void * scan_ws;
+};
+
+ChildListBuffers carve_child_lists(Carver & c, int64_t n, int group) {
+    const int64_t lists = 8 / group, items = lists * grid_for(n, kListRows);
+    ChildListBuffers b;
+    b.entries = static_cast<int4 *>(c.take(static_cast<size_t>(lists * n) * sizeof(int4)));
+    b.start = static_cast<int64_t *>(c.take(static_cast<size_t>(items + 1) * sizeof(int64_t)));
+    b.counts = static_cast<int32_t *>(c.take(static_cast<size_t>(items) * sizeof(int32_t)));
+    b.scan_ws = c.take(scan_workspace_bytes(items));
+    return b;
+}
+
 } // namespace
+
+size_t child_lists_bytes(int64_t n, int group) {
+    Carver c(nullptr);
+    carve_child_lists(c, n, group);
+    return c.used();
+}
+
+int child_lists(const float * subdivision, int64_t n, int group, const void * c2s_ws,
+                const int64_t * m_dev, void * ws, const void ** entries, int64_t * info,
+                hipStream_t s) {
+    Carver c(ws);
+    const ChildListBuffers b = carve_child_lists(c, n, group);
+    *entries = b.entries;
+    const unsigned blocks = grid_for(n, kListRows);
+    const int64_t items = static_cast<int64_t>(8 / group) * blocks;
+    hipLaunchKernelGGL(child_count_kernel, dim3(blocks), dim3(kListRows), 0, s, subdivision, n,
+                       group, b.counts);
+    if (int rc = exclusive_scan_i32(b.counts, b.start, items, b.start + items, b.scan_ws, s)) return rc;
+    // pxs_channel_to_spatial's workspace begins with each row's first child row
+    hipLaunchKernelGGL(child_list_kernel, dim3(blocks), dim3(kListRows), 0, s, subdivision, n,
+                       group, static_cast<const int64_t *>(c2s_ws), m_dev, b.start, b.entries, info);
+    return check_launch("child lists");
+}
 
 } // namespace pxs
 

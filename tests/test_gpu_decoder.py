@@ -139,6 +139,55 @@ def test_resblock_c2s(px, orc, dtype, mode):
         assert_bf16(host(y), ref_y, what=f"c2s bf16 {mode}")
 
 
+# (rows, channels, children's width, which children are kept).  The kept
+# children's convolution lists 1, 2 or 4 children together by their width, and
+# takes 128 x 128, 128 x 256, 256 x 256 or 192 x 256 tiles by the lists' lengths
+# (about 250, 2,048, 4,096 and 5,779 rows of 512 columns); 96 columns a child
+# stay on the convolution of all children.
+@pytest.mark.parametrize("rows,C,out,kept", [
+    (500, 64, 512, "half"), (4096, 64, 512, "half"), (8192, 64, 512, "half"),
+    (11558, 64, 512, "half"), (700, 128, 64, "half"), (33, 64, 128, "half"), (1, 64, 64, "all"),
+    (129, 64, 192, "all"), (300, 64, 128, "one"), (300, 64, 64, "one"), (300, 64, 64, "none"),
+    (6000, 512, 64, "half"), (300, 64, 96, "half")])
+def test_resblock_c2s_kept_children(px, rows, C, out, kept):
+    """A bf16 up-block with a subdivision against the same block from its
+    single ops (all children convolved, the kept ones copied).  conv1's sums
+    may round differently: at most one bf16 step, 2^-8, of its outputs, which
+    the norm and conv2 pass on at that relative size."""
+    dev = torch.device("cuda:0")
+    coords = ti32(W.shell_coords(64, [[(22.0, 29.0)]], 46)[:rows])
+    assert coords.shape[0] == rows
+    g = torch.Generator(device=dev).manual_seed(rows + out)
+    rnd = lambda *s, std=1.0: torch.randn(*s, generator=g, device=dev) * std  # noqa: E731
+    w = {"norm1_weight": 1.0 + rnd(C, std=0.1), "norm1_bias": rnd(C, std=0.1),
+         "conv1_weight": rnd(27, 8 * out, C, std=(27 * C) ** -0.5).to(torch.bfloat16),
+         "conv1_bias": rnd(8 * out, std=0.1),
+         "conv2_weight": rnd(27, out, out, std=(27 * out) ** -0.5).to(torch.bfloat16),
+         "conv2_bias": rnd(out, std=0.1)}
+    x = rnd(rows, C)
+    sub = {"half": rnd(rows, 8), "all": torch.ones(rows, 8, device=dev),
+           "none": -torch.ones(rows, 8, device=dev)}.get(kept)
+    if sub is None:  # a single child of a single row, the last
+        sub = -torch.ones(rows, 8, device=dev)
+        sub[rows - 1, 7] = 1.0
+    print(f"kept children rows={rows} C={C} out={out} {kept}", flush=True)
+    oc, y, _ = px.resblock_c2s(coords, x, out, 1e-6, pxs.decoder_block_weights(w), pxs.PXS_BF16,
+                               subdivision=sub)
+    silu = 2
+    h = px.activation(px.layer_norm(x, 1e-6, w["norm1_weight"], w["norm1_bias"], torch.bfloat16), silu)
+    packed = px.subm_conv3d(h, w["conv1_weight"], w["conv1_bias"], *px.neighbor_map(coords))
+    ref_c, h = px.channel_to_spatial(coords, packed, sub)
+    _, skip = px.channel_to_spatial(coords, x, sub)
+    assert torch.equal(oc, ref_c)
+    if kept == "none":
+        assert y.shape[0] == 0
+        return
+    h = px.activation(px.layer_norm(h, 1e-6), silu)
+    ref = px.add_repeat(px.subm_conv3d(h, w["conv2_weight"], w["conv2_bias"],
+                                       *px.neighbor_map(ref_c)), skip)
+    assert_bf16(host(y), host(ref), tol=2.0 ** -8, what="kept children")
+
+
 def test_resblock_c2s_zero_conv_is_repeated_skip(px, orc):
     """conv2 = 0 leaves y = repeat_channels(channel_to_spatial(x)) exactly."""
     C, O_ = 32, 16
