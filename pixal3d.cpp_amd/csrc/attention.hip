@@ -1232,6 +1232,188 @@ window_attn_bf16_kernel(AttnArgs a, int heads, int heads_per_group, int groups) 
     }
 }
 
+// fp32, head_dim and value_dim 64, unpermuted rows: 64 queries per workgroup,
+// two waves of 32 queries for each of two key groups.  64-key K and V tiles
+// (16 KB each) stream by LDS DMA into two buffers, the next tile in flight
+// while one is multiplied; key group g takes keys 32 g .. 32 g + 31 of each
+// tile with a running max, sum and output of its own, and the two are merged
+// once at the end.  Rows stay row-major, 16-byte pieces XOR-swizzled: f32_kswz
+// spreads the 16 key rows one 16-byte K read covers over all banks, f32_vswz
+// the two key rows (4 apart) one 4-byte V read covers.
+// Bound by the fp32 matrix cores and the softmax's vector work beside them:
+// 4,600 x 4,600 keys x 16 heads in 0.90 ms, 96 TFLOP/s (1.04 ms with 128
+// queries per workgroup and unsplit keys, whose 592 workgroups leave the CUs
+// 2 or 3 each; the generic kernel, which stages each tile through registers
+// with nothing in flight, took the block it is in from 2.50 to 2.85 ms).
+__device__ __forceinline__ int f32_kswz(int row) { return row & 15; }
+__device__ __forceinline__ int f32_vswz(int row) { return ((row >> 2) & 1) << 3; }
+
+constexpr int kF32Queries = 64;  // queries per workgroup
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+flash_attn_f32_kernel(AttnArgs a, int heads, int64_t tiles_bound) {
+    constexpr int NW = 4;
+    constexpr int kRow = 256, kTile = kKeys * kRow;  // one K or V tile
+    constexpr int kInstr = kTile / (1024 * NW);      // DMA instructions per wave per tile (4 rows each)
+    __shared__ __align__(16) char lds[4 * kTile];    // K, V, K, V
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int qg = wave & 1, kg = wave >> 1;
+    const int h = lane >> 5, r = lane & 31;
+
+    const int64_t logical = remap_xcd64(blockIdx.x, tiles_bound * heads);
+    const int head = static_cast<int>(logical / tiles_bound);
+    const int64_t t = logical - static_cast<int64_t>(head) * tiles_bound;
+    if (t >= a.tile_start[a.nseg]) return;
+    const int seg = find_segment(a.tile_start, a.nseg, t, lane);
+    const int64_t q_begin = a.cu_q[seg] + (t - a.tile_start[seg]) * kF32Queries;
+    const int64_t q_end = a.cu_q[seg + 1];
+    const int64_t k_begin = a.cu_k[seg], k_end = a.cu_k[seg + 1];
+    const float * __restrict__ kp = static_cast<const float *>(a.k) + head * 64;
+    const float * __restrict__ vp = static_cast<const float *>(a.v) + head * 64;
+
+    // This lane's query, dims 32h .. 32h+31.
+    const int64_t qi = q_begin + qg * 32 + r;
+    const bool q_valid = qi < q_end;
+    f32x4 qv[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+        qv[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (q_valid)
+            qv[u] = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(a.q) + qi * a.ldq +
+                                                     head * 64 + 32 * h + 4 * u);
+    }
+
+    const int ntiles = static_cast<int>((k_end - k_begin + kKeys - 1) / kKeys);
+    const int lrow = lane >> 4, lslot = lane & 15;
+    const uint32_t lds_base = lds_offset(&lds[0]);
+    // Tile j into buffer j & 1; rows past the segment come from the zero line.
+    auto issue = [&](int j) __attribute__((always_inline)) {
+        const int64_t key0 = k_begin + static_cast<int64_t>(j) * kKeys;
+#pragma unroll
+        for (int i = 0; i < 2 * kInstr; ++i) {
+            const bool is_v = i >= kInstr;
+            const int row0 = (wave * kInstr + i % kInstr) * 4;
+            const int row = row0 + lrow;
+            const int64_t key = key0 + row;
+            const float * src = is_v ? vp + key * a.ldv + (lslot ^ f32_vswz(row)) * 4
+                                     : kp + key * a.ldk + (lslot ^ f32_kswz(row)) * 4;
+            lds_dma16(key < k_end ? static_cast<const void *>(src) : static_cast<const void *>(g_attn_zero),
+                      lds_base + (j & 1) * 2 * kTile + (is_v ? kTile : 0) + row0 * kRow);
+        }
+    };
+
+    f32x16 oacc[2];
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) oacc[dt][v] = 0.0f;
+    float m_run = -INFINITY, l_run = 0.0f;
+
+    if (ntiles > 0) issue(0);
+    for (int j = 0; j < ntiles; ++j) {
+        wait_vmcnt0();
+        barrier_no_fence();  // tile j has landed; every wave is done with tile j - 1
+        if (j + 1 < ntiles) issue(j + 1);
+        const char * kl = lds + (j & 1) * 2 * kTile + kg * 32 * kRow;
+        const char * vl = kl + kTile;
+
+        // S^T of the group's 32 keys: even and odd dims in two accumulators.
+        f32x16 sacc[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sacc[e][v] = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const f32x4 af = *reinterpret_cast<const f32x4 *>(kl + r * kRow + (((8 * h + u) ^ f32_kswz(r)) << 4));
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                sacc[e & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[e], qv[u][e], sacc[e & 1], 0, 0, 0);
+        }
+
+        // Online softmax (log2 domain).  Register v holds key 8*(v/4) + 4h + v%4.
+        const int64_t left = k_end - (k_begin + static_cast<int64_t>(j) * kKeys + kg * 32);
+        f32x16 p;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) p[v] = (sacc[0][v] + sacc[1][v]) * a.scale_log2;
+        if (left < 32) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                if (8 * (v >> 2) + 4 * h + (v & 3) >= left) p[v] = -INFINITY;
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) mx = fmaxf(mx, p[v]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float m_new = fmaxf(m_run, mx);
+        const float alpha = (m_new == -INFINITY) ? 1.0f : exp2f(m_run - m_new);
+        float rs = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            p[v] = (m_new == -INFINITY) ? 0.0f : exp2f(p[v] - m_new);
+            rs += p[v];
+        }
+        rs += __shfl_xor(rs, 32, 64);
+        l_run = l_run * alpha + rs;
+        m_run = m_new;
+        // 1 for every lane once the maxima have settled
+        if (__ballot(alpha != 1.0f)) {
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) oacc[dt][v] *= alpha;
+        }
+
+        // O^T += V^T P^T.
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = 8 * i + 4 * h + e;
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt) {
+                    const int piece = dt * 8 + (r >> 2);
+                    const float va = *reinterpret_cast<const float *>(
+                        vl + row * kRow + ((piece ^ f32_vswz(row)) << 4) + (r & 3) * 4);
+                    oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(va, p[4 * i + e], oacc[dt], 0, 0, 0);
+                }
+            }
+    }
+
+    // Key group 1 hands its max, sum and output over through the idle tiles.
+    barrier_no_fence();
+    float * xch = reinterpret_cast<float *>(lds) + qg * 34 * 64 + lane;
+    if (kg == 1) {
+        xch[0] = m_run;
+        xch[64] = l_run;
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) xch[(2 + dt * 16 + v) * 64] = oacc[dt][v];
+    }
+    barrier_no_fence();
+    if (kg == 1 || !q_valid) return;
+    const float m1 = xch[0], l1 = xch[64];
+    const float m = fmaxf(m_run, m1);
+    // a group without keys (or with every score -inf) has max -inf and sum 0
+    const float w0 = m_run == -INFINITY ? 0.0f : exp2f(m_run - m);
+    const float w1 = m1 == -INFINITY ? 0.0f : exp2f(m1 - m);
+    const float l = l_run * w0 + l1 * w1;
+    const float inv_l = l > 0.0f ? 1.0f / l : 0.0f;
+    float * op = static_cast<float *>(a.o) + qi * a.ldo + head * 64;
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int d = dt * 32 + 8 * i + 4 * h;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                op[d + e] = (oacc[dt][4 * i + e] * w0 + xch[(2 + dt * 16 + 4 * i + e) * 64] * w1) * inv_l;
+        }
+}
+
 // Segments in the order the short-segment kernel takes them: a counting sort
 // by item count (query passes x key chunks, the same for every head group),
 // costliest class first, empty segments last.  The order within a class is
@@ -1288,6 +1470,14 @@ int launch_attn_bf16(const AttnArgs & args, int64_t total_q, int heads, hipStrea
     hipLaunchKernelGGL((flash_attn_bf16_kernel<NW, DH>), dim3(static_cast<unsigned>(bound * heads)),
                        dim3(NW * 64), 0, stream, args, heads, bound);
     return check_launch("flash attention (bf16)");
+}
+
+int launch_attn_f32(const AttnArgs & args, int64_t total_q, int heads, hipStream_t stream) {
+    const int64_t bound = total_q / kF32Queries + args.nseg + 1;
+    if (bound * heads > INT32_MAX) return fail(PXS_ERR_ARG, "attention grid too large");
+    hipLaunchKernelGGL(flash_attn_f32_kernel, dim3(static_cast<unsigned>(bound * heads)), dim3(256), 0,
+                       stream, args, heads, bound);
+    return check_launch("flash attention (fp32)");
 }
 
 template <typename T, int NW>
@@ -1482,7 +1672,11 @@ int pxs_varlen_attention(int dtype, const void * q, int64_t ld_q, const void * k
     // (windows of ~100 rows run 3.6x faster with 4 waves than with 1).  The
     // generic kernel drops to one wave for short segments.
     const int nw = (fast || fast128 || total_q / nseg >= PXS_ATTN_NW4_MIN) ? 4 : 1;
-    const int q_tile = 32 * nw;
+    const int vec = dtype == PXS_BF16 ? 8 : 4;
+    const bool vec_ok = (head_dim % vec == 0) && (value_dim % vec == 0) && (ld_q % vec == 0) &&
+                        (ld_k % vec == 0) && (ld_v % vec == 0) && aligned16(q) && aligned16(k) && aligned16(v);
+    const bool fast32 = dtype == PXS_F32 && nw == 4 && head_dim == 64 && value_dim == 64 && vec_ok && !row_map;
+    const int q_tile = fast32 ? kF32Queries : 32 * nw;
     int64_t * tile_start = static_cast<int64_t *>(workspace);
     int32_t * tiles = reinterpret_cast<int32_t *>(tile_start + nseg + 1);
     void * scan_ws = reinterpret_cast<void *>(
@@ -1496,15 +1690,14 @@ int pxs_varlen_attention(int dtype, const void * q, int64_t ld_q, const void * k
     a.cu_q = cu_q; a.cu_k = cu_k; a.nseg = nseg; a.tile_start = tile_start;
     a.row_map = row_map; a.hd = head_dim; a.vd = value_dim;
     a.scale_log2 = scale * kLog2e; a.o = o; a.ldo = ld_o;
-    const int vec = dtype == PXS_BF16 ? 8 : 4;
-    a.vec_ok = (head_dim % vec == 0) && (value_dim % vec == 0) && (ld_q % vec == 0) && (ld_k % vec == 0) &&
-               (ld_v % vec == 0) && aligned16(q) && aligned16(k) && aligned16(v);
+    a.vec_ok = vec_ok;
     if (dtype == PXS_BF16) {
         if (fast) return launch_attn_bf16<4, 64>(a, total_q, heads, s);
         if (fast128) return launch_attn_bf16<4, 128>(a, total_q, heads, s);
         return nw == 4 ? launch_attn<uint16_t, 4>(a, total_q, heads, s)
                        : launch_attn<uint16_t, 1>(a, total_q, heads, s);
     }
+    if (fast32) return launch_attn_f32(a, total_q, heads, s);
     return nw == 4 ? launch_attn<float, 4>(a, total_q, heads, s)
                    : launch_attn<float, 1>(a, total_q, heads, s);
 }

@@ -62,6 +62,29 @@ def test_attention_fp32_random(px, orc, lens, heads, hd):
     assert_fp32(o, orc.varlen_attention(q, k, v, cu, cu, heads, hd, np.float32(scale)), what="attn")
 
 
+# fp32 segments of 256 queries and more on average, 64-wide heads: 64-query
+# workgroups whose two key groups take 32 keys each of every 64-key tile.  Key
+# counts at the edges of both (a group without keys, a ragged last tile, none at
+# all), query counts at the edges of the workgroup, scores up to +-40 that
+# come late.
+@pytest.mark.parametrize("q_lens,k_lens,gain", [
+    ((256,), (1,), 1.0), ((257, 319, 320), (32, 33, 64), 1.0), ((300, 300), (0, 65), 1.0),
+    ((511, 1, 640), (97, 1000, 31), 1.0), ((600,), (777,), 8.0)])
+def test_attention_fp32_tiled(px, orc, q_lens, k_lens, gain):
+    heads, hd = 3, 64
+    cu_q = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int64)
+    cu_k = np.concatenate([[0], np.cumsum(k_lens)]).astype(np.int64)
+    nq, nk, C = int(cu_q[-1]), int(cu_k[-1]), heads * hd
+    q = W.normal(67, nq * C, 1).reshape(nq, C)
+    k = W.normal(67, nk * C, 2).reshape(nk, C)
+    k[nk // 2:] *= gain
+    v = W.normal(67, nk * C, 3).reshape(nk, C)
+    print(f"[attn fp32 tiled] q={q_lens} k={k_lens}", flush=True)
+    o = host(px.varlen_attention(t32(q), t32(k), t32(v), ti64(cu_q), ti64(cu_k), heads, hd, 0.125))
+    assert_fp32(o, orc.varlen_attention(q, k, v, cu_q, cu_k, heads, hd, np.float32(0.125)),
+                what="attn fp32 tiled")
+
+
 def test_attention_bf16_random(px, orc):
     lens = (1000, 1536, 77)
     heads, hd = 4, 64
