@@ -85,6 +85,24 @@ def test_attention_fp32_tiled(px, orc, q_lens, k_lens, gain):
                 what="attn fp32 tiled")
 
 
+# Up to 64 segments the kernels find a tile's segment themselves, more take a
+# table: counts on both sides, with empty segments first, last and between.
+@pytest.mark.parametrize("nseg", [2, 63, 64, 65])
+@pytest.mark.parametrize("long", [0, 1500])
+def test_attention_fp32_segment_lookup(px, orc, nseg, long):
+    lens = np.arange(nseg) * 37 % 90
+    lens[[0, nseg // 2, nseg - 1]] = 0
+    lens[nseg // 2 - 1] += long + 1
+    heads, hd = 2, 64
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    n, C = int(cu[-1]), heads * hd
+    q, k, v = (W.normal(68, n * C, i).reshape(n, C) for i in (1, 2, 3))
+    print(f"[attn fp32 segments] nseg={nseg} n={n}", flush=True)
+    o = host(px.varlen_attention(t32(q), t32(k), t32(v), ti64(cu), ti64(cu), heads, hd, 0.125))
+    assert_fp32(o, orc.varlen_attention(q, k, v, cu, cu, heads, hd, np.float32(0.125)),
+                what="attn fp32 segments")
+
+
 def test_attention_bf16_random(px, orc):
     lens = (1000, 1536, 77)
     heads, hd = 4, 64
