@@ -29,7 +29,13 @@ struct BlockBuffers {
     void * ckv;   // [T, 2C]         context K | V
     void * ck;    // [T, C]          RMS-normed context K
     void * attn_ws;
+    float * partial;  // [splits, rows, C] of the residual linears split over K, or null
 };
+
+// Splits of a block's residual linears (0: one pass).
+int residual_splits(int dtype, int64_t rows, int cin, int channels) {
+    return residual_norm_takes(channels) ? dense_splits(dtype, rows, cin, channels) : 0;
+}
 
 BlockBuffers carve_block(Carver & c, int dtype, const pxs_block_config & cfg, int64_t rows,
                          int64_t tokens, int batch_size) {
@@ -48,6 +54,11 @@ BlockBuffers carve_block(Carver & c, int dtype, const pxs_block_config & cfg, in
     b.ckv = c.take(t * 2 * C * e);
     b.ck = c.take(t * C * e);
     b.attn_ws = c.take(pxs_attention_workspace_bytes(batch_size));
+    int splits = std::max(residual_splits(dtype, rows, cfg.channels, cfg.channels),
+                                residual_splits(dtype, rows, cfg.mlp_hidden, cfg.channels));
+    if (cfg.use_projection)
+        splits = std::max(splits, residual_splits(dtype, rows, cfg.proj_in_channels, cfg.channels));
+    b.partial = static_cast<float *>(c.take(static_cast<size_t>(splits) * r * C * 4));
     return b;
 }
 
@@ -78,6 +89,37 @@ int check_block_args(const pxs_block_config * cfg, const pxs_block_weights * w) 
 }
 
 
+bool aligned16(const void * p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+// hidden += (x w^T + bias) [* gate], then b.xm = the layer norm that n asks
+// for (n.y null: none).  Few rows: split over K, with the update and the norm
+// in one pass over the partial sums; otherwise the linear's residual epilogue
+// and a norm of its own.
+int residual_linear_norm(int dtype, const void * x, int64_t rows, int cin, const void * w, int C,
+                         ResidualNorm n, float * hidden, float * partial, void * stream) {
+    const int splits = residual_splits(dtype, rows, cin, C);
+    const bool aligned = aligned16(x) && aligned16(w) && aligned16(hidden) && aligned16(n.bias) &&
+                         aligned16(n.block_mod) && aligned16(n.time_mod) && aligned16(n.gamma) &&
+                         aligned16(n.beta);
+    if (splits > 0 && aligned) {
+        PXS_TRY(dense_partial(dtype, x, rows, cin, w, C, splits, partial, as_stream(stream)));
+        n.partial = partial;
+        n.splits = splits;
+        return residual_norm(n, rows, C, hidden, dtype, as_stream(stream));
+    }
+    if (n.gate_offset >= 0) {
+        PXS_TRY(pxs_linear_gate_residual(dtype, x, rows, cin, w, n.bias, C, n.coords, n.block_mod,
+                                         n.time_mod, n.gate_offset, hidden, stream));
+    } else {
+        PXS_TRY(pxs_linear_residual(dtype, x, rows, cin, w, n.bias, C, hidden, stream));
+    }
+    if (!n.y) return PXS_OK;
+    if (n.mod_offset >= 0)
+        return pxs_layer_norm_modulate(PXS_F32, hidden, rows, C, n.eps, n.coords, n.block_mod,
+                                       n.time_mod, n.mod_offset, dtype, n.y, stream);
+    return pxs_layer_norm(PXS_F32, hidden, rows, C, n.eps, n.gamma, n.beta, dtype, n.y, stream);
+}
+
 int run_block(int dtype, const pxs_block_config & cfg, const pxs_block_weights & w,
               const int32_t * coords, int64_t rows, int batch_size, const int64_t * cu_rows,
               float * hidden, const float * time_mod, const void * context,
@@ -98,13 +140,14 @@ int run_block(int dtype, const pxs_block_config & cfg, const pxs_block_weights &
                             cfg.rope_freq_base, b.q, b.k, b.v, stream));
     PXS_TRY(pxs_varlen_attention(dtype, b.q, C, b.k, C, b.v, C, cu_rows, cu_rows, batch_size, rows,
                                  nullptr, H, hd, hd, scale, b.att, C, b.attn_ws, stream));
-    PXS_TRY(pxs_linear_gate_residual(dtype, b.att, rows, C, w.self_to_out_weight,
-                                     w.self_to_out_bias, C, coords, w.modulation, time_mod, 2 * C,
-                                     hidden, stream));
+    ResidualNorm n{};
+    n.coords = coords; n.block_mod = w.modulation; n.time_mod = time_mod; n.eps = cfg.norm_eps;
+    n.bias = w.self_to_out_bias; n.gate_offset = 2 * C;
+    n.gamma = w.norm2_weight; n.beta = w.norm2_bias; n.mod_offset = -1; n.y = b.xm;
+    PXS_TRY(residual_linear_norm(dtype, b.att, rows, C, w.self_to_out_weight, C, n, hidden,
+                                 b.partial, stream));
 
-    // Cross-attention branch.
-    PXS_TRY(pxs_layer_norm(PXS_F32, hidden, rows, C, cfg.norm_eps, w.norm2_weight, w.norm2_bias,
-                           dtype, b.xm, stream));
+    // Cross-attention branch (its norm is above).
     PXS_TRY(pxs_linear(dtype, b.xm, rows, C, w.cross_to_q_weight, w.cross_to_q_bias, C,
                        PXS_ACT_NONE, b.q, stream));
     if (cfg.qk_rms_norm_cross) {
@@ -124,21 +167,22 @@ int run_block(int dtype, const pxs_block_config & cfg, const pxs_block_weights &
     PXS_TRY(pxs_varlen_attention(dtype, b.q, C, ck, ld_k, cv, 2 * C, cu_rows, context_offsets,
                                  batch_size, rows, nullptr, H, hd, hd, scale, b.att, C, b.attn_ws,
                                  stream));
-    PXS_TRY(pxs_linear_residual(dtype, b.att, rows, C, w.cross_to_out_weight, w.cross_to_out_bias,
-                                C, hidden, stream));
+    n.bias = w.cross_to_out_bias; n.gate_offset = -1; n.gamma = nullptr; n.beta = nullptr;
+    n.mod_offset = 3 * C; n.y = cfg.use_projection ? nullptr : b.xm;
+    PXS_TRY(residual_linear_norm(dtype, b.att, rows, C, w.cross_to_out_weight, C, n, hidden,
+                                 b.partial, stream));
     if (cfg.use_projection) {
-        PXS_TRY(pxs_linear_residual(dtype, projected, rows, cfg.proj_in_channels, w.proj_weight,
-                                    w.proj_bias, C, hidden, stream));
+        n.bias = w.proj_bias; n.y = b.xm;
+        PXS_TRY(residual_linear_norm(dtype, projected, rows, cfg.proj_in_channels, w.proj_weight, C,
+                                     n, hidden, b.partial, stream));
     }
 
-    // MLP branch.
-    PXS_TRY(pxs_layer_norm_modulate(PXS_F32, hidden, rows, C, cfg.norm_eps, coords, w.modulation,
-                                    time_mod, 3 * C, dtype, b.xm, stream));
+    // MLP branch (its norm is above).
     PXS_TRY(pxs_linear(dtype, b.xm, rows, C, w.mlp0_weight, w.mlp0_bias, cfg.mlp_hidden,
                        PXS_ACT_GELU_TANH, b.big, stream));
-    PXS_TRY(pxs_linear_gate_residual(dtype, b.big, rows, cfg.mlp_hidden, w.mlp2_weight,
-                                     w.mlp2_bias, C, coords, w.modulation, time_mod, 5 * C, hidden,
-                                     stream));
+    n.bias = w.mlp2_bias; n.gate_offset = 5 * C; n.mod_offset = -1; n.y = nullptr;
+    PXS_TRY(residual_linear_norm(dtype, b.big, rows, cfg.mlp_hidden, w.mlp2_weight, C, n, hidden,
+                                 b.partial, stream));
     return PXS_OK;
 }
 

@@ -41,10 +41,12 @@
 
 #include "pxs_common.h"
 
+#include <algorithm>
+
 namespace pxs {
 namespace {
 
-enum DenseEpi { kDenseStore = 0, kDenseAddResidual = 1, kDenseGate = 2 };
+enum DenseEpi { kDenseStore = 0, kDenseAddResidual = 1, kDenseGate = 2, kDensePartial = 3 };
 
 struct DenseArgs {
     const void * x;        // [m, k]
@@ -62,6 +64,7 @@ struct DenseArgs {
     int gate_offset;
     int vec_out;           // 1: 4-channel vector accesses; 2: also whole 16-byte row pieces
     int group_m;           // tile order: groups of group_m row tiles, each walked down its rows first
+    int splits;            // kDensePartial: K split over gridDim.y, sums to residual[split][m][n]
 };
 
 // Output tile (row tile, column tile) of logical tile t: groups of g row
@@ -120,7 +123,10 @@ __device__ __forceinline__ void dense_epilogue(const DenseArgs & a, const f32x16
                 float v[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * g + e];
-                if (a.vec_out && c + 3 < a.n) {
+                if constexpr (EPI == kDensePartial) {
+                    // cout is a multiple of 4 (dense_splits)
+                    *reinterpret_cast<float4 *>(a.residual + row * a.n + c) = make_float4(v[0], v[1], v[2], v[3]);
+                } else if (a.vec_out && c + 3 < a.n) {
                     if (a.bias) {
                         const float4 b = *reinterpret_cast<const float4 *>(a.bias + c);
                         v[0] = v[0] + b.x; v[1] = v[1] + b.y; v[2] = v[2] + b.z; v[3] = v[3] + b.w;
@@ -284,8 +290,17 @@ dense_gemm_kernel(DenseArgs a) {
 
     const char * xs = static_cast<const char *>(a.x) + p0 * a.k * static_cast<int64_t>(sizeof(T));
     const char * wsb = static_cast<const char *>(a.w) + static_cast<int64_t>(n0) * a.k * sizeof(T);
-    const int stages = (a.k + kChunk - 1) / kChunk;
-    const bool ragged = a.k % kChunk != 0;  // the last chunk holds pieces past k
+    // Stages of this workgroup: all of K, or its split's share of them.
+    const int all_stages = (a.k + kChunk - 1) / kChunk;
+    int stage0 = 0, stages = all_stages;
+    if constexpr (EPI == kDensePartial) {
+        stage0 = static_cast<int>(blockIdx.y) * all_stages / a.splits;
+        stages = (static_cast<int>(blockIdx.y) + 1) * all_stages / a.splits - stage0;
+        a.residual += static_cast<int64_t>(blockIdx.y) * a.m * a.n;
+        xs += static_cast<int64_t>(stage0) * KB;
+        wsb += static_cast<int64_t>(stage0) * KB;
+    }
+    const bool ragged = a.k % kChunk != 0;  // the last chunk of K holds pieces past k
     // Fixed per-lane parts of the loads: row lane / P of each instruction,
     // clamped into the operand, and the swizzled piece it fetches.
     const int lrow = lane / P, lslot = lane % P;
@@ -317,9 +332,9 @@ dense_gemm_kernel(DenseArgs a) {
         const uint32_t lds = lds_offset(base + ((is_x ? 0 : BM) + (wave * (is_x ? AI : BI) + j) * RPI) * KB);
         const char * src = is_x ? xs : wsb;
         const uint32_t off = is_x ? a_off[j] : b_off[j];
-        if (ragged && s == stages - 1) {
+        if (ragged && stage0 + s == all_stages - 1) {
             // Pieces past k come from the zero line.
-            const bool in = s * kChunk + (lslot ^ piece_swz<KB>(row)) * kVec < a.k;
+            const bool in = (stage0 + s) * kChunk + (lslot ^ piece_swz<KB>(row)) * kVec < a.k;
             lds_dma16(in ? static_cast<const void *>(src + kb + off) : static_cast<const void *>(g_dense_zero), lds);
         } else {
             lds_dma16_sbase(src + kb, off, lds);
@@ -432,7 +447,8 @@ int launch_dense(const DenseArgs & a, hipStream_t stream) {
     if (a.vec_out == 2 && smem < kStagedBytes) smem = kStagedBytes;
     const int64_t blocks = ((a.m + BM - 1) / BM) * ((a.n + BN - 1) / BN);
     if (blocks > INT32_MAX) return fail(PXS_ERR_ARG, "dense GEMM grid too large");
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(NW * 64), smem, stream, a);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks), EPI == kDensePartial ? a.splits : 1),
+                       dim3(NW * 64), smem, stream, a);
     return check_launch("dense GEMM");
 }
 
@@ -523,6 +539,37 @@ int dense_linear_gate(int dtype, const void * x, int64_t rows, int cin, const vo
                 aligned_to(time_mod, 16);
     *done = true;
     return run_dense<kDenseGate>(dtype, a, s);
+}
+
+// Few rows leave most CUs without a 128 x 128 tile, and smaller tiles move
+// more operand bytes per product through each CU (about 40 GB/s, the bound
+// here: 1,000 x 4096 -> 1024 in bf16 takes 38 us on 128 x 64 tiles and 28 us on
+// 64 x 64 tiles, with two stages in flight or six).  K is then split so that
+// the tiles come near to one per CU, two splits still paying at 170 tiles.
+// Six blocks of width 1024 with their three residual linears in one pass
+// against 2, 3, 4, 5 splits: 248 rows 1,775 us against 1,628, 1,596, 1,586, 1,590;
+// 1,288 rows 1,632 against 1,500, 1,515, 1,508, 1,539; 2,600 rows (168 tiles) 2,118
+// against 2,037, 2,077, 2,202, 2,229; 4,064 rows (256 tiles) 2,503 against 2,522,
+// 2,698, 2,736, 2,863.
+int dense_splits(int dtype, int64_t rows, int cin, int cout) {
+    const int vec = dtype == PXS_BF16 ? 8 : 4, chunk = 8 * vec;
+    if (rows <= 0 || cin % vec != 0 || cout % 4 != 0 || cout <= 64) return 0;
+    const int64_t tiles = ((rows + 127) / 128) * ((cout + 127) / 128);
+    if (tiles > 170) return 0;
+    const int64_t most = std::min<int64_t>(4, cin / (4 * chunk));  // 4 stages of K each
+    const int64_t splits = std::min(most, std::max<int64_t>(2, 256 / tiles));
+    return splits >= 2 ? static_cast<int>(splits) : 0;
+}
+
+int dense_partial(int dtype, const void * x, int64_t rows, int cin, const void * w, int cout,
+                  int splits, float * partial, hipStream_t s) {
+    DenseArgs a{};
+    a.x = x; a.w = w; a.m = rows; a.k = cin; a.n = cout; a.residual = partial; a.splits = splits;
+    a.vec_out = 1;
+    a.group_m = 8;
+    return dtype == PXS_BF16
+               ? launch_dense<uint16_t, 128, 128, 8, 2, 2, 128, kDensePartial, false, false>(a, s)
+               : launch_dense<float, 128, 128, 8, 2, 2, 128, kDensePartial, false, false>(a, s);
 }
 
 } // namespace pxs

@@ -669,6 +669,73 @@ __global__ void timestep_embedding_kernel(const float * __restrict__ t, int64_t 
     out[i] = v;
 }
 
+// residual_norm: one wavefront per row of 256 NV channels, the row in
+// registers between the update of the residual and its norm (the norm's
+// arithmetic is layer_norm_rows_kernel's).
+template <typename TY, int NV>
+__global__ void __launch_bounds__(256)
+residual_norm_kernel(ResidualNorm a, int64_t rows, float * __restrict__ residual) {
+    constexpr int C = 256 * NV;
+    const int lane = threadIdx.x & 63;
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const float * tm = nullptr;
+    if (a.gate_offset >= 0 || a.mod_offset >= 0) tm = a.time_mod + static_cast<int64_t>(a.coords[row * 4]) * 6 * C;
+    auto at = [](const float * p) { return *reinterpret_cast<const float4 *>(p); };
+    float4 v[NV];
+    float s = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = (j * 64 + lane) * 4;
+        float4 u = at(a.partial + row * C + c);
+        for (int q = 1; q < a.splits; ++q) {
+            const float4 w = at(a.partial + (q * rows + row) * C + c);
+            u.x += w.x; u.y += w.y; u.z += w.z; u.w += w.w;
+        }
+        const float4 b = at(a.bias + c);
+        u.x += b.x; u.y += b.y; u.z += b.z; u.w += b.w;
+        if (a.gate_offset >= 0) {
+            const float4 g = at(a.block_mod + a.gate_offset + c), t = at(tm + a.gate_offset + c);
+            u.x *= g.x + t.x; u.y *= g.y + t.y; u.z *= g.z + t.z; u.w *= g.w + t.w;
+        }
+        v[j] = at(residual + row * C + c);
+        v[j].x += u.x; v[j].y += u.y; v[j].z += u.z; v[j].w += u.w;
+        *reinterpret_cast<float4 *>(residual + row * C + c) = v[j];
+        s += v[j].x; s += v[j].y; s += v[j].z; s += v[j].w;
+    }
+    if (!a.y) return;
+    const float mean = group_sum<64>(s) / static_cast<float>(C);
+    float q = 0.0f;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const float d[4] = {v[j].x - mean, v[j].y - mean, v[j].z - mean, v[j].w - mean};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) q += d[e] * d[e];
+    }
+    const float var = group_sum<64>(q) / static_cast<float>(C);
+    const float inv = 1.0f / sqrtf(var + a.eps);
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = (j * 64 + lane) * 4;
+        float o[4] = {(v[j].x - mean) * inv, (v[j].y - mean) * inv, (v[j].z - mean) * inv, (v[j].w - mean) * inv};
+        if (a.mod_offset >= 0) {
+            const float4 bs = at(a.block_mod + a.mod_offset + C + c), ts = at(tm + a.mod_offset + C + c);
+            const float4 bh = at(a.block_mod + a.mod_offset + c), th = at(tm + a.mod_offset + c);
+            o[0] = o[0] * (1.0f + (bs.x + ts.x)) + (bh.x + th.x);
+            o[1] = o[1] * (1.0f + (bs.y + ts.y)) + (bh.y + th.y);
+            o[2] = o[2] * (1.0f + (bs.z + ts.z)) + (bh.z + th.z);
+            o[3] = o[3] * (1.0f + (bs.w + ts.w)) + (bh.w + th.w);
+        } else {
+            const float4 ga = at(a.gamma + c), be = at(a.beta + c);
+            o[0] = o[0] * ga.x + be.x;
+            o[1] = o[1] * ga.y + be.y;
+            o[2] = o[2] * ga.z + be.z;
+            o[3] = o[3] * ga.w + be.w;
+        }
+        store_vec<TY, 4>(static_cast<TY *>(a.y) + row * C + c, o);
+    }
+}
+
 int check_dtype(int dtype) { return dtype == PXS_F32 || dtype == PXS_BF16; }
 
 template <typename TX, typename TY, int L, int NV, bool kMod>
@@ -755,6 +822,25 @@ int run_head_op(const void * x, int64_t ld_x, int64_t rows, int heads, int head_
 }
 
 } // namespace
+bool residual_norm_takes(int channels) { return channels % 256 == 0 && channels <= 1024; }
+
+int residual_norm(const ResidualNorm & a, int64_t rows, int channels, float * residual, int y_dtype,
+                  hipStream_t s) {
+    const dim3 grid(grid_for(rows, 4)), block(256);
+    auto launch = [&](auto tag) {
+        using T = decltype(tag);
+        switch (channels / 256) {
+        case 1: hipLaunchKernelGGL((residual_norm_kernel<T, 1>), grid, block, 0, s, a, rows, residual); break;
+        case 2: hipLaunchKernelGGL((residual_norm_kernel<T, 2>), grid, block, 0, s, a, rows, residual); break;
+        case 3: hipLaunchKernelGGL((residual_norm_kernel<T, 3>), grid, block, 0, s, a, rows, residual); break;
+        default: hipLaunchKernelGGL((residual_norm_kernel<T, 4>), grid, block, 0, s, a, rows, residual); break;
+        }
+    };
+    if (y_dtype == PXS_BF16) launch(uint16_t{});
+    else launch(float{});
+    return check_launch("residual and layer norm");
+}
+
 } // namespace pxs
 
 using namespace pxs;

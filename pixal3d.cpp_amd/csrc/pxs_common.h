@@ -36,6 +36,35 @@ int dense_linear_gate(int dtype, const void * x, int64_t rows, int cin, const vo
                       const float * block_mod, const float * time_mod, int gate_offset,
                       float * residual, hipStream_t s, bool * done);
 
+// A residual linear of few rows split over K, and the layer norm that reads
+// its result (csrc/dense.hip, csrc/pointwise.hip).
+//   dense_splits: splits of K for this shape (rows of x and w 16-byte
+//     aligned), 0 when one pass is better.
+//   dense_partial: partial[s] [rows, cout] fp32 = split s of x w^T.
+//   residual_norm: residual += (sum of the partials in order + bias) [* gate],
+//     then y = layer norm of the row with gamma and beta, or the adaLN modulate
+//     at mod_offset >= 0, or nothing (y null).  channels as residual_norm_takes.
+struct ResidualNorm {
+    const float * partial;
+    int splits;
+    const float * bias;
+    const int32_t * coords;
+    const float * block_mod;
+    const float * time_mod;
+    int gate_offset;  // < 0: no gate
+    float eps;
+    const float * gamma;
+    const float * beta;
+    int mod_offset;   // < 0: gamma and beta
+    void * y;
+};
+int dense_splits(int dtype, int64_t rows, int cin, int cout);
+int dense_partial(int dtype, const void * x, int64_t rows, int cin, const void * w, int cout,
+                  int splits, float * partial, hipStream_t s);
+bool residual_norm_takes(int channels);
+int residual_norm(const ResidualNorm & a, int64_t rows, int channels, float * residual, int y_dtype,
+                  hipStream_t s);
+
 // The C -> 8 out SubMConv3d of a channel-to-spatial up-block with a
 // subdivision, bf16, computed for the kept children only and written straight
 // to their rows (csrc/gemm.hip; the lists come from csrc/topology.hip).

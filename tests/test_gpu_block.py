@@ -155,3 +155,37 @@ def test_block_fp32_wide_heads(px, orc):
     ref = orc.transformer_block(coords, 2, x, tmod, ctx, off, [C, H, M, CC, 0, 1, 1, 1, 0],
                                 [1e-6, 1.0, 10000.0], ws)
     assert_fp32(host(hidden), ref, what="block wide heads")
+
+
+@pytest.mark.parametrize("C,rows,M,PC", [(256, 1, 512, 0), (512, 130, 1024, 0), (768, 129, 520, 36),
+                                         (1024, 260, 1024, 256)])
+def test_block_residual_linears_split_over_k(px, orc, C, rows, M, PC):
+    """Blocks of few rows: the residual linears whose K is long enough run split
+    over K, with the residual's update and the next norm in one pass (each
+    width of that pass; MLP-2 with a ragged last K chunk; a projection that
+    is split and one that is not), fp32, against the oracle block."""
+    from test_gpu_configs import flow_block_weights, normal
+    rng = np.random.default_rng(95)
+    coords = W.shell_coords(16, [[(4.0, 6.0)], [(3.0, 5.0)]], 95)
+    keep = np.sort(rng.permutation(coords.shape[0])[:rows])
+    coords = np.ascontiguousarray(coords[keep])
+    H, CC, T = C // 64, 64, 9
+    ws = flow_block_weights(rng, C, M, CC)
+    proj = None
+    if PC:
+        ws[17], ws[18] = normal(rng, (C, PC), 0.02), normal(rng, (C,), 0.02)
+        proj = normal(rng, (rows, PC))
+    x = normal(rng, (rows, C))
+    tmod = normal(rng, (2, 6 * C), 0.3)
+    ctx = normal(rng, (2 * T, CC))
+    off = np.array([0, T, 2 * T], np.int64)
+    print(f"[block split] rows={rows} C={C} M={M} PC={PC}", flush=True)
+    c = ti32(coords)
+    hidden = t32(x).clone()
+    dws = device_weights(ws, torch.float32)  # kept alive: the struct holds raw pointers
+    px.transformer_block(block_cfg(C, H, M, CC, PC, PC > 0), pxs.block_weights(dws), c, 2,
+                         px.batch_cu_seqlens(c, 2), hidden, t32(tmod), t32(ctx), ti64(off),
+                         projected=t32(proj) if PC else None)
+    ref = orc.transformer_block(coords, 2, x, tmod, ctx, off, [C, H, M, CC, PC, 1, 1, 1, int(PC > 0)],
+                                [1e-6, 1.0, 10000.0], ws, projected=proj)
+    assert_fp32(host(hidden), ref, what="block split")
