@@ -120,26 +120,19 @@ struct AttnArgs {
 };
 
 // Query tile t (of q_tile queries, a power of two): its segment and the
-// segment's first tile; false past the last tile.  SELF (at most 64 segments):
-// no tile_start table, lane i takes segment i and the wave sums the tile
-// counts.  The table costs two launches, 9.4 us before each call, half of what
-// the attention of 1,300 tokens takes; on 32,768 tokens (4,096 workgroups) the
-// SELF form of the kernel ran 0.5% slower, 14 us, so large calls keep the
-// table (self_tiles).
+// segment's first tile; false past the last tile.  Used by the SELF kernels (at
+// most 64 segments), which take no tile_start table: lane i takes segment i and
+// the wave sums the tile counts.  The table costs two launches, 9.4 us before
+// each call, half of what the attention of 1,300 tokens takes; on 32,768
+// tokens (4,096 workgroups) the SELF form of the kernel ran 0.5% slower, 14 us,
+// so large calls keep the table (self_tiles).
 constexpr int kSelfSegments = 64;
 constexpr int64_t kSelfWorkgroups = 2048;
 inline bool self_tiles(int64_t total_q, int nseg, int q_tile, int heads) {
     return nseg <= kSelfSegments && (total_q / q_tile + nseg + 1) * heads <= kSelfWorkgroups;
 }
-template <bool SELF>
 __device__ __forceinline__ bool locate_tile(const AttnArgs & a, int q_tile, int64_t t, int lane,
                                             int & seg, int64_t & first) {
-    if constexpr (!SELF) {
-        if (t >= a.tile_start[a.nseg]) return false;
-        seg = find_segment(a.tile_start, a.nseg, t, lane);
-        first = a.tile_start[seg];
-        return true;
-    }
     const int shift = 31 - __clz(q_tile);
     int tiles = 0;
     if (lane < a.nseg) tiles = static_cast<int>((a.cu_q[lane + 1] - a.cu_q[lane] + q_tile - 1) >> shift);
@@ -207,9 +200,16 @@ flash_attn_kernel(AttnArgs a) {
 
     const int64_t t = blockIdx.x;
     int seg;
-    int64_t first;
-    if (!locate_tile<SELF>(a, 32 * NW, t, lane, seg, first)) return;
-    const int64_t q_begin = a.cu_q[seg] + (t - first) * (32 * NW);
+    int64_t q_begin;
+    if constexpr (SELF) {
+        int64_t first;
+        if (!locate_tile(a, 32 * NW, t, lane, seg, first)) return;
+        q_begin = a.cu_q[seg] + (t - first) * (32 * NW);
+    } else {
+        if (t >= a.tile_start[a.nseg]) return;
+        seg = find_segment(a.tile_start, a.nseg, t, lane);
+        q_begin = a.cu_q[seg] + (t - a.tile_start[seg]) * (32 * NW);
+    }
     const int64_t q_end = a.cu_q[seg + 1];
     const int64_t k_begin = a.cu_k[seg], k_end = a.cu_k[seg + 1];
 
@@ -540,9 +540,16 @@ flash_attn_bf16_kernel(AttnArgs a, int heads, int64_t tiles_bound) {
     const int head = static_cast<int>(logical / tiles_bound);
     const int64_t t = logical - static_cast<int64_t>(head) * tiles_bound;
     int seg;
-    int64_t first;
-    if (!locate_tile<SELF>(a, 32 * NW, t, lane, seg, first)) return;
-    const int64_t q_begin = a.cu_q[seg] + (t - first) * (32 * NW);
+    int64_t q_begin;
+    if constexpr (SELF) {
+        int64_t first;
+        if (!locate_tile(a, 32 * NW, t, lane, seg, first)) return;
+        q_begin = a.cu_q[seg] + (t - first) * (32 * NW);
+    } else {
+        if (t >= a.tile_start[a.nseg]) return;
+        seg = find_segment(a.tile_start, a.nseg, t, lane);
+        q_begin = a.cu_q[seg] + (t - a.tile_start[seg]) * (32 * NW);
+    }
     const int64_t q_end = a.cu_q[seg + 1];
     const int64_t k_begin = a.cu_k[seg], k_end = a.cu_k[seg + 1];
 
@@ -1306,9 +1313,16 @@ flash_attn_f32_kernel(AttnArgs a, int heads, int64_t tiles_bound) {
     const int head = static_cast<int>(logical / tiles_bound);
     const int64_t t = logical - static_cast<int64_t>(head) * tiles_bound;
     int seg;
-    int64_t first;
-    if (!locate_tile<SELF>(a, kF32Queries, t, lane, seg, first)) return;
-    const int64_t q_begin = a.cu_q[seg] + (t - first) * kF32Queries;
+    int64_t q_begin;
+    if constexpr (SELF) {
+        int64_t first;
+        if (!locate_tile(a, kF32Queries, t, lane, seg, first)) return;
+        q_begin = a.cu_q[seg] + (t - first) * kF32Queries;
+    } else {
+        if (t >= a.tile_start[a.nseg]) return;
+        seg = find_segment(a.tile_start, a.nseg, t, lane);
+        q_begin = a.cu_q[seg] + (t - a.tile_start[seg]) * kF32Queries;
+    }
     const int64_t q_end = a.cu_q[seg + 1];
     const int64_t k_begin = a.cu_k[seg], k_end = a.cu_k[seg + 1];
     const float * __restrict__ kp = static_cast<const float *>(a.k) + head * 64;
