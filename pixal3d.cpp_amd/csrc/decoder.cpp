@@ -206,6 +206,13 @@ int pxs_convnext_block(int dtype, const int32_t * coords, int64_t rows, const fl
     }
     PXS_TRY(pxs_subm_conv3d(dtype, xin, rows, channels, w->conv1_weight, w->conv1_bias, channels,
                             nbr, masks, b.conv, stream));
+    if (dtype == PXS_BF16) {
+        bool done = false;
+        PXS_TRY(convnext_mlp(b.conv, rows, channels, eps, w->norm_weight, w->norm_bias,
+                             w->mlp0_weight, w->mlp0_bias, w->mlp2_weight, w->mlp2_bias,
+                             mlp_hidden, x, y, s, &done));
+        if (done) return PXS_OK;
+    }
     PXS_TRY(pxs_layer_norm(dtype, b.conv, rows, channels, eps, w->norm_weight, w->norm_bias, dtype,
                            b.norm, stream));
     PXS_TRY(pxs_linear(dtype, b.norm, rows, channels, w->mlp0_weight, w->mlp0_bias, mlp_hidden,

@@ -65,6 +65,14 @@ bool residual_norm_takes(int channels);
 int residual_norm(const ResidualNorm & a, int64_t rows, int channels, float * residual, int y_dtype,
                   hipStream_t s);
 
+// x_out = x_in + the ConvNeXt MLP (layer norm, linear, SiLU, linear) of y, bf16
+// operands, in one kernel (csrc/mlp.hip); x_out may be x_in.  *done is left
+// false for shapes and alignments it does not take.
+int convnext_mlp(const void * y, int64_t rows, int channels, float eps, const float * gamma,
+                 const float * beta, const void * w0, const float * b0, const void * w2,
+                 const float * b2, int hidden, const float * x_in, float * x_out, hipStream_t s,
+                 bool * done);
+
 // The C -> 8 out SubMConv3d of a channel-to-spatial up-block with a
 // subdivision, bf16, computed for the kept children only and written straight
 // to their rows (csrc/gemm.hip; the lists come from csrc/topology.hip).

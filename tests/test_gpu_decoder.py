@@ -77,6 +77,41 @@ def test_convnext_block(px, orc, dtype):
         assert_bf16(got, ref, what="convnext bf16")
 
 
+# Rows at the edges of a wave's 32 and a workgroup's 256, each width of the
+# one-kernel MLP with one and several chunks of 64 hidden channels, and a hidden
+# width it does not take.
+@pytest.mark.parametrize("C,M,rows", [(64, 64, 1), (64, 256, 33), (64, 320, 256), (128, 512, 257),
+                                      (128, 1024, 31), (256, 1024, 300), (256, 128, 513),
+                                      (64, 96, 100)])
+def test_convnext_block_bf16_mlp(px, C, M, rows):
+    """A bf16 ConvNeXt block, in place and not, against the same block from its
+    single ops.  Both round the norm and the hidden tensor to bf16; sums taken
+    in another order may move either by one step, 2^-8, at most."""
+    dev = torch.device("cuda:0")
+    coords = ti32(W.shell_coords(24, [[(6.0, 9.0)]], 47)[:rows])
+    assert coords.shape[0] == rows
+    g = torch.Generator(device=dev).manual_seed(rows + C)
+    rnd = lambda *s, std=1.0: torch.randn(*s, generator=g, device=dev) * std  # noqa: E731
+    bf = torch.bfloat16
+    w = {"norm_weight": 1.0 + rnd(C, std=0.1), "norm_bias": rnd(C, std=0.1),
+         "conv1_weight": rnd(27, C, C, std=(27 * C) ** -0.5).to(bf), "conv1_bias": rnd(C, std=0.1),
+         "mlp0_weight": rnd(M, C, std=C ** -0.5).to(bf), "mlp0_bias": rnd(M, std=0.1),
+         "mlp2_weight": rnd(C, M, std=M ** -0.5).to(bf), "mlp2_bias": rnd(C, std=0.1)}
+    x = rnd(rows, C)
+    print(f"convnext mlp rows={rows} C={C} M={M}", flush=True)
+    dw = pxs.decoder_block_weights(w)
+    y = px.convnext_block(coords, x, M, 1e-6, dw, pxs.PXS_BF16)
+    h = x.clone()
+    px.convnext_block(coords, h, M, 1e-6, dw, pxs.PXS_BF16, out=h)
+    assert torch.equal(h, y)
+    c = px.subm_conv3d(x.to(bf), w["conv1_weight"], w["conv1_bias"], *px.neighbor_map(coords))
+    n = px.layer_norm(c, 1e-6, w["norm_weight"], w["norm_bias"])
+    ref = torch.zeros_like(x)
+    px.linear_residual(px.linear(n, w["mlp0_weight"], w["mlp0_bias"], act=2), w["mlp2_weight"],
+                       w["mlp2_bias"], ref)
+    assert_bf16(host(y - x), host(ref), tol=2.0 ** -8, what="convnext mlp")
+
+
 def test_convnext_block_in_place_with_given_map(px, orc):
     """y aliasing x and a caller-built neighbor map give the same result."""
     C, M = 32, 128
