@@ -20,8 +20,8 @@
 // instruction's A operand and the X fragment its B operand, so D = Y^T per
 // 32 x 32 block and lane (h, r) holds output row r, channels 8g + 4h + 0..3
 // for g = 0..3: four consecutive channels per lane.
-//   bf16: v_mfma_f32_32x32x16_bf16, 4 K steps of 16 per chunk;
-//   fp32: v_mfma_f32_32x32x2_f32, 16 K steps of 2 per chunk.
+//   bf16: v_mfma_f32_32x32x16_bf16, 4 K steps of 16 per chunk (dense_gemm_kernel);
+//   fp32: the same instruction on operands split in three (dense_split_kernel).
 // The K order inside a chunk is permuted identically for both operands so a
 // lane reads 16 contiguous bytes per LDS access; pieces are XOR-swizzled by
 // row so the 16 rows one LDS cycle serves read 16 different bank groups.
@@ -265,6 +265,7 @@ dense_gemm_kernel(DenseArgs a) {
     constexpr int WAVES_N = NW / WAVES_M;
     constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
     constexpr int TI = WM / 32, TJ = WN / 32;
+    static_assert(sizeof(T) == 2, "fp32 products run on dense_split_kernel");
     static_assert(TI * 32 * WAVES_M == BM && TJ * 32 * WAVES_N == BN, "wave blocks must tile");
     constexpr int kStage = (BM + BN) * KB;
     constexpr int AI = BM / (RPI * NW);  // DMA instructions per wave per stage
@@ -393,25 +394,13 @@ dense_gemm_kernel(DenseArgs a) {
             if (u + 1 < P / 2) read_frags(u + 1, xr[(u + 1) & 1], wr[(u + 1) & 1]);
             const uint4 (&xc)[TI] = xr[u & 1];
             const uint4 (&wc)[TJ] = wr[u & 1];
-            if constexpr (sizeof(T) == 2) {
 #pragma unroll
-                for (int i = 0; i < TI; ++i)
+            for (int i = 0; i < TI; ++i)
 #pragma unroll
-                    for (int j = 0; j < TJ; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            __builtin_bit_cast(bf16x8, wc[j]), __builtin_bit_cast(bf16x8, xc[i]),
-                            acc[i][j], 0, 0, 0);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int i = 0; i < TI; ++i)
-#pragma unroll
-                        for (int j = 0; j < TJ; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                                __builtin_bit_cast(f32x4, wc[j])[e], __builtin_bit_cast(f32x4, xc[i])[e],
-                                acc[i][j], 0, 0, 0);
-            }
+                for (int j = 0; j < TJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        __builtin_bit_cast(bf16x8, wc[j]), __builtin_bit_cast(bf16x8, xc[i]),
+                        acc[i][j], 0, 0, 0);
         }
     }
     if constexpr (STAGED && EPI == kDenseStore) {
@@ -423,6 +412,273 @@ dense_gemm_kernel(DenseArgs a) {
         }
     }
     dense_epilogue<T, TI, TJ, EPI>(a, acc, p0 + wm * WM, n0 + wn * WN, h, r);
+}
+
+// ---- fp32 products on the bf16 matrix cores --------------------------------
+// Each fp32 operand is split without loss into three bf16 terms, a = a1 + a2 +
+// a3 (each the rounding of what the ones before leave), and a product takes
+// the six terms above 2^-26 of it: a1 b1, a1 b2, a2 b1, a2 b2, a1 b3, a3 b1.
+// Six v_mfma_f32_32x32x16_bf16 cost 192 matrix-core cycles where the eight
+// v_mfma_f32_32x32x2_f32 of the same 16 K steps cost 512.  Against 64-bit
+// products of N(0, 1) operands the results are closer than that instruction's:
+// relative error (2-norm) 3.4e-7 against 4.0e-7 at K = 1024, 7.1e-7 against
+// 8.1e-7 at 4096, 8.1e-8 against 1.05e-7 at 64.
+//
+// What bounds it: the vector instructions that split the operands (12 per pair
+// of values) beside the matrix cores, so a split is shared by as large a tile
+// as registers and a balanced grid allow.  206,980 x 1024 -> 256: 627 us
+// against 873 on fp32 MFMA tiles (173 against 124 TFLOP/s); 4,736 x 1024 ->
+// 4096: 224 against 315; 1,000 x 4096 -> 1024: 105 against 155.  Tiles of 256 x
+// 256 or 256 x 128 (8 or 16 waves, one workgroup per CU) ran slower: 683-1,173
+// us on the first shape.
+//
+// Valid while no operand exceeds 2^50 in magnitude and no sum is nonzero below
+// 2^-60: operands below 2^-102 lose low bits to bf16's least exponent, which
+// moves a sum by at most K 2^-84.  A tile that meets a larger operand, or ends
+// with a smaller or a non-finite sum (as any infinity or NaN operand gives), is
+// computed again on v_mfma_f32_32x32x2_f32 from global memory.
+constexpr float kSplitHigh = 0x1p50f, kSplitLow = 0x1p-60f;
+
+// Splits 4 values into the three planes' 8-byte pieces; hi follows the largest
+// magnitude seen.
+__device__ __forceinline__ void split4(const float4 & f, uint2 (&out)[3], float & hi) {
+    const float v[4] = {f.x, f.y, f.z, f.w};
+    uint32_t w[3][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        float a = v[2 * i], b = v[2 * i + 1];
+        hi = fmaxf(hi, fmaxf(fabsf(a), fabsf(b)));
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            uint32_t pk = pack_bf16x2(a, b);
+            asm("" : "+v"(pk));  // one conversion, not one more to take the low half apart
+            w[q][i] = pk;
+            if (q < 2) {
+                a = a - __builtin_bit_cast(float, pk << 16);
+                b = b - __builtin_bit_cast(float, pk & 0xffff0000u);
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) out[q] = make_uint2(w[q][0], w[q][1]);
+}
+
+// One tile of BM x BN, NWM x NWN waves.  Per 32-element K chunk every thread
+// splits its share of the X and W rows (loaded into registers while the chunk
+// before is multiplied) and writes the planes to LDS as [plane][8-element
+// piece][row] pieces of 16 bytes (piece columns 64 bytes apart modulo the
+// banks, so that the 4 pieces of a row that neighbouring lanes write do not
+// conflict; fragment reads cover 256 contiguous bytes per 16 lanes).
+template <int BM, int BN, int NWM, int NWN, int WPE, int EPI>
+__global__ void __launch_bounds__(NWM * NWN * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
+dense_split_kernel(DenseArgs a) {
+    constexpr int NT = NWM * NWN * 64, RS = NT / 8;  // rows apart a thread's pieces are
+    constexpr int WM = BM / NWM, WN = BN / NWN, TI = WM / 32, TJ = WN / 32;
+    constexpr int kColX = BM * 16 + 64, kColW = BN * 16 + 64;  // bytes per piece column
+    constexpr int kPlaneX = 4 * kColX, kPlaneW = 4 * kColW;
+    constexpr int XI = BM / RS, WI = BN / RS;  // pieces per thread and chunk
+    extern __shared__ __align__(16) char smem[];
+    char * sx = smem;
+    char * sw = smem + 3 * kPlaneX;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / NWN, wn = wave % NWN;
+    const int h = lane >> 5, r = lane & 31;
+    const int tiles_n = (a.n + BN - 1) / BN;
+    const int tiles_m = static_cast<int>((a.m + BM - 1) / BM);
+    int tm, tn;
+    tile_of(remap_xcd(blockIdx.x, gridDim.x), tiles_m, tiles_n, a.group_m, tm, tn);
+    const int64_t p0 = static_cast<int64_t>(tm) * BM;
+    const int n0 = tn * BN;
+    const float * x = static_cast<const float *>(a.x);
+    const float * w = static_cast<const float *>(a.w);
+
+    // This thread's 16-byte pieces of the 128-byte chunk rows: piece `piece`,
+    // rows row + RS i (clamped; outputs past the end are not stored).
+    const int piece = tid & 7, row = tid >> 3;
+    const char * xb = reinterpret_cast<const char *>(x + p0 * a.k);
+    const char * wb = reinterpret_cast<const char *>(w + static_cast<int64_t>(n0) * a.k);
+    const int64_t last_x = a.m - 1 - p0;
+    const int last_w = a.n - 1 - n0;
+    uint32_t x_off[XI], w_off[WI];  // bytes
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        const int m = row + RS * i;
+        x_off[i] = static_cast<uint32_t>(((m < last_x ? m : last_x) * a.k + piece * 4) * 4);
+    }
+#pragma unroll
+    for (int i = 0; i < WI; ++i) {
+        const int n = row + RS * i;
+        w_off[i] = static_cast<uint32_t>((static_cast<int64_t>(n < last_w ? n : last_w) * a.k + piece * 4) * 4);
+    }
+    // K chunks of this workgroup: all, or its split's share of them.
+    const int all_chunks = (a.k + 31) / 32;
+    int chunk0 = 0, chunks = all_chunks;
+    if constexpr (EPI == kDensePartial) {
+        chunk0 = static_cast<int>(blockIdx.y) * all_chunks / a.splits;
+        chunks = (static_cast<int>(blockIdx.y) + 1) * all_chunks / a.splits - chunk0;
+        a.residual += static_cast<int64_t>(blockIdx.y) * a.m * a.n;
+    }
+    float4 vx[XI], vw[WI];
+    auto load = [&](int s) __attribute__((always_inline)) {
+        const char * xs = xb + static_cast<int64_t>(s) * 128;
+        const char * wsb = wb + static_cast<int64_t>(s) * 128;
+        if (s * 32 + 32 <= a.k) {
+#pragma unroll
+            for (int i = 0; i < XI; ++i) vx[i] = *reinterpret_cast<const float4 *>(xs + x_off[i]);
+#pragma unroll
+            for (int i = 0; i < WI; ++i) vw[i] = *reinterpret_cast<const float4 *>(wsb + w_off[i]);
+        } else {
+            const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const bool in = s * 32 + piece * 4 < a.k;
+#pragma unroll
+            for (int i = 0; i < XI; ++i) {
+                vx[i] = zero;
+                if (in) vx[i] = *reinterpret_cast<const float4 *>(xs + x_off[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < WI; ++i) {
+                vw[i] = zero;
+                if (in) vw[i] = *reinterpret_cast<const float4 *>(wsb + w_off[i]);
+            }
+        }
+    };
+
+    f32x16 acc[TI][TJ];
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+
+    float hi = 0.0f;
+    load(chunk0);
+    for (int s = 0; s < chunks; ++s) {
+        barrier_no_fence();  // every wave has read the previous chunk
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            uint2 t[3];
+            split4(vx[i], t, hi);
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                *reinterpret_cast<uint2 *>(sx + q * kPlaneX + (piece >> 1) * kColX + (row + RS * i) * 16 + (piece & 1) * 8) = t[q];
+        }
+#pragma unroll
+        for (int i = 0; i < WI; ++i) {
+            uint2 t[3];
+            split4(vw[i], t, hi);
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                *reinterpret_cast<uint2 *>(sw + q * kPlaneW + (piece >> 1) * kColW + (row + RS * i) * 16 + (piece & 1) * 8) = t[q];
+        }
+        if (s + 1 < chunks) load(chunk0 + s + 1);
+        barrier_no_fence();
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            bf16x8 xf[3][TI];
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+#pragma unroll
+                for (int i = 0; i < TI; ++i)
+                    xf[q][i] = *reinterpret_cast<const bf16x8 *>(
+                        sx + q * kPlaneX + (2 * u + h) * kColX + (wm * WM + i * 32 + r) * 16);
+#pragma unroll
+            for (int j = 0; j < TJ; ++j) {
+                bf16x8 wf[3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    wf[q] = *reinterpret_cast<const bf16x8 *>(
+                        sw + q * kPlaneW + (2 * u + h) * kColW + (wn * WN + j * 32 + r) * 16);
+                // the smaller terms first
+                constexpr int kTermX[6] = {2, 0, 1, 1, 0, 0}, kTermW[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+                for (int t = 0; t < 6; ++t)
+#pragma unroll
+                    for (int i = 0; i < TI; ++i)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[kTermW[t]], xf[kTermX[t]][i],
+                                                                            acc[i][j], 0, 0, 0);
+            }
+        }
+    }
+    bool odd = hi > kSplitHigh;
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const float m = fabsf(acc[i][j][v]);
+                odd |= !(m == 0.0f || (m >= kSplitLow && m < INFINITY));
+            }
+    if (__syncthreads_or(odd)) {
+        // rare: the whole tile again in fp32
+#pragma unroll
+        for (int i = 0; i < TI; ++i)
+#pragma unroll
+            for (int j = 0; j < TJ; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+        const float * xr[TI];
+        const float * wr[TJ];
+#pragma unroll
+        for (int i = 0; i < TI; ++i) {
+            const int64_t m = p0 + wm * WM + i * 32 + r;
+            xr[i] = x + (m < a.m ? m : a.m - 1) * a.k;
+        }
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) {
+            const int n = n0 + wn * WN + j * 32 + r;
+            wr[j] = w + static_cast<int64_t>(n < a.n ? n : a.n - 1) * a.k;
+        }
+        const int k_end = min(a.k, (chunk0 + chunks) * 32);  // a multiple of 4, as chunk0 * 32 is
+        for (int k = chunk0 * 32 + h; k < k_end; k += 2)
+#pragma unroll
+            for (int i = 0; i < TI; ++i)
+#pragma unroll
+                for (int j = 0; j < TJ; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(wr[j][k], xr[i][k], acc[i][j], 0, 0, 0);
+    }
+    if constexpr (EPI == kDenseStore) {
+        if (a.vec_out == 2) {
+            // 32 rows of each wave's block at a time through the idle planes
+            barrier_no_fence();
+#pragma unroll
+            for (int i = 0; i < TI; ++i) {
+                f32x16 part[1][TJ];
+#pragma unroll
+                for (int j = 0; j < TJ; ++j) part[0][j] = acc[i][j];
+                dense_store_staged<float, 1, TJ>(a, part, smem + wave * 32 * staged_pitch<float, WN>(),
+                                                 p0 + wm * WM + i * 32, n0 + wn * WN, h, r, lane);
+            }
+            return;
+        }
+    }
+    dense_epilogue<float, TI, TJ, EPI>(a, acc, p0 + wm * WM, n0 + wn * WN, h, r);
+}
+
+template <int BM, int BN, int NWM, int NWN, int WPE, int EPI>
+int launch_dense_split(const DenseArgs & a, hipStream_t stream) {
+    constexpr int kPlanes = 3 * 4 * ((BM + BN) * 16 + 128);
+    constexpr int kStaged = EPI == kDenseStore ? NWM * NWN * 32 * staged_pitch<float, BN / NWN>() : 0;
+    constexpr int smem = kPlanes > kStaged ? kPlanes : kStaged;
+    auto kernel = &dense_split_kernel<BM, BN, NWM, NWN, WPE, EPI>;
+    if constexpr (smem > 64 * 1024) {
+        static bool configured = false;
+        if (!configured) {
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+            if (e != hipSuccess) return check_hip(e, "hipFuncSetAttribute(dense_split)");
+            configured = true;
+        }
+    }
+    const int64_t blocks = ((a.m + BM - 1) / BM) * ((a.n + BN - 1) / BN);
+    if (blocks > INT32_MAX) return fail(PXS_ERR_ARG, "dense GEMM grid too large");
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks), EPI == kDensePartial ? a.splits : 1),
+                       dim3(NWM * NWN * 64), smem, stream, a);
+    return check_launch("dense GEMM (fp32 split)");
 }
 
 template <typename T, int BM, int BN, int NW, int WAVES_M, int NSTAGE, int KB, int EPI,
@@ -454,32 +710,46 @@ int launch_dense(const DenseArgs & a, hipStream_t stream) {
 
 // Tile shape by the estimated time of the whole grid: rounds of tiles over
 // the 256 CUs (workgroups resident per CU in parallel) times the time of one
-// round, from each shape's measured rate (bf16: 256 x 256 tiles about 1000
-// TFLOP/s, 128 x 128 about 880, 128 x 64 about 700; fp32: 128 x 128 about
-// 130, 128 x 64 about 128).  256 x 256 tiles go down 8-row-tile groups, the
-// others down groups of 16 when a row holds at most 4 column tiles, else 8.
-template <typename T, int EPI>
-int dispatch_dense(DenseArgs a, hipStream_t s) {
-    constexpr bool bf16 = sizeof(T) == 2;
+// round, from each shape's measured rate (256 x 256 tiles about 1000 TFLOP/s,
+// 128 x 128 about 880, 128 x 64 about 700).  256 x 256 tiles go down
+// 8-row-tile groups, the others down groups of 16 when a row holds at most 4
+// column tiles, else 8.
+template <int EPI>
+int dispatch_bf16(DenseArgs a, hipStream_t s) {
     auto rounds = [&](int bm, int bn, int per_cu) {
         const int64_t tiles = ((a.m + bm - 1) / bm) * ((a.n + bn - 1) / bn);
         return static_cast<double>((tiles + 256 * per_cu - 1) / (256 * per_cu));
     };
-    const double t_b = rounds(128, 128, 2) * 2.0 * 128 * 128 / (bf16 ? 880.0 : 130.0);
-    const double t_c = rounds(128, 64, 3) * 3.0 * 128 * 64 / (bf16 ? 700.0 : 128.0);
-    if constexpr (bf16) {
-        const double t_a = rounds(256, 256, 1) * 256.0 * 256 / 1000.0;
-        if (a.n > 128 && t_a <= t_b) {
-            a.group_m = 8;
-            return launch_dense<T, 256, 256, 16, 4, 2, 128, EPI, true, true>(a, s);
-        }
+    const double t_a = rounds(256, 256, 1) * 256.0 * 256 / 1000.0;
+    const double t_b = rounds(128, 128, 2) * 2.0 * 128 * 128 / 880.0;
+    const double t_c = rounds(128, 64, 3) * 3.0 * 128 * 64 / 700.0;
+    if (a.n > 128 && t_a <= t_b) {
+        a.group_m = 8;
+        return launch_dense<uint16_t, 256, 256, 16, 4, 2, 128, EPI, true, true>(a, s);
     }
     if (a.n <= 64 || t_c < t_b) {
         a.group_m = (a.n + 63) / 64 <= 4 ? 16 : 8;
-        return launch_dense<T, 128, 64, 4, 2, 2, 128, EPI, false, true>(a, s);
+        return launch_dense<uint16_t, 128, 64, 4, 2, 2, 128, EPI, false, true>(a, s);
     }
     a.group_m = (a.n + 127) / 128 <= 4 ? 16 : 8;
-    return launch_dense<T, 128, 128, 8, 2, 2, 128, EPI, false, true>(a, s);
+    return launch_dense<uint16_t, 128, 128, 8, 2, 2, 128, EPI, false, true>(a, s);
+}
+
+// fp32: the tile with the least estimated time, in us per 1024 of K: what a
+// lone workgroup takes, or the workgroups a CU gets times what each adds
+// (measured on 1,000 to 206,980 rows).  A tie goes to the larger tile.
+template <int EPI>
+int dispatch_f32(DenseArgs a, hipStream_t s) {
+    auto time = [&](int bm, int bn, double alone, double each) {
+        const int64_t tiles = ((a.m + bm - 1) / bm) * ((a.n + bn - 1) / bn);
+        return std::max(alone, static_cast<double>((tiles + 255) / 256) * each);
+    };
+    const double t_a = time(128, 128, 64.0, 48.0), t_b = time(128, 64, 44.0, 28.0);
+    const double t_c = time(64, 64, 31.0, 16.0);
+    a.group_m = 8;
+    if (a.n > 64 && t_a <= t_b && t_a <= t_c) return launch_dense_split<128, 128, 2, 2, 3, EPI>(a, s);
+    if (t_b <= t_c) return launch_dense_split<128, 64, 2, 2, 3, EPI>(a, s);
+    return launch_dense_split<64, 64, 2, 2, 4, EPI>(a, s);
 }
 
 bool aligned_to(const void * p, uintptr_t bytes) { return (reinterpret_cast<uintptr_t>(p) % bytes) == 0; }
@@ -494,7 +764,7 @@ bool dense_takes(int dtype, const void * x, int cin, const void * w) {
 
 template <int EPI>
 int run_dense(int dtype, const DenseArgs & a, hipStream_t s) {
-    return dtype == PXS_BF16 ? dispatch_dense<uint16_t, EPI>(a, s) : dispatch_dense<float, EPI>(a, s);
+    return dtype == PXS_BF16 ? dispatch_bf16<EPI>(a, s) : dispatch_f32<EPI>(a, s);
 }
 
 } // namespace
@@ -569,7 +839,7 @@ int dense_partial(int dtype, const void * x, int64_t rows, int cin, const void *
     a.group_m = 8;
     return dtype == PXS_BF16
                ? launch_dense<uint16_t, 128, 128, 8, 2, 2, 128, kDensePartial, false, false>(a, s)
-               : launch_dense<float, 128, 128, 8, 2, 2, 128, kDensePartial, false, false>(a, s);
+               : launch_dense_split<128, 128, 2, 2, 3, kDensePartial>(a, s);
 }
 
 } // namespace pxs

@@ -3,6 +3,7 @@ layer norm (+modulation), multi-head RMS norm, RoPE, the QKV prologue."""
 
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 import workloads as W
@@ -31,6 +32,39 @@ def test_linear_fp32(px, orc, rows, cin, cout):
     print(f"[linear fp32] {rows}x{cin}->{cout}", flush=True)
     y = host(px.linear(t32(x), t32(w), t32(b)))
     assert_fp32(y, orc.linear(x, w, b), what="linear fp32")
+
+
+def test_linear_fp32_split_range(px):
+    """fp32 linears multiply operands split into three bf16 terms; a tile that
+    meets values out of the split's range (infinities, NaN, 2^50 and more,
+    sums below 2^-60) is computed again in fp32.  Rows of such values beside
+    ordinary ones, on each tile shape, against 64-bit products: finite results
+    within K 2^-24 sum |x w| (the bound of a K-term sum rounded at every step),
+    infinities and NaN where the products have them."""
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(57)
+    for rows, k, n in ((3, 64, 20), (200, 64, 132), (4000, 36, 520), (40000, 64, 260)):
+        x = torch.randn(rows, k, generator=g, device=dev)
+        w = torch.randn(n, k, generator=g, device=dev)
+        x[0, 1], x[1, 2] = float("inf"), float("nan")
+        # sums near 1e-27: products stay above fp32's denormals (1.2e-38), which the
+        # fp32 matrix instruction may flush, an error that room does not cover
+        x[2] *= 1e-28
+        if rows > 100:
+            x[rows - 1] *= 1e30
+            x[rows - 2] = 0.0
+            x[rows // 2] *= 1e-25
+            w[n - 1, 0] = -float("inf")
+        print(f"[linear fp32 range] {rows}x{k}->{n}", flush=True)
+        y = px.linear(x, w, None).double()
+        ref = x.double() @ w.double().t()
+        room = (x.double().abs() @ w.double().abs().t()) * k * 2.0 ** -24
+        ok = torch.isfinite(ref)
+        over = torch.where(ok, (y - ref).abs() / room, torch.zeros_like(ref))
+        over = torch.nan_to_num(over)  # 0 / 0 in a row of zeros
+        assert torch.equal(torch.isnan(y), torch.isnan(ref))
+        assert torch.equal(y[torch.isinf(ref)], ref[torch.isinf(ref)])
+        assert over.max() <= 1.0, (over.max(), (over > 1.0).nonzero()[:8])
 
 
 def test_linear_reference_vectors(px):
