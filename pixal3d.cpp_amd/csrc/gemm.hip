@@ -1687,22 +1687,22 @@ int launch_range_conv(const GemmArgs & args, hipStream_t stream) {
 // ---------------------------------------------------------------------------
 // fp32 split-K gather GEMM (SubMConv3d and linears in fp32).  A workgroup
 // owns 32*TI output rows x 64 output channels; its (offset, 32-channel chunk)
-// steps are dealt round-robin to the 4 waves, so even a few hundred tiles
+// steps are dealt round-robin to its NW waves, so even a few hundred tiles
 // keep every CU busy.  Each wave loads its operands straight into VGPRs --
 // lane (h, r) takes the 64 contiguous bytes k = 16h .. 16h+15 of A row r (of
 // each 32-row block) and of weight row r, the same K permutation on both
 // sides of v_mfma_f32_32x32x2_f32 -- with the next step's loads in flight
 // during the current step's MFMAs, and no barrier until the end, where waves
-// 1-3 hand their partial sums to wave 0 through LDS (a fixed summation order:
+// 1 and up hand their partial sums to wave 0 through LDS (a fixed summation order:
 // deterministic).  The operand loads return through the per-CU vector-memory
 // path, which bounds the kernel: TI = 2 reads each weight chunk once for 64
 // rows instead of 32 (16 KB per 64x64x32 step instead of 24 KB), at 64
 // accumulator registers per lane.
 
-template <int EPI, int TI>
-__global__ void __launch_bounds__(256)
+template <int EPI, int TI, int NW>
+__global__ void __launch_bounds__(NW * 64)
 split_gemm_f32_kernel(GemmArgs a) {
-    constexpr int BM = 32 * TI, BN = 64, NW = 4;
+    constexpr int BM = 32 * TI, BN = 64;
     __shared__ float red[NW - 1][TI * 2][16][64];
     __shared__ int32_t idx_lds[32 * BM];
     __shared__ uint32_t tile_mask;
@@ -1871,14 +1871,14 @@ split_gemm_f32_kernel(GemmArgs a) {
 #define PXS_SPLIT_F32_WIDE_MAX 1024
 #endif
 
-template <int EPI, int TI>
+template <int EPI, int TI, int NW>
 int launch_split_f32_ti(const GemmArgs & args, hipStream_t stream) {
     const int64_t tiles_m = (args.m + 32 * TI - 1) / (32 * TI);
     const int64_t tiles_n = (args.cout + 63) / 64;
     const int64_t blocks = tiles_m * tiles_n;
     if (blocks > INT32_MAX) return fail(PXS_ERR_ARG, "gather GEMM grid too large");
-    hipLaunchKernelGGL((split_gemm_f32_kernel<EPI, TI>), dim3(static_cast<unsigned>(blocks)),
-                       dim3(256), 0, stream, args);
+    hipLaunchKernelGGL((split_gemm_f32_kernel<EPI, TI, NW>), dim3(static_cast<unsigned>(blocks)),
+                       dim3(NW * 64), 0, stream, args);
     return check_launch("gather GEMM (fp32 split-K)");
 }
 
@@ -1887,10 +1887,13 @@ int launch_split_f32(const GemmArgs & args, hipStream_t stream) {
     const int64_t wide = ((args.m + 63) / 64) * ((args.cout + 63) / 64);
     // (Only for the 27-offset gathers: plain linears, with 2 K steps per
     // tile, run 1.5x slower on 64-row tiles, 19 against 13 us at 16k x 64.)
-    if ((args.rowmap || args.grid) && args.noff >= 27 && wide >= PXS_SPLIT_F32_WIDE_MIN &&
-        wide <= PXS_SPLIT_F32_WIDE_MAX)
-        return launch_split_f32_ti<EPI, 2>(args, stream);
-    return launch_split_f32_ti<EPI, 1>(args, stream);
+    const bool gather = (args.rowmap || args.grid) && args.noff >= 27;
+    if (gather && wide >= PXS_SPLIT_F32_WIDE_MIN && wide <= PXS_SPLIT_F32_WIDE_MAX)
+        return launch_split_f32_ti<EPI, 2, 4>(args, stream);
+    // At most one tile per CU: twice the waves halve each one's chain of steps.
+    const int64_t tiles = ((args.m + 31) / 32) * ((args.cout + 63) / 64);
+    if (gather && tiles <= 256) return launch_split_f32_ti<EPI, 1, 8>(args, stream);
+    return launch_split_f32_ti<EPI, 1, 4>(args, stream);
 }
 
 template <typename T, int BM, int BN, int EPI, int NSTAGE, int NW, int WAVES_M, int KSPLIT>

@@ -205,6 +205,33 @@ neighbor_map_kernel(const int4 * __restrict__ coords, int64_t n,
     if (masks && present) atomicOr(masks + p, present);
 }
 
+// The same map with one lane per (row, offset), 32 lanes per row: one probe per
+// lane instead of nine, and the row's mask from one ballot, so masks needs no
+// clearing launch.  Its 4-byte stores are n apart, so only for few rows.
+constexpr int64_t kMapLanesRows = 16384;
+__global__ void __launch_bounds__(kThreads)
+neighbor_map_lanes_kernel(const int4 * __restrict__ coords, int64_t n,
+                          const HashSlot * __restrict__ slots, uint64_t mask,
+                          int32_t * __restrict__ nbr, uint32_t * __restrict__ masks) {
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t p = t >> 5;
+    const int k = static_cast<int>(t & 31);
+    int32_t row = -1;
+    if (p < n && k < 27) {
+        const int4 c = coords[p];
+        const int x = c.y + k / 9 - 1, y = c.z + (k / 3) % 3 - 1, z = c.w + k % 3 - 1;
+        if (k == 13) row = static_cast<int32_t>(p);
+        else if (x >= 0 && y >= 0 && z >= 0) {
+            const uint64_t key = voxel_key(c.x, x, y, z), slot = home_slot(key, mask);
+            row = probe_from(slots, mask, key, slot, load_slot(slots, slot));
+        }
+        nbr[k * n + p] = row >= 0 ? row : static_cast<int32_t>(n);
+    }
+    const uint64_t present = __ballot(row >= 0);
+    if (masks && p < n && k == 0)
+        masks[p] = static_cast<uint32_t>(present >> (threadIdx.x & 32));
+}
+
 // ---- voxel bricks: a locality-preserving hash --------------------------------------
 // The voxel hash puts the 27 neighbours of a row in 27 unrelated 128-byte
 // lines.  Here the hash holds 4x4x4 bricks: a slot keys brick (b, x>>2,
@@ -1311,6 +1338,11 @@ int pxs_neighbor_map_k3(const int32_t * coords, int64_t n, const void * table, i
     PXS_CHECK(coords && table && nbr, PXS_ERR_ARG, "pxs_neighbor_map_k3: null pointer");
     const HashView h = hash_view(const_cast<void *>(table), n);
     hipStream_t s = as_stream(stream);
+    if (n <= kMapLanesRows) {
+        hipLaunchKernelGGL(neighbor_map_lanes_kernel, dim3(grid_for(32 * n, kThreads)), dim3(kThreads), 0,
+                           s, reinterpret_cast<const int4 *>(coords), n, h.slots, h.mask, nbr, masks);
+        return check_launch("pxs_neighbor_map_k3");
+    }
     if (masks) {
         if (int rc = fill_u32(masks, n, 0u, s)) return rc;
     }
