@@ -111,6 +111,7 @@ struct DecoderBuffers {
     float * hid[2];
     int32_t * crd[2];
     MapBuffers map[2];  // the current level's map and the next one's (built by the C2S block)
+    uint16_t * x16;     // bf16 copy of a C2S block's output for the ConvNeXt block after it
     void * block_ws;
 };
 
@@ -123,7 +124,7 @@ int64_t grow8(int64_t n, int64_t cap) { return n > cap / 8 ? cap : 8 * n; }
 DecoderBuffers carve_decoder(Carver & c, int dtype, const pxs_decoder_config & cfg,
                              const pxs_decoder_block * blocks, int n_blocks, int64_t rows,
                              int64_t max_rows) {
-    size_t hid = 0, ws = 0;
+    size_t hid = 0, ws = 0, x16 = 0;
     int64_t cap = rows, cap_max = rows;
     int bi = 0;
     for (int l = 0; l < cfg.levels; ++l) {
@@ -131,6 +132,7 @@ DecoderBuffers carve_decoder(Carver & c, int dtype, const pxs_decoder_config & c
         cap_max = std::max(cap_max, cap);
         const int C = cfg.model_channels[l];
         hid = std::max(hid, static_cast<size_t>(cap) * static_cast<size_t>(std::max(C, 1)));
+        if (l > 0) x16 = std::max(x16, static_cast<size_t>(cap) * static_cast<size_t>(std::max(C, 1)));
         for (int k = 0; k < cfg.num_blocks[l] && bi < n_blocks; ++k, ++bi)
             ws = std::max(ws, pxs_convnext_block_workspace_bytes(dtype, cap, C, blocks[bi].mlp_hidden, 1));
         if (l + 1 < cfg.levels && bi < n_blocks) {
@@ -148,6 +150,7 @@ DecoderBuffers carve_decoder(Carver & c, int dtype, const pxs_decoder_config & c
     b.crd[1] = static_cast<int32_t *>(c.take(static_cast<size_t>(cap_max) * 16));
     b.map[0] = carve_map(c, cap_max);
     b.map[1] = carve_map(c, cap_max);
+    if (dtype == PXS_BF16) b.x16 = static_cast<uint16_t *>(c.take(x16 * 2));
     b.block_ws = c.take(ws);
     return b;
 }
@@ -167,10 +170,11 @@ size_t pxs_convnext_block_workspace_bytes(int dtype, int64_t rows, int channels,
     return c.used();
 }
 
-int pxs_convnext_block(int dtype, const int32_t * coords, int64_t rows, const float * x,
-                       int channels, int mlp_hidden, float eps,
-                       const pxs_decoder_block_weights * w, const int32_t * nbr,
-                       const uint32_t * masks, float * y, void * workspace, void * stream) {
+// The ConvNeXt block; x16 (bf16, or null) is x already converted.
+static int convnext_block(int dtype, const int32_t * coords, int64_t rows, const float * x,
+                          const uint16_t * x16, int channels, int mlp_hidden, float eps,
+                          const pxs_decoder_block_weights * w, const int32_t * nbr,
+                          const uint32_t * masks, float * y, void * workspace, void * stream) {
     PXS_CHECK_WORKSPACE(workspace, "pxs_convnext_block");
     PXS_CHECK(dtype == PXS_F32 || dtype == PXS_BF16, PXS_ERR_ARG, "pxs_convnext_block: bad dtype");
     PXS_CHECK(eps > 0.0f && std::isfinite(eps), PXS_ERR_ARG,
@@ -200,7 +204,9 @@ int pxs_convnext_block(int dtype, const int32_t * coords, int64_t rows, const fl
         masks = b.map.masks;
     }
     const void * xin = x;
-    if (dtype == PXS_BF16) {
+    if (dtype == PXS_BF16 && x16) {
+        xin = x16;
+    } else if (dtype == PXS_BF16) {
         PXS_TRY(pxs_convert(PXS_F32, x, rows * channels, PXS_BF16, b.xd, stream));
         xin = b.xd;
     }
@@ -228,6 +234,14 @@ int pxs_convnext_block(int dtype, const int32_t * coords, int64_t rows, const fl
                                channels, y, stream);
 }
 
+int pxs_convnext_block(int dtype, const int32_t * coords, int64_t rows, const float * x,
+                       int channels, int mlp_hidden, float eps,
+                       const pxs_decoder_block_weights * w, const int32_t * nbr,
+                       const uint32_t * masks, float * y, void * workspace, void * stream) {
+    return convnext_block(dtype, coords, rows, x, nullptr, channels, mlp_hidden, eps, w, nbr, masks, y,
+                          workspace, stream);
+}
+
 size_t pxs_resblock_c2s_workspace_bytes(int dtype, int64_t rows, int channels,
                                         int out_channels) {
     if (rows < 0 || channels <= 0 || out_channels <= 0) return 0;
@@ -236,7 +250,7 @@ size_t pxs_resblock_c2s_workspace_bytes(int dtype, int64_t rows, int channels,
     return c.used();
 }
 
-// The C2S block; in_map (the map of coords, already built) and out_map
+// The C2S block, with a bf16 copy of y where y16 is set; in_map (the map of coords, already built) and out_map
 // (where to build the map of out_coords) come from a caller that keeps one
 // map per level, or are null for the block's own in its workspace.
 static int resblock_c2s(int dtype, const int32_t * coords, int64_t rows, const float * x,
@@ -244,7 +258,8 @@ static int resblock_c2s(int dtype, const int32_t * coords, int64_t rows, const f
                         const pxs_decoder_block_weights * w, int pred_subdiv,
                         const float * subdivision, float * predicted_subdiv,
                         int32_t * out_coords, float * y, int64_t * rows_out, void * workspace,
-                        void * stream, const MapBuffers * in_map, const MapBuffers * out_map) {
+                        void * stream, const MapBuffers * in_map, const MapBuffers * out_map,
+                        uint16_t * y16) {
     PXS_CHECK_WORKSPACE(workspace, "pxs_resblock_c2s");
     PXS_CHECK(dtype == PXS_F32 || dtype == PXS_BF16, PXS_ERR_ARG, "pxs_resblock_c2s: bad dtype");
     PXS_CHECK(eps > 0.0f && std::isfinite(eps), PXS_ERR_ARG,
@@ -285,9 +300,8 @@ static int resblock_c2s(int dtype, const int32_t * coords, int64_t rows, const f
                                    pred, stream));
         selected = pred;
     }
-    PXS_TRY(pxs_layer_norm(PXS_F32, x, rows, channels, eps, w->norm1_weight, w->norm1_bias, dtype,
-                           b.norm, stream));
-    PXS_TRY(pxs_activation(dtype, b.norm, rows * channels, PXS_ACT_SILU, stream));
+    PXS_TRY(layer_norm_silu(PXS_F32, x, rows, channels, eps, w->norm1_weight, w->norm1_bias, dtype,
+                            b.norm, s));
     if (!in_map) PXS_TRY(build_map(coords, rows, map1, stream));
     // With a subdivision, about half the children are dropped: the bf16
     // convolution then runs over the kept ones only, once their count is known.
@@ -324,14 +338,12 @@ static int resblock_c2s(int dtype, const int32_t * coords, int64_t rows, const f
     }
     *rows_out = m;
     if (m == 0) return PXS_OK;
-    PXS_TRY(pxs_layer_norm(dtype, b.hidden, m, out_channels, eps, nullptr, nullptr, dtype, b.hnorm,
-                           stream));
-    PXS_TRY(pxs_activation(dtype, b.hnorm, m * out_channels, PXS_ACT_SILU, stream));
+    PXS_TRY(layer_norm_silu(dtype, b.hidden, m, out_channels, eps, nullptr, nullptr, dtype, b.hnorm, s));
     PXS_TRY(build_map(out_coords, m, map2, stream));
     void * conv_out = dtype == PXS_BF16 ? b.conv2 : static_cast<void *>(y);
     PXS_TRY(pxs_subm_conv3d(dtype, b.hnorm, m, out_channels, w->conv2_weight, w->conv2_bias,
                             out_channels, map2.nbr, map2.masks, conv_out, stream));
-    return pxs_add_repeat(dtype, conv_out, m, out_channels, b.skip, channels / 8, y, stream);
+    return add_repeat(dtype, conv_out, m, out_channels, b.skip, channels / 8, y, y16, stream);
 }
 
 int pxs_resblock_c2s(int dtype, const int32_t * coords, int64_t rows, const float * x,
@@ -341,7 +353,7 @@ int pxs_resblock_c2s(int dtype, const int32_t * coords, int64_t rows, const floa
                      float * y, int64_t * rows_out, void * workspace, void * stream) {
     return resblock_c2s(dtype, coords, rows, x, channels, out_channels, eps, w, pred_subdiv,
                         subdivision, predicted_subdiv, out_coords, y, rows_out, workspace, stream,
-                        nullptr, nullptr);
+                        nullptr, nullptr, nullptr);
 }
 
 size_t pxs_slat_decoder_workspace_bytes(int dtype, const pxs_decoder_config * cfg,
@@ -418,6 +430,7 @@ int pxs_slat_decoder_forward(int dtype, const pxs_decoder_config * cfg,
     // ConvNeXt blocks and C2S conv1 reuse it.
     int mc = 0;
     bool map_ready = false;
+    const uint16_t * x16 = nullptr;  // bf16 copy of b.hid[cur], while there is one
     for (int l = 0; l < levels; ++l) {
         const int C = cfg->model_channels[l];
         if (upsample && l == upsample_times) {
@@ -440,9 +453,9 @@ int pxs_slat_decoder_forward(int dtype, const pxs_decoder_config * cfg,
                                : "SLat decoder expected ConvNeXt block");
             PXS_CHECK(blk.channels == C, PXS_ERR_ARG,
                       "pxs_slat_decoder_forward: block channels do not match the level");
-            PXS_TRY(pxs_convnext_block(dtype, ccur, n, b.hid[cur], C, blk.mlp_hidden, eps, &blk.w,
-                                       b.map[mc].nbr, b.map[mc].masks, b.hid[cur], b.block_ws,
-                                       stream));
+            PXS_TRY(convnext_block(dtype, ccur, n, b.hid[cur], x16, C, blk.mlp_hidden, eps, &blk.w,
+                                   b.map[mc].nbr, b.map[mc].masks, b.hid[cur], b.block_ws, stream));
+            x16 = nullptr;  // the block has updated the state in place
         }
         if (l + 1 == levels) break;
         const pxs_decoder_block & blk = blocks[bi++];
@@ -460,7 +473,8 @@ int pxs_slat_decoder_forward(int dtype, const pxs_decoder_config * cfg,
         int64_t m = 0;
         PXS_TRY(resblock_c2s(dtype, ccur, n, b.hid[cur], C, blk.out_channels, eps, &blk.w,
                              pred ? 1 : 0, g, logits, b.crd[nxt], b.hid[nxt], &m, b.block_ws,
-                             stream, &b.map[mc], &b.map[1 - mc]));
+                             stream, &b.map[mc], &b.map[1 - mc], b.x16));
+        x16 = b.x16;
         ccur = b.crd[nxt];
         cur = nxt;
         n = m;

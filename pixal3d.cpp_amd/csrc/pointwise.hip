@@ -21,12 +21,19 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
+// SiLU of a normalised value as the activation pass over the stored norm
+// computes it: the value rounded to the output's type first.
+template <typename TY> __device__ __forceinline__ float silu_of_stored(float v) {
+    if constexpr (sizeof(TY) == 2) v = bf16_to_f32(f32_to_bf16(v));
+    return silu_f(v);
+}
+
 template <typename TX, typename TY, bool kModulate>
 __global__ void __launch_bounds__(64 * kRowsPerBlock)
 layer_norm_kernel(const TX * __restrict__ x, int64_t rows, int channels, float eps,
                   const float * __restrict__ gamma, const float * __restrict__ beta,
                   const int32_t * __restrict__ coords, const float * __restrict__ block_mod,
-                  const float * __restrict__ time_mod, int mod_offset, TY * __restrict__ y) {
+                  const float * __restrict__ time_mod, int mod_offset, bool silu, TY * __restrict__ y) {
     const int lane = threadIdx.x & 63;
     const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + (threadIdx.x >> 6);
     if (row >= rows) return;
@@ -52,6 +59,7 @@ layer_norm_kernel(const TX * __restrict__ x, int64_t rows, int channels, float e
             const float shift = block_mod[mod_offset + c] + tm[mod_offset + c];
             val = val * (1.0f + scale) + shift;
         }
+        if (silu) val = silu_of_stored<TY>(val);
         store_f32(dst + c, val);
     }
 }
@@ -110,7 +118,8 @@ __global__ void __launch_bounds__(256)
 layer_norm_rows_kernel(const TX * __restrict__ x, int64_t rows, float eps,
                        const float * __restrict__ gamma, const float * __restrict__ beta,
                        const int32_t * __restrict__ coords, const float * __restrict__ block_mod,
-                       const float * __restrict__ time_mod, int mod_offset, TY * __restrict__ y) {
+                       const float * __restrict__ time_mod, int mod_offset, bool silu,
+                       TY * __restrict__ y) {
     constexpr int V = Vec16<TX>::kN;
     constexpr int C = L * NV * V;
     const int lane = threadIdx.x & 63;
@@ -178,6 +187,7 @@ layer_norm_rows_kernel(const TX * __restrict__ x, int64_t rows, float eps,
                 const float shift = bh[e] + th[e];
                 val = val * (1.0f + scale) + shift;
             }
+            if (silu) val = silu_of_stored<TY>(val);
             o[e] = val;
         }
         store_vec<TY, V>(y + row * C + c0, o);
@@ -610,7 +620,7 @@ __global__ void convert8_kernel(const TS * __restrict__ x, int64_t nvec, TD * __
 template <typename T>
 __global__ void add_repeat8_kernel(const T * a, uint32_t nvec, uint32_t vpr,
                                    const float * __restrict__ skip, int skip_channels, int repeats,
-                                   float * y) {
+                                   float * y, uint16_t * __restrict__ y16) {
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nvec; i += stride) {
         const uint32_t r = i / vpr;
@@ -621,6 +631,7 @@ __global__ void add_repeat8_kernel(const T * a, uint32_t nvec, uint32_t vpr,
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = v[e] + sk[(j0 + e) / repeats];
         store8(y + static_cast<int64_t>(i) * 8, v);
+        if (y16) store8(y16 + static_cast<int64_t>(i) * 8, v);
     }
 }
 
@@ -741,11 +752,11 @@ int check_dtype(int dtype) { return dtype == PXS_F32 || dtype == PXS_BF16; }
 template <typename TX, typename TY, int L, int NV, bool kMod>
 void launch_ln_rows(const void * x, int64_t rows, float eps, const float * gamma,
                     const float * beta, const int32_t * coords, const float * bm, const float * tm,
-                    int off, void * y, hipStream_t s) {
+                    int off, bool silu, void * y, hipStream_t s) {
     hipLaunchKernelGGL((layer_norm_rows_kernel<TX, TY, L, NV, kMod>),
                        dim3(grid_for(rows, 4 * (64 / L))), dim3(256), 0, s,
                        static_cast<const TX *>(x), rows, eps, gamma, beta, coords, bm, tm, off,
-                       static_cast<TY *>(y));
+                       silu, static_cast<TY *>(y));
 }
 
 // The row-group kernel when a row is 2^k 16-byte vectors (up to 64 lanes of
@@ -753,22 +764,22 @@ void launch_ln_rows(const void * x, int64_t rows, float eps, const float * gamma
 template <typename TX, typename TY, bool kMod>
 bool try_ln_rows(const void * x, int64_t rows, int channels, float eps, const float * gamma,
                  const float * beta, const int32_t * coords, const float * bm, const float * tm,
-                 int off, void * y, hipStream_t s) {
+                 int off, bool silu, void * y, hipStream_t s) {
     constexpr int V = Vec16<TX>::kN;
     auto a16 = [](const void * p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     if (channels % V != 0 || !a16(x) || !a16(y) || (gamma && (!a16(gamma) || !a16(beta))))
         return false;
     if (kMod && (!a16(bm) || !a16(tm) || off % 4 != 0)) return false;
     switch (channels / V) {
-    case 1: launch_ln_rows<TX, TY, 1, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, y, s); return true;
-    case 2: launch_ln_rows<TX, TY, 2, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, y, s); return true;
-    case 4: launch_ln_rows<TX, TY, 4, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, y, s); return true;
-    case 8: launch_ln_rows<TX, TY, 8, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, y, s); return true;
-    case 16: launch_ln_rows<TX, TY, 16, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, y, s); return true;
-    case 32: launch_ln_rows<TX, TY, 32, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, y, s); return true;
-    case 64: launch_ln_rows<TX, TY, 64, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, y, s); return true;
-    case 128: launch_ln_rows<TX, TY, 64, 2, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, y, s); return true;
-    case 256: launch_ln_rows<TX, TY, 64, 4, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, y, s); return true;
+    case 1: launch_ln_rows<TX, TY, 1, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, silu, y, s); return true;
+    case 2: launch_ln_rows<TX, TY, 2, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, silu, y, s); return true;
+    case 4: launch_ln_rows<TX, TY, 4, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, silu, y, s); return true;
+    case 8: launch_ln_rows<TX, TY, 8, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, silu, y, s); return true;
+    case 16: launch_ln_rows<TX, TY, 16, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, silu, y, s); return true;
+    case 32: launch_ln_rows<TX, TY, 32, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, silu, y, s); return true;
+    case 64: launch_ln_rows<TX, TY, 64, 1, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, silu, y, s); return true;
+    case 128: launch_ln_rows<TX, TY, 64, 2, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, silu, y, s); return true;
+    case 256: launch_ln_rows<TX, TY, 64, 4, kMod>(x, rows, eps, gamma, beta, coords, bm, tm, off, silu, y, s); return true;
     default: return false;
     }
 }
@@ -776,30 +787,30 @@ bool try_ln_rows(const void * x, int64_t rows, int channels, float eps, const fl
 template <typename TX, typename TY, bool kMod>
 void launch_ln(const void * x, int64_t rows, int channels, float eps, const float * gamma,
                const float * beta, const int32_t * coords, const float * bm, const float * tm,
-               int off, void * y, hipStream_t s) {
+               int off, bool silu, void * y, hipStream_t s) {
 #ifndef PXS_LN_ROWS
 #define PXS_LN_ROWS 1
 #endif
     if (PXS_LN_ROWS &&
-        try_ln_rows<TX, TY, kMod>(x, rows, channels, eps, gamma, beta, coords, bm, tm, off, y, s))
+        try_ln_rows<TX, TY, kMod>(x, rows, channels, eps, gamma, beta, coords, bm, tm, off, silu, y, s))
         return;
     hipLaunchKernelGGL((layer_norm_kernel<TX, TY, kMod>), dim3(grid_for(rows, kRowsPerBlock)),
                        dim3(64 * kRowsPerBlock), 0, s, static_cast<const TX *>(x), rows, channels,
-                       eps, gamma, beta, coords, bm, tm, off, static_cast<TY *>(y));
+                       eps, gamma, beta, coords, bm, tm, off, silu, static_cast<TY *>(y));
 }
 
 template <bool kMod>
 int run_ln(int xd, const void * x, int64_t rows, int channels, float eps, const float * gamma,
            const float * beta, const int32_t * coords, const float * bm, const float * tm, int off,
-           int yd, void * y, hipStream_t s) {
+           int yd, void * y, hipStream_t s, bool silu = false) {
     if (xd == PXS_F32 && yd == PXS_F32)
-        launch_ln<float, float, kMod>(x, rows, channels, eps, gamma, beta, coords, bm, tm, off, y, s);
+        launch_ln<float, float, kMod>(x, rows, channels, eps, gamma, beta, coords, bm, tm, off, silu, y, s);
     else if (xd == PXS_F32 && yd == PXS_BF16)
-        launch_ln<float, uint16_t, kMod>(x, rows, channels, eps, gamma, beta, coords, bm, tm, off, y, s);
+        launch_ln<float, uint16_t, kMod>(x, rows, channels, eps, gamma, beta, coords, bm, tm, off, silu, y, s);
     else if (xd == PXS_BF16 && yd == PXS_F32)
-        launch_ln<uint16_t, float, kMod>(x, rows, channels, eps, gamma, beta, coords, bm, tm, off, y, s);
+        launch_ln<uint16_t, float, kMod>(x, rows, channels, eps, gamma, beta, coords, bm, tm, off, silu, y, s);
     else
-        launch_ln<uint16_t, uint16_t, kMod>(x, rows, channels, eps, gamma, beta, coords, bm, tm, off, y, s);
+        launch_ln<uint16_t, uint16_t, kMod>(x, rows, channels, eps, gamma, beta, coords, bm, tm, off, silu, y, s);
     return check_launch("layer norm");
 }
 
@@ -822,6 +833,49 @@ int run_head_op(const void * x, int64_t ld_x, int64_t rows, int heads, int head_
 }
 
 } // namespace
+// pxs_add_repeat, and where y16 is set a bf16 copy of y.
+int add_repeat(int a_dtype, const void * a, int64_t rows, int channels, const float * skip,
+               int skip_channels, float * y, uint16_t * y16, void * stream) {
+    PXS_CHECK(check_dtype(a_dtype), PXS_ERR_ARG, "pxs_add_repeat: bad dtype");
+    PXS_CHECK(rows >= 0 && channels > 0 && skip_channels > 0 && channels % skip_channels == 0,
+              PXS_ERR_ARG, "SLat decoder skip channels are not repeatable");
+    if (rows == 0) return PXS_OK;
+    PXS_CHECK(a && skip && y, PXS_ERR_ARG, "pxs_add_repeat: null pointer");
+    const int64_t count = rows * channels;
+    const int repeats = channels / skip_channels;
+    if (channels % 8 == 0 && count / 8 <= UINT32_MAX && vec8_ok(count, a, y) &&
+        (reinterpret_cast<uintptr_t>(y16) & 15) == 0) {
+        const uint32_t nv = static_cast<uint32_t>(count / 8), vpr = static_cast<uint32_t>(channels / 8);
+        if (a_dtype == PXS_F32)
+            hipLaunchKernelGGL(add_repeat8_kernel<float>, dim3(vec8_blocks(count)), dim3(256), 0,
+                               as_stream(stream), static_cast<const float *>(a), nv, vpr, skip,
+                               skip_channels, repeats, y, y16);
+        else
+            hipLaunchKernelGGL(add_repeat8_kernel<uint16_t>, dim3(vec8_blocks(count)), dim3(256), 0,
+                               as_stream(stream), static_cast<const uint16_t *>(a), nv, vpr, skip,
+                               skip_channels, repeats, y, y16);
+        return check_launch("pxs_add_repeat");
+    }
+    const unsigned blocks = static_cast<unsigned>(std::min<int64_t>((count + 255) / 256, 16384));
+    if (a_dtype == PXS_F32) {
+        hipLaunchKernelGGL(add_repeat_kernel<float>, dim3(blocks), dim3(256), 0, as_stream(stream),
+                           static_cast<const float *>(a), rows, channels, skip, skip_channels,
+                           repeats, y);
+    } else {
+        hipLaunchKernelGGL(add_repeat_kernel<uint16_t>, dim3(blocks), dim3(256), 0,
+                           as_stream(stream), static_cast<const uint16_t *>(a), rows, channels,
+                           skip, skip_channels, repeats, y);
+    }
+    if (int rc = check_launch("pxs_add_repeat")) return rc;
+    return y16 ? pxs_convert(PXS_F32, y, count, PXS_BF16, y16, stream) : PXS_OK;
+}
+
+int layer_norm_silu(int x_dtype, const void * x, int64_t rows, int channels, float eps,
+                    const float * gamma, const float * beta, int y_dtype, void * y, hipStream_t s) {
+    return run_ln<false>(x_dtype, x, rows, channels, eps, gamma, beta, nullptr, nullptr, nullptr, 0,
+                         y_dtype, y, s, true);
+}
+
 bool residual_norm_takes(int channels) { return channels % 256 == 0 && channels <= 1024; }
 
 int residual_norm(const ResidualNorm & a, int64_t rows, int channels, float * residual, int y_dtype,
@@ -1091,36 +1145,7 @@ int pxs_convert(int src_dtype, const void * x, int64_t count, int dst_dtype, voi
 
 int pxs_add_repeat(int a_dtype, const void * a, int64_t rows, int channels, const float * skip,
                    int skip_channels, float * y, void * stream) {
-    PXS_CHECK(check_dtype(a_dtype), PXS_ERR_ARG, "pxs_add_repeat: bad dtype");
-    PXS_CHECK(rows >= 0 && channels > 0 && skip_channels > 0 && channels % skip_channels == 0,
-              PXS_ERR_ARG, "SLat decoder skip channels are not repeatable");
-    if (rows == 0) return PXS_OK;
-    PXS_CHECK(a && skip && y, PXS_ERR_ARG, "pxs_add_repeat: null pointer");
-    const int64_t count = rows * channels;
-    const int repeats = channels / skip_channels;
-    if (channels % 8 == 0 && count / 8 <= UINT32_MAX && vec8_ok(count, a, y)) {
-        const uint32_t nv = static_cast<uint32_t>(count / 8), vpr = static_cast<uint32_t>(channels / 8);
-        if (a_dtype == PXS_F32)
-            hipLaunchKernelGGL(add_repeat8_kernel<float>, dim3(vec8_blocks(count)), dim3(256), 0,
-                               as_stream(stream), static_cast<const float *>(a), nv, vpr, skip,
-                               skip_channels, repeats, y);
-        else
-            hipLaunchKernelGGL(add_repeat8_kernel<uint16_t>, dim3(vec8_blocks(count)), dim3(256), 0,
-                               as_stream(stream), static_cast<const uint16_t *>(a), nv, vpr, skip,
-                               skip_channels, repeats, y);
-        return check_launch("pxs_add_repeat");
-    }
-    const unsigned blocks = static_cast<unsigned>(std::min<int64_t>((count + 255) / 256, 16384));
-    if (a_dtype == PXS_F32) {
-        hipLaunchKernelGGL(add_repeat_kernel<float>, dim3(blocks), dim3(256), 0, as_stream(stream),
-                           static_cast<const float *>(a), rows, channels, skip, skip_channels,
-                           repeats, y);
-    } else {
-        hipLaunchKernelGGL(add_repeat_kernel<uint16_t>, dim3(blocks), dim3(256), 0,
-                           as_stream(stream), static_cast<const uint16_t *>(a), rows, channels,
-                           skip, skip_channels, repeats, y);
-    }
-    return check_launch("pxs_add_repeat");
+    return add_repeat(a_dtype, a, rows, channels, skip, skip_channels, y, nullptr, stream);
 }
 
 int pxs_timestep_embedding(const float * timesteps, int64_t batch, int dim, int max_period,

@@ -65,6 +65,13 @@ bool residual_norm_takes(int channels);
 int residual_norm(const ResidualNorm & a, int64_t rows, int channels, float * residual, int y_dtype,
                   hipStream_t s);
 
+// pxs_layer_norm and then SiLU in place (pxs_activation), in one pass; same values.
+int layer_norm_silu(int x_dtype, const void * x, int64_t rows, int channels, float eps,
+                    const float * gamma, const float * beta, int y_dtype, void * y, hipStream_t s);
+// pxs_add_repeat, and where y16 is set a bf16 copy of y.
+int add_repeat(int a_dtype, const void * a, int64_t rows, int channels, const float * skip,
+               int skip_channels, float * y, uint16_t * y16, void * stream);
+
 // x_out = x_in + the ConvNeXt MLP (layer norm, linear, SiLU, linear) of y, bf16
 // operands, in one kernel (csrc/mlp.hip); x_out may be x_in.  *done is left
 // false for shapes and alignments it does not take.
