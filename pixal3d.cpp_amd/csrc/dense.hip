@@ -251,6 +251,21 @@ __device__ __forceinline__ void dense_store_staged(const DenseArgs & a, const f3
 template <int KB> __device__ __forceinline__ int piece_swz(int row);
 template <> __device__ __forceinline__ int piece_swz<128>(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
+// Waits until at most min(later, MAX) stages of PER instructions each are in
+// flight (s_waitcnt's count is a constant, six bits of it vmcnt).
+template <int MAX, int PER>
+__device__ __forceinline__ void wait_stages(int later) {
+    constexpr int n = MAX * PER;
+    static_assert(n < 64, "vmcnt has six bits");
+    if constexpr (MAX > 0) {
+        if (later < MAX) {
+            wait_stages<MAX - 1, PER>(later);
+            return;
+        }
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (n & 15) | ((n >> 4) << 14));
+}
+
 // NW waves in a WAVES_M x (NW / WAVES_M) grid, each owning a (BM / WAVES_M) x
 // (BN / WAVES_N) block of the tile; NSTAGE K chunks of KB bytes per row in
 // flight (one DMA instruction fills 1 KiB: 1024 / KB rows).
@@ -359,8 +374,7 @@ dense_gemm_kernel(DenseArgs a) {
         if (s < stages) issue(s);
 
     for (int s = 0; s < stages; ++s) {
-        const int after = min(NSTAGE - 2, stages - 1 - s);
-        wait_vmcnt(after * kPerStage);
+        wait_stages<NSTAGE - 2, kPerStage>(stages - 1 - s);
         barrier_no_fence();
         const bool more = s + NSTAGE - 1 < stages;
         if (!SPREAD && more) issue(s + NSTAGE - 1);
@@ -726,6 +740,13 @@ int dispatch_bf16(DenseArgs a, hipStream_t s) {
     if (a.n > 128 && t_a <= t_b) {
         a.group_m = 8;
         return launch_dense<uint16_t, 256, 256, 16, 4, 2, 128, EPI, true, true>(a, s);
+    }
+    // At most one 128 x 64 tile per CU: nothing else hides a workgroup's waits, so
+    // 8 waves of 32 x 32 and three stages (1,000 x 1024 -> 1024: 10.1 against 12.4
+    // us, 4096 -> 1024: 29 against 38 us; 300 x 1024 -> 4096: 10.2 against 12.5 us).
+    if (((a.m + 127) / 128) * ((a.n + 63) / 64) <= 256) {
+        a.group_m = 8;
+        return launch_dense<uint16_t, 128, 64, 8, 4, 3, 128, EPI, false, true>(a, s);
     }
     if (a.n <= 64 || t_c < t_b) {
         a.group_m = (a.n + 63) / 64 <= 4 ? 16 : 8;

@@ -693,23 +693,37 @@ residual_norm_kernel(ResidualNorm a, int64_t rows, float * __restrict__ residual
     const float * tm = nullptr;
     if (a.gate_offset >= 0 || a.mod_offset >= 0) tm = a.time_mod + static_cast<int64_t>(a.coords[row * 4]) * 6 * C;
     auto at = [](const float * p) { return *reinterpret_cast<const float4 *>(p); };
-    float4 v[NV];
+    // Every load of the row before the first use: at 1,288 rows the chain of
+    // dependent loads was the kernel's time.
+    constexpr int kMaxSplits = 4;
+    float4 part[kMaxSplits][NV], v[NV], b[NV], g[NV], t[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        const int c = (j * 64 + lane) * 4;
+#pragma unroll
+        for (int q = 0; q < kMaxSplits; ++q)
+            if (q < a.splits) part[q][j] = at(a.partial + (q * rows + row) * C + c);
+        v[j] = at(residual + row * C + c);
+        b[j] = at(a.bias + c);
+        if (a.gate_offset >= 0) {
+            g[j] = at(a.block_mod + a.gate_offset + c);
+            t[j] = at(tm + a.gate_offset + c);
+        }
+    }
     float s = 0.0f;
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         const int c = (j * 64 + lane) * 4;
-        float4 u = at(a.partial + row * C + c);
-        for (int q = 1; q < a.splits; ++q) {
-            const float4 w = at(a.partial + (q * rows + row) * C + c);
-            u.x += w.x; u.y += w.y; u.z += w.z; u.w += w.w;
+        float4 u = part[0][j];
+#pragma unroll
+        for (int q = 1; q < kMaxSplits; ++q) {
+            if (q >= a.splits) break;
+            u.x += part[q][j].x; u.y += part[q][j].y; u.z += part[q][j].z; u.w += part[q][j].w;
         }
-        const float4 b = at(a.bias + c);
-        u.x += b.x; u.y += b.y; u.z += b.z; u.w += b.w;
+        u.x += b[j].x; u.y += b[j].y; u.z += b[j].z; u.w += b[j].w;
         if (a.gate_offset >= 0) {
-            const float4 g = at(a.block_mod + a.gate_offset + c), t = at(tm + a.gate_offset + c);
-            u.x *= g.x + t.x; u.y *= g.y + t.y; u.z *= g.z + t.z; u.w *= g.w + t.w;
+            u.x *= g[j].x + t[j].x; u.y *= g[j].y + t[j].y; u.z *= g[j].z + t[j].z; u.w *= g[j].w + t[j].w;
         }
-        v[j] = at(residual + row * C + c);
         v[j].x += u.x; v[j].y += u.y; v[j].z += u.z; v[j].w += u.w;
         *reinterpret_cast<float4 *>(residual + row * C + c) = v[j];
         s += v[j].x; s += v[j].y; s += v[j].z; s += v[j].w;
