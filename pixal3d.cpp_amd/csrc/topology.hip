@@ -1016,18 +1016,58 @@ __global__ void window_place_kernel(const int4 * __restrict__ coords, int64_t n,
     tmp[start[wid] + slot[p]] = static_cast<int32_t>(p);
 }
 
+// Ranks of R members per thread (thread t: members t, t + kThreads, ...) among
+// the len members staged in LDS, padded to a multiple of 4 by INT_MAX.
+template <int R>
+__device__ __forceinline__ void window_rank(const int32_t * members, int len, int64_t begin,
+                                            int32_t * __restrict__ fwd, int32_t * __restrict__ bwd) {
+    int32_t mine[R], rank[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+        const int i = static_cast<int>(threadIdx.x) + q * kThreads;
+        mine[q] = i < len ? members[i] : 0;
+        rank[q] = 0;
+    }
+    const int4 * m4 = reinterpret_cast<const int4 *>(members);
+    for (int j = 0; j < (len + 3) / 4; ++j) {
+        const int4 m = m4[j];
+#pragma unroll
+        for (int q = 0; q < R; ++q)
+            rank[q] += (m.x < mine[q]) + (m.y < mine[q]) + (m.z < mine[q]) + (m.w < mine[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+        const int i = static_cast<int>(threadIdx.x) + q * kThreads;
+        if (i < len) {
+            fwd[begin + rank[q]] = mine[q];
+            bwd[mine[q]] = static_cast<int32_t>(begin + rank[q]);
+        }
+    }
+}
+
 // One workgroup per window: rank each member by counting smaller row
-// indices (rows are unique), giving the stable order.  Windows hold at most
-// window^3 rows; larger segments are ranked in LDS chunks.
+// indices (rows are unique), giving the stable order.  Windows of up to 1,024
+// members (8^3 hold at most 512) are staged once and compared four at a time;
+// larger ones are ranked in LDS chunks.
 __global__ void __launch_bounds__(kThreads)
 window_sort_kernel(const int32_t * __restrict__ tmp, const int64_t * __restrict__ cu,
                    const int64_t * __restrict__ nwin, int32_t * __restrict__ fwd,
                    int32_t * __restrict__ bwd) {
-    __shared__ int32_t members[1024];
+    __shared__ __align__(16) int32_t members[1024];
     const int64_t w = blockIdx.x;
     if (w >= *nwin) return;
     const int64_t begin = cu[w], end = cu[w + 1];
     const int64_t len = end - begin;
+    if (len <= 1024) {
+        const int count = static_cast<int>(len);
+        for (int j = threadIdx.x; j < (count + 3) / 4 * 4; j += kThreads)
+            members[j] = j < count ? tmp[begin + j] : INT_MAX;
+        __syncthreads();
+        if (count <= kThreads) window_rank<1>(members, count, begin, fwd, bwd);
+        else if (count <= 2 * kThreads) window_rank<2>(members, count, begin, fwd, bwd);
+        else window_rank<4>(members, count, begin, fwd, bwd);
+        return;
+    }
     for (int64_t i0 = 0; i0 < len; i0 += kThreads) {
         const int64_t i = i0 + threadIdx.x;
         const int32_t mine = i < len ? tmp[begin + i] : INT_MAX;
