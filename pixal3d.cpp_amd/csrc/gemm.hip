@@ -939,8 +939,11 @@ __device__ __forceinline__ void gemm_lds_tile(const GemmArgs & a, int logical, c
     // thread of the launch).
     constexpr int kStagedPitch = BN * 2 + 16;
     constexpr bool kStageable =
-        EPI == kEpiStore && sizeof(T) == 2 && BM * kStagedPitch <= NSTAGE * kStageBytes;
-    const bool staged = kStageable && a.cout % 8 == 0 && a.ldy % 8 == 0 &&
+        EPI == kEpiStore && sizeof(T) == 2 && BM * kStagedPitch <= lds_gemm_bytes<BM, BN, NSTAGE>(27);
+    // (A 256 x 256 tile reaches into the source table of 27 offsets, which no
+    // wave reads any more.)
+    const bool staged = kStageable && BM * kStagedPitch <= NSTAGE * kStageBytes + a.noff * BM * 4 &&
+                        a.cout % 8 == 0 && a.ldy % 8 == 0 &&
                         (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
     if constexpr (KSPLIT == 1) {
         if constexpr (CHILD) {
