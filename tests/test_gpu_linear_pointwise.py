@@ -23,6 +23,22 @@ def orc():
     return O.Oracle()
 
 
+@pytest.mark.parametrize("rows,cin,cout,act", [(1, 4, 1, 0), (2, 252, 7, 2), (3, 260, 130, 1),
+                                              (4, 1024, 513, 0), (5, 1024, 40, 2)])
+def test_linear_fp32_few_rows(px, orc, rows, cin, cout, act):
+    """One wave per output up to 4 rows (K below, at and past a wave's 256
+    values), the tiled kernel from 5."""
+    x = W.normal(56, rows * cin, 1).reshape(rows, cin)
+    w = W.normal(56, cout * cin, 2, std=cin ** -0.5).reshape(cout, cin)
+    b = W.normal(56, cout, 3)
+    ref = orc.linear(x, w, b).astype(np.float64)
+    if act == 1:
+        ref = 0.5 * ref * (1.0 + np.tanh(np.sqrt(2.0 / np.pi) * (ref + 0.044715 * ref ** 3)))
+    elif act == 2:
+        ref = ref / (1.0 + np.exp(-ref))
+    assert_fp32(host(px.linear(t32(x), t32(w), t32(b), act=act)), ref, what="linear few rows")
+
+
 @pytest.mark.parametrize("rows,cin,cout", [(200, 24, 40), (1000, 64, 64), (777, 256, 384),
                                           (300, 8, 1024), (513, 1024, 8), (5, 3, 4)])
 def test_linear_fp32(px, orc, rows, cin, cout):
