@@ -40,6 +40,7 @@
 // chosen per shape by the number of rounds of tiles over the 256 CUs.
 
 #include "pxs_common.h"
+#include "split3.h"
 
 #include <algorithm>
 
@@ -429,10 +430,8 @@ dense_gemm_kernel(DenseArgs a) {
 }
 
 // ---- fp32 products on the bf16 matrix cores --------------------------------
-// Each fp32 operand is split without loss into three bf16 terms, a = a1 + a2 +
-// a3 (each the rounding of what the ones before leave), and a product takes
-// the six terms above 2^-26 of it: a1 b1, a1 b2, a2 b1, a2 b2, a1 b3, a3 b1.
-// Six v_mfma_f32_32x32x16_bf16 cost 192 matrix-core cycles where the eight
+// Each fp32 operand is split into three bf16 terms and a product takes six of
+// their products (split3.h).  Six v_mfma_f32_32x32x16_bf16 cost 192 matrix-core cycles where the eight
 // v_mfma_f32_32x32x2_f32 of the same 16 K steps cost 512.  Against 64-bit
 // products of N(0, 1) operands the results are closer than that instruction's:
 // relative error (2-norm) 3.4e-7 against 4.0e-7 at K = 1024, 7.1e-7 against
@@ -445,38 +444,6 @@ dense_gemm_kernel(DenseArgs a) {
 // 4096: 224 against 315; 1,000 x 4096 -> 1024: 105 against 155.  Tiles of 256 x
 // 256 or 256 x 128 (8 or 16 waves, one workgroup per CU) ran slower: 683-1,173
 // us on the first shape.
-//
-// Valid while no operand exceeds 2^50 in magnitude and no sum is nonzero below
-// 2^-60: operands below 2^-102 lose low bits to bf16's least exponent, which
-// moves a sum by at most K 2^-84.  A tile that meets a larger operand, or ends
-// with a smaller or a non-finite sum (as any infinity or NaN operand gives), is
-// computed again on v_mfma_f32_32x32x2_f32 from global memory.
-constexpr float kSplitHigh = 0x1p50f, kSplitLow = 0x1p-60f;
-
-// Splits 4 values into the three planes' 8-byte pieces; hi follows the largest
-// magnitude seen.
-__device__ __forceinline__ void split4(const float4 & f, uint2 (&out)[3], float & hi) {
-    const float v[4] = {f.x, f.y, f.z, f.w};
-    uint32_t w[3][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        float a = v[2 * i], b = v[2 * i + 1];
-        hi = fmaxf(hi, fmaxf(fabsf(a), fabsf(b)));
-#pragma unroll
-        for (int q = 0; q < 3; ++q) {
-            uint32_t pk = pack_bf16x2(a, b);
-            asm("" : "+v"(pk));  // one conversion, not one more to take the low half apart
-            w[q][i] = pk;
-            if (q < 2) {
-                a = a - __builtin_bit_cast(float, pk << 16);
-                b = b - __builtin_bit_cast(float, pk & 0xffff0000u);
-            }
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) out[q] = make_uint2(w[q][0], w[q][1]);
-}
-
 // One tile of BM x BN, NWM x NWN waves.  Per 32-element K chunk every thread
 // splits its share of the X and W rows (loaded into registers while the chunk
 // before is multiplied) and writes the planes to LDS as [plane][8-element
@@ -606,13 +573,11 @@ dense_split_kernel(DenseArgs a) {
                 for (int q = 0; q < 3; ++q)
                     wf[q] = *reinterpret_cast<const bf16x8 *>(
                         sw + q * kPlaneW + (2 * u + h) * kColW + (wn * WN + j * 32 + r) * 16);
-                // the smaller terms first
-                constexpr int kTermX[6] = {2, 0, 1, 1, 0, 0}, kTermW[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
                 for (int t = 0; t < 6; ++t)
 #pragma unroll
                     for (int i = 0; i < TI; ++i)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[kTermW[t]], xf[kTermX[t]][i],
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[kSplitTermB[t]], xf[kSplitTermA[t]][i],
                                                                             acc[i][j], 0, 0, 0);
             }
         }
@@ -623,10 +588,7 @@ dense_split_kernel(DenseArgs a) {
 #pragma unroll
         for (int j = 0; j < TJ; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const float m = fabsf(acc[i][j][v]);
-                odd |= !(m == 0.0f || (m >= kSplitLow && m < INFINITY));
-            }
+            for (int v = 0; v < 16; ++v) odd |= split_sum_odd(acc[i][j][v]);
     if (__syncthreads_or(odd)) {
         // rare: the whole tile again in fp32
 #pragma unroll

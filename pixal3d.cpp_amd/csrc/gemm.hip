@@ -20,6 +20,7 @@
 
 #include "pxs_common.h"
 #include "s2emit.h"
+#include "split3.h"
 #include "scan.h"
 
 #include <algorithm>
@@ -1689,23 +1690,21 @@ int launch_range_conv(const GemmArgs & args, hipStream_t stream) {
 
 // ---------------------------------------------------------------------------
 // fp32 split-K gather GEMM (SubMConv3d and linears in fp32).  A workgroup
-// owns 32*TI output rows x 64 output channels; its (offset, 32-channel chunk)
+// owns 32 output rows x 64 output channels; its (offset, 32-channel chunk)
 // steps are dealt round-robin to its NW waves, so even a few hundred tiles
 // keep every CU busy.  Each wave loads its operands straight into VGPRs --
-// lane (h, r) takes the 64 contiguous bytes k = 16h .. 16h+15 of A row r (of
-// each 32-row block) and of weight row r, the same K permutation on both
-// sides of v_mfma_f32_32x32x2_f32 -- with the next step's loads in flight
-// during the current step's MFMAs, and no barrier until the end, where waves
-// 1 and up hand their partial sums to wave 0 through LDS (a fixed summation order:
+// lane (h, r) takes the 64 contiguous bytes k = 16h .. 16h+15 of A row r and
+// of weight row r, the same K permutation on both sides of
+// v_mfma_f32_32x32x2_f32 -- with the next step's loads in flight during the
+// current step's MFMAs, and no barrier until the end, where waves 1 and up hand
+// their partial sums to wave 0 through LDS (a fixed summation order:
 // deterministic).  The operand loads return through the per-CU vector-memory
-// path, which bounds the kernel: TI = 2 reads each weight chunk once for 64
-// rows instead of 32 (16 KB per 64x64x32 step instead of 24 KB), at 64
-// accumulator registers per lane.
+// path, which bounds the kernel.
 
-template <int EPI, int TI, int NW>
+template <int EPI, int NW>
 __global__ void __launch_bounds__(NW * 64)
 split_gemm_f32_kernel(GemmArgs a) {
-    constexpr int BM = 32 * TI, BN = 64;
+    constexpr int TI = 1, BM = 32 * TI, BN = 64;  // 32-row blocks per tile
     __shared__ float red[NW - 1][TI * 2][16][64];
     __shared__ int32_t idx_lds[32 * BM];
     __shared__ uint32_t tile_mask;
@@ -1861,42 +1860,191 @@ split_gemm_f32_kernel(GemmArgs a) {
 #ifndef PXS_SPLIT_F32
 #define PXS_SPLIT_F32 1
 #endif
-// 64-row tiles (one workgroup, one wave per SIMD, per CU) for grids of
-// about one to four rounds over the 256 CUs; past that, 32-row tiles at two
-// workgroups per CU hide more latency.  Measured on SubMConv3d over shell
-// voxels: 64 -> 64 at 16k rows 57 against 67 us, 128 -> 128 at 8k-32k rows
-// 0.79-0.89x; at 8k rows 64 -> 64 (128 wide tiles) 1.66x slower, at 96k rows
-// 1.03-1.12x slower.
-#ifndef PXS_SPLIT_F32_WIDE_MIN
-#define PXS_SPLIT_F32_WIDE_MIN 224
-#endif
-#ifndef PXS_SPLIT_F32_WIDE_MAX
-#define PXS_SPLIT_F32_WIDE_MAX 1024
-#endif
 
-template <int EPI, int TI, int NW>
-int launch_split_f32_ti(const GemmArgs & args, hipStream_t stream) {
-    const int64_t tiles_m = (args.m + 32 * TI - 1) / (32 * TI);
+// fp32 SubMConv3d on the bf16 matrix cores (split3.h), for enough rows to
+// fill the CUs: 64 x 64 tiles, 4 waves of 32 x 32.  Per (offset, 32-channel
+// chunk) every thread splits two 16-byte pieces of gathered rows and two of
+// weight rows, loaded into registers two steps ahead, into planes in LDS laid
+// out as in dense_split_kernel.  Bound by the split's vector instructions and,
+// below a few tiles per CU, by a step's latency.
+__global__ void __launch_bounds__(256)
+split_conv_f32_kernel(GemmArgs a) {
+    constexpr int BM = 64, BN = 64, NT = 256;
+    constexpr int kCol = 64 * 16 + 64, kPlane = 4 * kCol;  // bytes of a piece column, of a plane
+    __shared__ __align__(16) char sx[3 * kPlane], sw[3 * kPlane];
+    __shared__ int32_t idx_lds[32 * BM];
+    __shared__ uint32_t tile_mask;
+    __shared__ int koff[32];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const int h = lane >> 5, r = lane & 31;
+    const int tiles_n = (a.cout + BN - 1) / BN;
+    const int logical = remap_xcd(blockIdx.x, gridDim.x);
+    const int64_t p0 = static_cast<int64_t>(logical / tiles_n) * BM;
+    const int n0 = (logical % tiles_n) * BN;
+    const float * __restrict__ x = static_cast<const float *>(a.x);
+    const float * __restrict__ w = static_cast<const float *>(a.w);
+
+    if (tid == 0) tile_mask = 0;
+    __syncthreads();
+    if (a.grid) {
+        grid_tile_sources<BM>(a, p0, tid, NT, idx_lds, &tile_mask);
+    } else {
+        uint32_t local = 0;
+        for (int e = tid; e < a.noff * BM; e += NT) {
+            const int k = e / BM, row = e % BM;
+            int32_t src = -1;
+            if (p0 + row < a.m) {
+                const int32_t v = a.rowmap[k * a.ld_map + p0 + row];
+                src = (v >= 0 && v < a.rows_in) ? v : -1;
+            }
+            idx_lds[e] = src;
+            if (src >= 0) local |= 1u << k;
+        }
+        if (local) atomicOr(&tile_mask, local);
+    }
+    __syncthreads();
+    const uint32_t present = tile_mask & ((1u << a.noff) - 1u);
+    const int kcount = __popc(present);
+    if (tid < 32 && (present >> tid & 1u)) koff[__popc(present & ((1u << tid) - 1u))] = tid;
+    __syncthreads();
+
+    const int chunks = (a.cin + 31) / 32;
+    const int steps = kcount * chunks;
+    const int piece = tid & 7, row = tid >> 3;
+    const float * zero = reinterpret_cast<const float *>(g_zero_chunk);
+    int next = 0, next_i = 0, next_chunk = 0;  // the step to load next
+    struct Pieces {
+        float4 x[2], w[2];
+    };
+    auto load = [&](Pieces & v) __attribute__((always_inline)) {
+        const bool live = next < steps;
+        const int k = live ? koff[next_i] : 0;
+        const int col = next_chunk * 32 + piece * 4;
+        const bool in = live && col < a.cin;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int32_t src = in ? idx_lds[k * BM + row + 32 * q] : -1;
+            v.x[q] = *reinterpret_cast<const float4 *>(src >= 0 ? x + static_cast<int64_t>(src) * a.ldx + col : zero);
+            const int n = n0 + row + 32 * q;
+            v.w[q] = *reinterpret_cast<const float4 *>(
+                in && n < a.cout ? w + (static_cast<int64_t>(k) * a.cout + n) * a.cin + col : zero);
+        }
+        ++next;
+        if (++next_chunk == chunks) {
+            next_chunk = 0;
+            ++next_i;
+        }
+    };
+
+    // Chains of sums: the leading term and the other five apart, each for both
+    // 16-channel halves.  The other five are 2^-8 of the leading one, so a sum is
+    // rounded at its own size once per 16 products.
+    f32x16 lead[2], rest[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) lead[u][v] = rest[u][v] = 0.0f;
+    float hi = 0.0f;
+    const int at = (piece >> 1) * kCol + row * 16 + (piece & 1) * 8;
+    auto step = [&](Pieces & v) __attribute__((always_inline)) {
+        barrier_no_fence();  // every wave has read the previous step's planes
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            uint2 t[3];
+            split4(v.x[q], t, hi);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2 *>(sx + p * kPlane + at + q * 512) = t[p];
+            split4(v.w[q], t, hi);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2 *>(sw + p * kPlane + at + q * 512) = t[p];
+        }
+        load(v);
+        barrier_no_fence();
+        bf16x8 xf[2][3], wf[2][3];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) {
+                xf[u][p] = *reinterpret_cast<const bf16x8 *>(sx + p * kPlane + (2 * u + h) * kCol + (wm * 32 + r) * 16);
+                wf[u][p] = *reinterpret_cast<const bf16x8 *>(sw + p * kPlane + (2 * u + h) * kCol + (wn * 32 + r) * 16);
+            }
+#pragma unroll
+        for (int t = 0; t < 6; ++t)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                f32x16 & sum = t == 5 ? lead[u] : rest[u];
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[u][kSplitTermA[t]], wf[u][kSplitTermB[t]],
+                                                              sum, 0, 0, 0);
+            }
+    };
+    Pieces even, odd_step;
+    load(even);
+    load(odd_step);
+    for (int s = 0; s < steps; s += 2) {
+        step(even);
+        if (s + 1 < steps) step(odd_step);
+    }
+    f32x16 sum[1][1];
+    bool odd = hi > kSplitHigh;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        sum[0][0][v] = (lead[0][v] + lead[1][v]) + (rest[0][v] + rest[1][v]);
+        odd |= split_sum_odd(sum[0][0][v]);
+    }
+    if (__syncthreads_or(odd)) {
+        // rare: the tile again on the fp32 matrix instruction
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sum[0][0][v] = 0.0f;
+        const int n = n0 + wn * 32 + r;
+        for (int i = 0; i < kcount; ++i) {
+            const int k = koff[i];
+            const int32_t src = idx_lds[k * BM + wm * 32 + r];
+            const float * xr = x + static_cast<int64_t>(src < 0 ? 0 : src) * a.ldx;
+            const float * wr = w + (static_cast<int64_t>(k) * a.cout + (n < a.cout ? n : 0)) * a.cin;
+            for (int c = h; c < a.cin; c += 2)  // cin is a multiple of 4
+                sum[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(src < 0 ? 0.0f : xr[c], wr[c], sum[0][0], 0, 0, 0);
+        }
+    }
+    gemm_epilogue<float, 1, 1, 32, 32, kEpiStore>(a, sum, p0, n0, wm, wn, h, r);
+}
+
+int launch_split_conv_f32(const GemmArgs & args, hipStream_t stream) {
+    const int64_t blocks = ((args.m + 63) / 64) * ((args.cout + 63) / 64);
+    if (blocks > INT32_MAX) return fail(PXS_ERR_ARG, "gather GEMM grid too large");
+    hipLaunchKernelGGL(split_conv_f32_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, args);
+    return check_launch("SubMConv3d (fp32 split)");
+}
+
+template <int EPI, int NW>
+int launch_split_f32_waves(const GemmArgs & args, hipStream_t stream) {
+    const int64_t tiles_m = (args.m + 31) / 32;
     const int64_t tiles_n = (args.cout + 63) / 64;
     const int64_t blocks = tiles_m * tiles_n;
     if (blocks > INT32_MAX) return fail(PXS_ERR_ARG, "gather GEMM grid too large");
-    hipLaunchKernelGGL((split_gemm_f32_kernel<EPI, TI, NW>), dim3(static_cast<unsigned>(blocks)),
+    hipLaunchKernelGGL((split_gemm_f32_kernel<EPI, NW>), dim3(static_cast<unsigned>(blocks)),
                        dim3(NW * 64), 0, stream, args);
     return check_launch("gather GEMM (fp32 split-K)");
 }
 
 template <int EPI>
 int launch_split_f32(const GemmArgs & args, hipStream_t stream) {
-    const int64_t wide = ((args.m + 63) / 64) * ((args.cout + 63) / 64);
-    // (Only for the 27-offset gathers: plain linears, with 2 K steps per
-    // tile, run 1.5x slower on 64-row tiles, 19 against 13 us at 16k x 64.)
     const bool gather = (args.rowmap || args.grid) && args.noff >= 27;
-    if (gather && wide >= PXS_SPLIT_F32_WIDE_MIN && wide <= PXS_SPLIT_F32_WIDE_MAX)
-        return launch_split_f32_ti<EPI, 2, 4>(args, stream);
+    // 64 x 64 tiles for nearly every CU: the split kernel.  Against this file's
+    // fp32 tiles (the whole call over a grid, us): 64 -> 64 at 22,032 rows (345
+    // tiles) 83 against 103, 88,448 rows 227 against 277; 96 -> 192 at 8,912 rows
+    // (420) 118 against 138; 128 -> 128 at 8,912 rows (280) 153 against 166; 16 -> 36
+    // at 22,032 rows 46 against 69; at 140 tiles the same, below up to 1.7 times as
+    // long.  Errors against 64 bits are 0.45 to 0.65 of the fp32 tiles'.
+    const int64_t squares = ((args.m + 63) / 64) * ((args.cout + 63) / 64);
+    if (EPI == kEpiStore && gather && args.noff < 32 && squares >= 224) return launch_split_conv_f32(args, stream);
     // At most one tile per CU: twice the waves halve each one's chain of steps.
     const int64_t tiles = ((args.m + 31) / 32) * ((args.cout + 63) / 64);
-    if (gather && tiles <= 256) return launch_split_f32_ti<EPI, 1, 8>(args, stream);
-    return launch_split_f32_ti<EPI, 1, 4>(args, stream);
+    if (gather && tiles <= 256) return launch_split_f32_waves<EPI, 8>(args, stream);
+    return launch_split_f32_waves<EPI, 4>(args, stream);
 }
 
 template <typename T, int BM, int BN, int EPI, int NSTAGE, int NW, int WAVES_M, int KSPLIT>

@@ -5,6 +5,7 @@ from pathlib import Path
 
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 import workloads as W
@@ -259,3 +260,45 @@ def test_unet_stage_conv_c_full_size(px):
     eye[13] = np.eye(256, dtype=np.float32)
     yi = px.subm_conv3d(xb, tbf(eye), t32(np.zeros(256)), nbr, masks)
     np.testing.assert_array_equal(host(yi), host(xb))
+
+
+# fp32 convolutions of at least 224 tiles of 64 x 64 multiply operands split into
+# three bf16 terms: ragged rows, a ragged last K chunk, one chunk and several
+# (odd and even step counts), output widths that leave a column tile part empty,
+# neighbours from a map and from a grid, and one row of values out of the
+# split's range, whose tile and its neighbours' run in fp32.
+@pytest.mark.parametrize("cin,cout", [(4, 130), (36, 192), (64, 200), (128, 129)])
+@pytest.mark.parametrize("odd", [False, True])
+def test_subm_conv3d_fp32_split(px, cin, cout, odd):
+    """Against 64-bit sums: within K 2^-24 sum |x w| (the bound of a K-term sum
+    rounded at every step), infinities and NaN where the sums have them."""
+    dev = torch.device("cuda:0")
+    coords = ti32(W.shell_coords(48, [[(11.0, 16.0)], [(9.0, 13.0)]], 48))
+    n = coords.shape[0]
+    assert ((n + 63) // 64) * ((cout + 63) // 64) >= 224
+    g = torch.Generator(device=dev).manual_seed(cin + cout)
+    x = torch.randn(n, cin, generator=g, device=dev)
+    if odd:
+        x[n // 2, 0], x[n // 3, 1], x[n // 4] = float("inf"), float("nan"), 1e20
+    w = torch.randn(27, cout, cin, generator=g, device=dev)
+    b = torch.randn(cout, generator=g, device=dev)
+    print(f"[conv fp32 split] n={n} {cin}->{cout} odd={odd}", flush=True)
+    nbr, masks = px.neighbor_map(coords)
+    y = px.subm_conv3d(x, w, b, nbr, masks)
+    grid = px.grid_build(coords, 2, (48, 48, 48))
+    assert torch.equal(px.subm_conv3d_grid(x, w, b, coords, 2, (48, 48, 48), grid).nan_to_num(),
+                       y.nan_to_num())
+    ref = b.double().repeat(n, 1)
+    room = ref.abs()
+    for k in range(27):
+        rows = (nbr[k] != n).nonzero()[:, 0]
+        xs = x[nbr[k][rows].long()].double()
+        ref[rows] += xs @ w[k].double().t()
+        room[rows] += xs.abs() @ w[k].double().abs().t()
+    ok = torch.isfinite(ref)
+    y = y.double()
+    assert torch.equal(torch.isnan(y), torch.isnan(ref))
+    assert torch.equal(y[torch.isinf(ref)], ref[torch.isinf(ref)])
+    over = torch.nan_to_num(torch.where(ok, (y - ref).abs() / (room * 27 * cin * 2.0 ** -24),
+                                        torch.zeros_like(ref)))
+    assert over.max() <= 1.0, over.max()
