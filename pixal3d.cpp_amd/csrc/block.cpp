@@ -14,6 +14,7 @@
 #include "pxs_common.h"
 #include "scan.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace pxs {
@@ -124,7 +125,7 @@ int run_block(int dtype, const pxs_block_config & cfg, const pxs_block_weights &
               const int32_t * coords, int64_t rows, int batch_size, const int64_t * cu_rows,
               float * hidden, const float * time_mod, const void * context,
               const int64_t * context_offsets, int64_t tokens, const void * projected,
-              const BlockBuffers & b, void * stream) {
+              const BlockBuffers & b, const void * context_kv, void * stream) {
     const int C = cfg.channels, H = cfg.num_heads, hd = C / H;
     const float scale = 1.0f / std::sqrt(static_cast<float>(hd));
     const size_t e = dtype_bytes(dtype);
@@ -153,17 +154,21 @@ int run_block(int dtype, const pxs_block_config & cfg, const pxs_block_weights &
     if (cfg.qk_rms_norm_cross) {
         PXS_TRY(pxs_mh_rms_norm(dtype, b.q, C, rows, H, hd, w.cross_q_gamma, b.q, C, stream));
     }
-    PXS_TRY(pxs_linear(dtype, context, tokens, cfg.context_channels, w.cross_to_kv_weight,
-                       w.cross_to_kv_bias, 2 * C, PXS_ACT_NONE, b.ckv, stream));
-    const void * ck = b.ckv;
+    const void * ckv = context_kv;  // this block's keys and values, when made ahead
+    if (!ckv) {
+        PXS_TRY(pxs_linear(dtype, context, tokens, cfg.context_channels, w.cross_to_kv_weight,
+                           w.cross_to_kv_bias, 2 * C, PXS_ACT_NONE, b.ckv, stream));
+        ckv = b.ckv;
+    }
+    const void * ck = ckv;
     int64_t ld_k = 2 * C;
     if (cfg.qk_rms_norm_cross) {
-        PXS_TRY(pxs_mh_rms_norm(dtype, b.ckv, 2 * C, tokens, H, hd, w.cross_k_gamma, b.ck, C,
+        PXS_TRY(pxs_mh_rms_norm(dtype, ckv, 2 * C, tokens, H, hd, w.cross_k_gamma, b.ck, C,
                                 stream));
         ck = b.ck;
         ld_k = C;
     }
-    const void * cv = static_cast<const char *>(b.ckv) + static_cast<size_t>(C) * e;
+    const void * cv = static_cast<const char *>(ckv) + static_cast<size_t>(C) * e;
     PXS_TRY(pxs_varlen_attention(dtype, b.q, C, ck, ld_k, cv, 2 * C, cu_rows, context_offsets,
                                  batch_size, rows, nullptr, H, hd, hd, scale, b.att, C, b.attn_ws,
                                  stream));
@@ -210,8 +215,21 @@ struct FlowBuffers {
     float * temb1;    // [batch, C]
     float * temb2;    // [batch, C]
     float * time_mod; // [batch, 6C]
+    void * context_kv;  // [blocks, tokens, 2C], or null: made block by block
     BlockBuffers block;
 };
+
+// The context's keys and values depend on no block's state.  For small objects
+// one launch makes them for every block: 24 x (1,370 x 1024 -> 2048) took 24 x
+// 17.4 us, each linear filling the CUs badly, and together 150 us.  With many
+// rows those launches are a small part, and the buffer is bounded.
+constexpr int64_t kContextAheadRows = 8192;
+constexpr int64_t kContextAheadBytes = int64_t{1} << 29;
+bool context_ahead(int dtype, const pxs_flow_config & f, int64_t rows, int64_t tokens) {
+    return dtype == PXS_BF16 && f.num_blocks > 1 && rows <= kContextAheadRows && tokens > 0 &&
+           dense_group_takes(f.cond_channels, 2 * f.model_channels) &&
+           tokens <= kContextAheadBytes / (int64_t{4} * f.model_channels * f.num_blocks);
+}
 
 constexpr int kTimestepFreqDim = 256;  // src/slat_flow.cpp:209
 
@@ -228,6 +246,9 @@ FlowBuffers carve_flow(Carver & c, int dtype, const pxs_flow_config & f, int64_t
     b.temb2 = static_cast<float *>(c.take(bs * C * 4));
     b.time_mod = static_cast<float *>(c.take(bs * 6 * C * 4));
     const pxs_block_config bc = flow_block_config(f);
+    b.context_kv = context_ahead(dtype, f, rows, tokens)
+                       ? c.take(static_cast<size_t>(f.num_blocks) * tokens * 2 * C * 2)
+                       : nullptr;
     b.block = carve_block(c, dtype, bc, rows, tokens, batch_size);
     return b;
 }
@@ -268,7 +289,7 @@ int pxs_transformer_block(int dtype, const pxs_block_config * cfg, const pxs_blo
     Carver c(workspace);
     const BlockBuffers b = carve_block(c, dtype, *cfg, rows, context_tokens, batch_size);
     return run_block(dtype, *cfg, *w, coords, rows, batch_size, cu_rows, hidden, time_mod, context,
-                     context_offsets, context_tokens, projected, b, stream);
+                     context_offsets, context_tokens, projected, b, nullptr, stream);
 }
 
 size_t pxs_slat_flow_workspace_bytes(int dtype, const pxs_flow_config * cfg, int64_t rows,
@@ -322,10 +343,27 @@ int pxs_slat_flow_forward(int dtype, const pxs_flow_config * cfg, const pxs_flow
                        PXS_ACT_SILU, b.temb2, stream));
     PXS_TRY(pxs_linear(PXS_F32, b.temb2, batch_size, C, w->modulation_weight, w->modulation_bias,
                        6 * C, PXS_ACT_NONE, b.time_mod, stream));
+    bool ahead = context_ahead(dtype, *cfg, rows, context_tokens) && aligned16(context);
+    for (int i = 0; ahead && i < cfg->num_blocks; ++i)
+        ahead = aligned16(w->blocks[i].cross_to_kv_weight) && aligned16(w->blocks[i].cross_to_kv_bias);
+    for (int g0 = 0; ahead && g0 < cfg->num_blocks; g0 += kDenseGroup) {
+        const void * weight[kDenseGroup];
+        const float * bias[kDenseGroup];
+        const int count = std::min(kDenseGroup, cfg->num_blocks - g0);
+        for (int i = 0; i < count; ++i) {
+            weight[i] = w->blocks[g0 + i].cross_to_kv_weight;
+            bias[i] = w->blocks[g0 + i].cross_to_kv_bias;
+        }
+        PXS_TRY(dense_linear_group(context, context_tokens, cfg->cond_channels, weight, bias, count, 2 * C,
+                                   static_cast<uint16_t *>(b.context_kv) + g0 * context_tokens * 2 * C, s));
+    }
     for (int i = 0; i < cfg->num_blocks; ++i) {
+        const void * context_kv =
+            ahead ? static_cast<const uint16_t *>(b.context_kv) + static_cast<int64_t>(i) * context_tokens * 2 * C
+                  : nullptr;
         PXS_TRY(run_block(dtype, bc, w->blocks[i], coords, rows, batch_size, cu_rows, b.hidden,
                           b.time_mod, context, context_offsets, context_tokens, projected, b.block,
-                          stream));
+                          context_kv, stream));
     }
     // Final layer norm keeps eps 1e-5 (src/slat_flow.cpp:244-248).
     PXS_TRY(pxs_layer_norm(PXS_F32, b.hidden, rows, C, 1e-5f, nullptr, nullptr, PXS_F32, b.normed,

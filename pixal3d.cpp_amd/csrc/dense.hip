@@ -68,6 +68,17 @@ struct DenseArgs {
     int splits;            // kDensePartial: K split over gridDim.y, sums to residual[split][m][n]
 };
 
+// Linears of one input with several weights: output g is at y + g m n.
+struct DenseGroup {
+    const void * w[kDenseGroup];
+    const float * bias[kDenseGroup];
+};
+template <typename T> __device__ __forceinline__ void select_group(DenseArgs & a, const DenseGroup & g) {
+    a.w = g.w[blockIdx.y];
+    a.bias = g.bias[blockIdx.y];
+    a.y = static_cast<T *>(a.y) + static_cast<int64_t>(blockIdx.y) * a.m * a.n;
+}
+
 // Output tile (row tile, column tile) of logical tile t: groups of g row
 // tiles share their column tiles, and inside a group consecutive t walk the
 // rows, so the tiles one XCD runs at a time cover g row tiles x (32 / g)
@@ -270,10 +281,11 @@ __device__ __forceinline__ void wait_stages(int later) {
 // NW waves in a WAVES_M x (NW / WAVES_M) grid, each owning a (BM / WAVES_M) x
 // (BN / WAVES_N) block of the tile; NSTAGE K chunks of KB bytes per row in
 // flight (one DMA instruction fills 1 KiB: 1024 / KB rows).
+// With a GROUP (DenseGroup) argument, blockIdx.y picks its weights, bias and output.
 template <typename T, int BM, int BN, int NW, int WAVES_M, int NSTAGE, int KB, int EPI, bool SPREAD,
-          bool STAGED>
+          bool STAGED, typename... GROUP>
 __global__ void __launch_bounds__(NW * 64)
-dense_gemm_kernel(DenseArgs a) {
+dense_gemm_kernel(DenseArgs a, GROUP... group) {
     constexpr int kVec = 16 / static_cast<int>(sizeof(T));  // elements per piece
     constexpr int P = KB / 16;                              // pieces per chunk row
     constexpr int kChunk = P * kVec;                        // elements per chunk row
@@ -290,6 +302,7 @@ dense_gemm_kernel(DenseArgs a) {
     constexpr int kPerStage = AI + BI;
 
     extern __shared__ __align__(16) char smem[];
+    if constexpr (sizeof...(GROUP) > 0) select_group<T>(a, group...);
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -658,15 +671,15 @@ int launch_dense_split(const DenseArgs & a, hipStream_t stream) {
 }
 
 template <typename T, int BM, int BN, int NW, int WAVES_M, int NSTAGE, int KB, int EPI,
-          bool SPREAD, bool STAGED>
-int launch_dense(const DenseArgs & a, hipStream_t stream) {
+          bool SPREAD, bool STAGED, typename... GROUP>
+int launch_dense(const DenseArgs & a, hipStream_t stream, int count = 1, const GROUP &... group) {
     constexpr int kStage = (BM + BN) * KB;
     constexpr int kChunk = KB / static_cast<int>(sizeof(T));
     constexpr int WN = BN / (NW / WAVES_M);
     constexpr int kStagedBytes = STAGED && EPI == kDenseStore ? NW * (BM / WAVES_M) * staged_pitch<T, WN>() : 0;
     constexpr int kMaxSmem = NSTAGE * kStage > kStagedBytes ? NSTAGE * kStage : kStagedBytes;
     static_assert(kMaxSmem <= 160 * 1024, "LDS");
-    auto kernel = &dense_gemm_kernel<T, BM, BN, NW, WAVES_M, NSTAGE, KB, EPI, SPREAD, STAGED>;
+    auto kernel = &dense_gemm_kernel<T, BM, BN, NW, WAVES_M, NSTAGE, KB, EPI, SPREAD, STAGED, GROUP...>;
     static bool configured = false;
     if (!configured) {
         const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
@@ -679,8 +692,8 @@ int launch_dense(const DenseArgs & a, hipStream_t stream) {
     if (a.vec_out == 2 && smem < kStagedBytes) smem = kStagedBytes;
     const int64_t blocks = ((a.m + BM - 1) / BM) * ((a.n + BN - 1) / BN);
     if (blocks > INT32_MAX) return fail(PXS_ERR_ARG, "dense GEMM grid too large");
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks), EPI == kDensePartial ? a.splits : 1),
-                       dim3(NW * 64), smem, stream, a);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks), EPI == kDensePartial ? a.splits : count),
+                       dim3(NW * 64), smem, stream, a, group...);
     return check_launch("dense GEMM");
 }
 
@@ -835,6 +848,25 @@ int dense_linear_gate(int dtype, const void * x, int64_t rows, int cin, const vo
                 aligned_to(time_mod, 16);
     *done = true;
     return run_dense<kDenseGate>(dtype, a, s);
+}
+
+// bf16 linears of one input with up to kDenseGroup weights [cout, cin] and
+// biases, in one launch: y [count, rows, cout].
+bool dense_group_takes(int cin, int cout) { return cin % 8 == 0 && cout % 8 == 0 && cout > 128; }
+
+int dense_linear_group(const void * x, int64_t rows, int cin, const void * const * w,
+                       const float * const * bias, int count, int cout, void * y, hipStream_t s) {
+    PXS_CHECK(count > 0 && count <= kDenseGroup, PXS_ERR_ARG, "dense linear group: bad count");
+    DenseGroup g{};
+    for (int i = 0; i < count; ++i) {
+        g.w[i] = w[i];
+        g.bias[i] = bias[i];
+    }
+    DenseArgs a{};
+    a.x = x; a.m = rows; a.k = cin; a.n = cout; a.y = y;
+    a.vec_out = 2;
+    a.group_m = 8;
+    return launch_dense<uint16_t, 256, 256, 16, 4, 2, 128, kDenseStore, true, true, DenseGroup>(a, s, count, g);
 }
 
 // Few rows leave most CUs without a 128 x 128 tile, and smaller tiles move

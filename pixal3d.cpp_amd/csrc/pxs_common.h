@@ -36,6 +36,14 @@ int dense_linear_gate(int dtype, const void * x, int64_t rows, int cin, const vo
                       const float * block_mod, const float * time_mod, int gate_offset,
                       float * residual, hipStream_t s, bool * done);
 
+// bf16 linears of one input with up to kDenseGroup weights [cout, cin] and fp32
+// biases, in one launch: y [count, rows, cout] (csrc/dense.hip).  x, y, weights and biases
+// 16-byte aligned, shapes as dense_group_takes.
+constexpr int kDenseGroup = 32;
+bool dense_group_takes(int cin, int cout);
+int dense_linear_group(const void * x, int64_t rows, int cin, const void * const * w,
+                       const float * const * bias, int count, int cout, void * y, hipStream_t s);
+
 // A residual linear of few rows split over K, and the layer norm that reads
 // its result (csrc/dense.hip, csrc/pointwise.hip).
 //   dense_splits: splits of K for this shape (rows of x and w 16-byte
