@@ -1690,8 +1690,8 @@ int launch_range_conv(const GemmArgs & args, hipStream_t stream) {
 
 // ---------------------------------------------------------------------------
 // fp32 split-K gather GEMM (SubMConv3d and linears in fp32).  A workgroup
-// owns 32 output rows x 64 output channels; its (offset, 32-channel chunk)
-// steps are dealt round-robin to its NW waves, so even a few hundred tiles
+// owns 32 output rows x 32 CT output channels; its (offset, 32-channel chunk)
+// steps are dealt round-robin to its 4 waves, so even a few hundred tiles
 // keep every CU busy.  Each wave loads its operands straight into VGPRs --
 // lane (h, r) takes the 64 contiguous bytes k = 16h .. 16h+15 of A row r and
 // of weight row r, the same K permutation on both sides of
@@ -1701,11 +1701,11 @@ int launch_range_conv(const GemmArgs & args, hipStream_t stream) {
 // deterministic).  The operand loads return through the per-CU vector-memory
 // path, which bounds the kernel.
 
-template <int EPI, int NW>
-__global__ void __launch_bounds__(NW * 64)
+template <int EPI, int CT>
+__global__ void __launch_bounds__(256)
 split_gemm_f32_kernel(GemmArgs a) {
-    constexpr int TI = 1, BM = 32 * TI, BN = 64;  // 32-row blocks per tile
-    __shared__ float red[NW - 1][TI * 2][16][64];
+    constexpr int NW = 4, TI = 1, BM = 32 * TI, BN = 32 * CT;
+    __shared__ float red[NW - 1][TI * CT][16][64];
     __shared__ int32_t idx_lds[32 * BM];
     __shared__ uint32_t tile_mask;
     __shared__ int koff[32];
@@ -1775,7 +1775,7 @@ split_gemm_f32_kernel(GemmArgs a) {
     // compiler's waits count exactly one step in flight.
     struct Ops {
         float4 av[TI][4];
-        float4 bv[2][4];
+        float4 bv[CT][4];
     };
     auto load = [&](int t, Ops & o) __attribute__((always_inline)) {
         const int s = wave + t * NW;
@@ -1795,7 +1795,7 @@ split_gemm_f32_kernel(GemmArgs a) {
             }
         }
 #pragma unroll
-        for (int ct = 0; ct < 2; ++ct) {
+        for (int ct = 0; ct < CT; ++ct) {
             const int c = n0 + ct * 32 + r;
             const bool ok = live && c < a.cout;
             const float * wrow = w + (static_cast<int64_t>(k) * a.cout + c) * a.cin;
@@ -1807,11 +1807,11 @@ split_gemm_f32_kernel(GemmArgs a) {
         }
     };
 
-    f32x16 acc[TI][2];
+    f32x16 acc[TI][CT];
 #pragma unroll
     for (int ti = 0; ti < TI; ++ti)
 #pragma unroll
-        for (int ct = 0; ct < 2; ++ct)
+        for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[ti][ct][v] = 0.0f;
     auto compute = [&](const Ops & o) __attribute__((always_inline)) {
@@ -1822,7 +1822,7 @@ split_gemm_f32_kernel(GemmArgs a) {
 #pragma unroll
                 for (int ti = 0; ti < TI; ++ti)
 #pragma unroll
-                    for (int ct = 0; ct < 2; ++ct)
+                    for (int ct = 0; ct < CT; ++ct)
                         acc[ti][ct] = __builtin_amdgcn_mfma_f32_32x32x2f32(
                             o.av[ti][q][e], o.bv[ct][q][e], acc[ti][ct], 0, 0, 0);
     };
@@ -1840,9 +1840,9 @@ split_gemm_f32_kernel(GemmArgs a) {
 #pragma unroll
         for (int ti = 0; ti < TI; ++ti)
 #pragma unroll
-            for (int ct = 0; ct < 2; ++ct)
+            for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) red[wave - 1][ti * 2 + ct][v][lane] = acc[ti][ct][v];
+                for (int v = 0; v < 16; ++v) red[wave - 1][ti * CT + ct][v][lane] = acc[ti][ct][v];
     }
     __syncthreads();
     if (wave != 0) return;
@@ -1851,10 +1851,10 @@ split_gemm_f32_kernel(GemmArgs a) {
 #pragma unroll
         for (int ti = 0; ti < TI; ++ti)
 #pragma unroll
-            for (int ct = 0; ct < 2; ++ct)
+            for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[ti][ct][v] += red[wv][ti * 2 + ct][v][lane];
-    gemm_epilogue<float, TI, 2, 32 * TI, 64, EPI>(a, acc, p0, n0, 0, 0, h, r);
+                for (int v = 0; v < 16; ++v) acc[ti][ct][v] += red[wv][ti * CT + ct][v][lane];
+    gemm_epilogue<float, TI, CT, 32 * TI, BN, EPI>(a, acc, p0, n0, 0, 0, h, r);
 }
 
 #ifndef PXS_SPLIT_F32
@@ -2019,14 +2019,14 @@ int launch_split_conv_f32(const GemmArgs & args, hipStream_t stream) {
     return check_launch("SubMConv3d (fp32 split)");
 }
 
-template <int EPI, int NW>
-int launch_split_f32_waves(const GemmArgs & args, hipStream_t stream) {
+template <int EPI, int CT>
+int launch_split_f32_cols(const GemmArgs & args, hipStream_t stream) {
     const int64_t tiles_m = (args.m + 31) / 32;
-    const int64_t tiles_n = (args.cout + 63) / 64;
+    const int64_t tiles_n = (args.cout + 32 * CT - 1) / (32 * CT);
     const int64_t blocks = tiles_m * tiles_n;
     if (blocks > INT32_MAX) return fail(PXS_ERR_ARG, "gather GEMM grid too large");
-    hipLaunchKernelGGL((split_gemm_f32_kernel<EPI, NW>), dim3(static_cast<unsigned>(blocks)),
-                       dim3(NW * 64), 0, stream, args);
+    hipLaunchKernelGGL((split_gemm_f32_kernel<EPI, CT>), dim3(static_cast<unsigned>(blocks)),
+                       dim3(256), 0, stream, args);
     return check_launch("gather GEMM (fp32 split-K)");
 }
 
@@ -2041,10 +2041,13 @@ int launch_split_f32(const GemmArgs & args, hipStream_t stream) {
     // long.  Errors against 64 bits are 0.45 to 0.65 of the fp32 tiles'.
     const int64_t squares = ((args.m + 63) / 64) * ((args.cout + 63) / 64);
     if (EPI == kEpiStore && gather && args.noff < 32 && squares >= 224) return launch_split_conv_f32(args, stream);
-    // At most one tile per CU: twice the waves halve each one's chain of steps.
-    const int64_t tiles = ((args.m + 31) / 32) * ((args.cout + 63) / 64);
-    if (gather && tiles <= 256) return launch_split_f32_waves<EPI, 8>(args, stream);
-    return launch_split_f32_waves<EPI, 4>(args, stream);
+    // Tiles of 32 columns where those still fit one per CU: a workgroup then
+    // takes in two thirds of the operand bytes (32 -> 48 at up to 2,900 rows 14.2
+    // against 20.8 us, 128 -> 128 at 1,592 rows 31 against 48; eight waves on the
+    // 64-column tile 24 and 56).
+    const int64_t narrow = ((args.m + 31) / 32) * ((args.cout + 31) / 32);
+    if (gather && narrow <= 256) return launch_split_f32_cols<EPI, 1>(args, stream);
+    return launch_split_f32_cols<EPI, 2>(args, stream);
 }
 
 template <typename T, int BM, int BN, int EPI, int NSTAGE, int NW, int WAVES_M, int KSPLIT>
