@@ -17,6 +17,7 @@
 
 #include "pxs_common.h"
 #include "scan.h"
+#include "split3.h"
 
 #include <cmath>
 #include <atomic>
@@ -1470,6 +1471,301 @@ flash_attn_f32_kernel(AttnArgs a, int heads, int64_t tiles_bound) {
         }
 }
 
+// fp32, head_dim and value_dim 64, unpermuted rows, on the bf16 matrix cores
+// (split3.h): 128 queries per workgroup, 4 waves of 32.  Q is split once, in
+// registers; each 64-key K and V tile, loaded into registers while the one
+// before is multiplied, is split by the workgroup's threads on its way into
+// three bf16 planes each in LDS, laid out and read as the bf16 kernel's tiles;
+// and a wave splits its own probabilities.  A workgroup whose operands or results leave the split's range
+// takes its queries again on v_mfma_f32_32x32x2_f32 (flash_f32_queries).
+// Bound by the vector instructions of the splits and the softmax: 4,560 x 4,560
+// x 16 heads in 613 us against 850 of flash_attn_f32_kernel and 1,106 of the
+// generic kernel, errors 1.07e-6 against 8.8e-7 (its two key groups are two
+// chains of sums) and 1.25e-6.
+constexpr int kSplitQueries = 128;  // queries per workgroup
+
+// One wave's 32 queries (lane r and its partner hold query r, dims 32h ..
+// 32h+31 in qv) against keys [k_begin, k_end), in fp32 from global memory.
+__device__ __forceinline__ void flash_f32_queries(const AttnArgs & a, const float * kp, const float * vp,
+                                                  const f32x4 (&qv)[8], int64_t k_begin, int64_t k_end, int h,
+                                                  int r, f32x16 (&oacc)[2], float & l_run) {
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) oacc[dt][v] = 0.0f;
+    float m_run = -INFINITY;
+    l_run = 0.0f;
+    for (int64_t key0 = k_begin; key0 < k_end; key0 += 32) {
+        const int64_t key = key0 + r < k_end ? key0 + r : k_end - 1;
+        f32x16 s = {};
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const f32x4 kf = *reinterpret_cast<const f32x4 *>(kp + key * a.ldk + 32 * h + 4 * u);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[e], qv[u][e], s, 0, 0, 0);
+        }
+        float mx = -INFINITY;
+        const int end = static_cast<int>(min<int64_t>(k_end - key0, 32)) - 4 * h;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            s[v] = 8 * (v >> 2) + (v & 3) < end ? s[v] * a.scale_log2 : -INFINITY;
+            mx = fmaxf(mx, s[v]);
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float m_new = fmaxf(m_run, mx);
+        const float alpha = m_new == -INFINITY ? 1.0f : exp2f(m_run - m_new);
+        float rs = 0.0f;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            s[v] = m_new == -INFINITY ? 0.0f : exp2f(s[v] - m_new);
+            rs += s[v];
+        }
+        rs += __shfl_xor(rs, 32, 64);
+        l_run = l_run * alpha + rs;
+        m_run = m_new;
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) oacc[dt][v] *= alpha;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int row = 8 * (v >> 2) + (v & 3);
+                const float vv = row < end ? vp[(key0 + 4 * h + row) * a.ldv + dt * 32 + r] : 0.0f;
+                oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, s[v], oacc[dt], 0, 0, 0);
+            }
+        }
+    }
+}
+
+template <bool SELF>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+flash_attn_f32_split_kernel(AttnArgs a, int heads, int64_t tiles_bound) {
+    constexpr int kPlane = kKeys * 128;  // a plane of a K or V tile: 64 rows of 64 bf16
+    __shared__ __align__(16) char k_lds[3 * kPlane], v_lds[3 * kPlane];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int h = lane >> 5, r = lane & 31;
+
+    const int64_t logical = remap_xcd64(blockIdx.x, tiles_bound * heads);
+    const int head = static_cast<int>(logical / tiles_bound);
+    const int64_t t = logical - static_cast<int64_t>(head) * tiles_bound;
+    int seg;
+    int64_t q_begin;
+    if constexpr (SELF) {
+        int64_t first;
+        if (!locate_tile(a, kSplitQueries, t, lane, seg, first)) return;
+        q_begin = a.cu_q[seg] + (t - first) * kSplitQueries;
+    } else {
+        if (t >= a.tile_start[a.nseg]) return;
+        seg = find_segment(a.tile_start, a.nseg, t, lane);
+        q_begin = a.cu_q[seg] + (t - a.tile_start[seg]) * kSplitQueries;
+    }
+    const int64_t q_end = a.cu_q[seg + 1];
+    const int64_t k_begin = a.cu_k[seg], k_end = a.cu_k[seg + 1];
+    const float * __restrict__ kp = static_cast<const float *>(a.k) + head * 64;
+    const float * __restrict__ vp = static_cast<const float *>(a.v) + head * 64;
+
+    // This lane's query, dims 32h .. 32h+31, in three planes: K step st holds
+    // dims 32h + 8 st .. + 7.
+    const int64_t qi = q_begin + wave * 32 + r;
+    const bool q_valid = qi < q_end;
+    const float * q = static_cast<const float *>(a.q) + (q_valid ? qi : q_begin) * a.ldq + head * 64 + 32 * h;
+    float hi = 0.0f;
+    bf16x8 qf[3][4];
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+        uint2 lo4[3], hi4[3];
+        split4(*reinterpret_cast<const float4 *>(q + 8 * st), lo4, hi);
+        split4(*reinterpret_cast<const float4 *>(q + 8 * st + 4), hi4, hi);
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+            qf[p][st] = __builtin_bit_cast(bf16x8, make_uint4(lo4[p].x, lo4[p].y, hi4[p].x, hi4[p].y));
+    }
+
+    // This thread's 16-byte pieces of a tile: dims 4 piece .. + 3 of keys row + 16 i.
+    const int piece = tid & 15, row = tid >> 4;
+    const int ntiles = static_cast<int>((k_end - k_begin + kKeys - 1) / kKeys);
+    float4 kr[4], vr[4];
+    auto load = [&](int j) __attribute__((always_inline)) {
+        const int64_t key0 = k_begin + static_cast<int64_t>(j) * kKeys + row;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int64_t key = key0 + 16 * i;
+            kr[i] = vr[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (key < k_end) {
+                kr[i] = *reinterpret_cast<const float4 *>(kp + key * a.ldk + piece * 4);
+                vr[i] = *reinterpret_cast<const float4 *>(vp + key * a.ldv + piece * 4);
+            }
+        }
+    };
+
+    // Lane-constant parts of the transposed V reads, as in the bf16 kernel.
+    const int G = lane >> 4, jl = lane & 15;
+    const int v_key_off = 4 * (G >> 1) + (jl >> 2);
+    const int v_dim_off = 16 * (G & 1) + 4 * (jl & 3);
+
+    f32x16 oacc[2];
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) oacc[dt][v] = 0.0f;
+    float m_run = -INFINITY, l_run = 0.0f;
+
+    if (ntiles > 0) load(0);
+    for (int j = 0; j < ntiles; ++j) {
+        barrier_no_fence();  // every wave has read the previous tile
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int rw = row + 16 * i;
+            uint2 w[3];
+            split4(kr[i], w, hi);
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+                *reinterpret_cast<uint2 *>(k_lds + p * kPlane + rw * 128 + (((piece >> 1) ^ kswz(rw)) << 4) +
+                                           (piece & 1) * 8) = w[p];
+            split4(vr[i], w, hi);
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+                *reinterpret_cast<uint2 *>(v_lds + p * kPlane + rw * 128 + (((piece >> 1) ^ vswz(rw)) << 4) +
+                                           (piece & 1) * 8) = w[p];
+        }
+        if (j + 1 < ntiles) load(j + 1);
+        barrier_no_fence();
+
+        // S^T for two 32-key sub-tiles.
+        f32x16 s[2] = {};
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+            bf16x8 kf[2][3];
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+                const int rw = kt * 32 + r;
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+                    kf[kt][p] = *reinterpret_cast<const bf16x8 *>(k_lds + p * kPlane + rw * 128 +
+                                                                  (((4 * h + st) ^ kswz(rw)) << 4));
+            }
+#pragma unroll
+            for (int n = 0; n < 6; ++n)
+#pragma unroll
+                for (int kt = 0; kt < 2; ++kt)
+                    s[kt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kt][kSplitTermA[n]], qf[kSplitTermB[n]][st],
+                                                                    s[kt], 0, 0, 0);
+        }
+
+        // Online softmax (log2 domain).  Register v of sub-tile kt holds key
+        // kt*32 + 8*(v/4) + 4h + v%4.
+        const int64_t left = k_end - (k_begin + static_cast<int64_t>(j) * kKeys);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) s[kt][v] *= a.scale_log2;
+        if (left < kKeys) {
+            const int end = static_cast<int>(left) - 4 * h;
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    if (kt * 32 + 8 * (v >> 2) + (v & 3) >= end) s[kt][v] = -INFINITY;
+        }
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) mx = fmaxf(mx, s[kt][v]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float m_new = fmaxf(m_run, mx);
+        if (__ballot(m_new != m_run)) {
+            const float alpha = m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+            l_run *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) oacc[dt][v] *= alpha;
+        }
+        m_run = m_new;
+        const float m_sub = m_new == -INFINITY ? 0.0f : m_new;  // scores -inf then give 0
+        float rs = 0.0f;
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                // (a probability below 2^-126 becomes 0)
+                s[kt][v] = __builtin_amdgcn_exp2f(s[kt][v] - m_sub);
+                rs += s[kt][v];
+            }
+        l_run += rs;  // this lane's keys; the partner's are added at the end
+
+        // O^T += V^T P^T, 16 keys at a time.
+#pragma unroll
+        for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                bf16x8 pf[3];
+                {
+                    uint2 lo4[3], hi4[3];
+                    float unused = 0.0f;
+                    split4(make_float4(s[kt][8 * u], s[kt][8 * u + 1], s[kt][8 * u + 2], s[kt][8 * u + 3]), lo4, unused);
+                    split4(make_float4(s[kt][8 * u + 4], s[kt][8 * u + 5], s[kt][8 * u + 6], s[kt][8 * u + 7]), hi4,
+                           unused);
+#pragma unroll
+                    for (int p = 0; p < 3; ++p)
+                        pf[p] = __builtin_bit_cast(bf16x8, make_uint4(lo4[p].x, lo4[p].y, hi4[p].x, hi4[p].y));
+                }
+                const int key_a = kt * 32 + 16 * u + v_key_off, key_b = key_a + 8;
+                bf16x8 vf[2][3];
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt) {
+                    const int dbyte = (dt * 32 + v_dim_off) * 2;
+                    const int vp16 = dbyte >> 4, within = dbyte & 15;
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) {
+                        const char * pa = v_lds + p * kPlane + key_a * 128 + ((vp16 ^ vswz(key_a)) << 4) + within;
+                        const char * pb = v_lds + p * kPlane + key_b * 128 + ((vp16 ^ vswz(key_b)) << 4) + within;
+                        const uint2 lo2 = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                                        (v4i16 __attribute__((address_space(3))) *)(pa)));
+                        const uint2 hi2 = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                                        (v4i16 __attribute__((address_space(3))) *)(pb)));
+                        vf[dt][p] = __builtin_bit_cast(bf16x8, make_uint4(lo2.x, lo2.y, hi2.x, hi2.y));
+                    }
+                }
+#pragma unroll
+                for (int n = 0; n < 6; ++n)
+#pragma unroll
+                    for (int dt = 0; dt < 2; ++dt)
+                        oacc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[dt][kSplitTermA[n]],
+                                                                           pf[kSplitTermB[n]], oacc[dt], 0, 0, 0);
+            }
+    }
+
+    l_run += __shfl_xor(l_run, 32, 64);
+    bool odd = hi > kSplitHigh || !(l_run < INFINITY);
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) odd |= split_sum_odd(oacc[dt][v]);
+    if (__syncthreads_or(odd)) {
+        f32x4 qv[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) qv[u] = *reinterpret_cast<const f32x4 *>(q + 4 * u);
+        flash_f32_queries(a, kp, vp, qv, k_begin, k_end, h, r, oacc, l_run);
+    }
+
+    if (!q_valid) return;
+    const float inv_l = l_run > 0.0f ? 1.0f / l_run : 0.0f;
+    float * op = static_cast<float *>(a.o) + qi * a.ldo + head * 64;
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int d = dt * 32 + 8 * i + 4 * h;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) op[d + e] = oacc[dt][4 * i + e] * inv_l;
+        }
+}
+
 // Segments in the order the short-segment kernel takes them: a counting sort
 // by item count (query passes x key chunks, the same for every head group),
 // costliest class first, empty segments last.  The order within a class is
@@ -1531,14 +1827,27 @@ int launch_attn_bf16(const AttnArgs & args, int64_t total_q, int heads, hipStrea
     return check_launch("flash attention (bf16)");
 }
 
+// fp32 attention that a grid of 64-query workgroups does not spread over more
+// than the CUs once: flash_attn_f32_kernel, whose workgroups are done sooner (300
+// x 1,370 x 16 heads 61 against 80 us, 256 x 256 x 4 16 against 20); otherwise the
+// split kernel (1,000 x 1,000 x 16, 288 workgroups, 61 against 85 us).
+bool f32_split_grid(int64_t total_q, int nseg, int heads) {
+    return (total_q / kF32Queries + nseg + 1) * heads > 256;
+}
+
+template <bool SPLIT>
 int launch_attn_f32(const AttnArgs & args, int64_t total_q, int heads, hipStream_t stream) {
-    const int64_t bound = total_q / kF32Queries + args.nseg + 1;
+    const int64_t bound = total_q / (SPLIT ? kSplitQueries : kF32Queries) + args.nseg + 1;
     if (bound * heads > INT32_MAX) return fail(PXS_ERR_ARG, "attention grid too large");
     const dim3 grid(static_cast<unsigned>(bound * heads)), block(256);
-    if (args.tile_start)
-        hipLaunchKernelGGL(flash_attn_f32_kernel<false>, grid, block, 0, stream, args, heads, bound);
-    else
-        hipLaunchKernelGGL(flash_attn_f32_kernel<true>, grid, block, 0, stream, args, heads, bound);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, stream, args, heads, bound); };
+    if constexpr (SPLIT) {
+        if (args.tile_start) launch(flash_attn_f32_split_kernel<false>);
+        else launch(flash_attn_f32_split_kernel<true>);
+    } else {
+        if (args.tile_start) launch(flash_attn_f32_kernel<false>);
+        else launch(flash_attn_f32_kernel<true>);
+    }
     return check_launch("flash attention (fp32)");
 }
 
@@ -1741,7 +2050,8 @@ int pxs_varlen_attention(int dtype, const void * q, int64_t ld_q, const void * k
     const bool vec_ok = (head_dim % vec == 0) && (value_dim % vec == 0) && (ld_q % vec == 0) &&
                         (ld_k % vec == 0) && (ld_v % vec == 0) && aligned16(q) && aligned16(k) && aligned16(v);
     const bool fast32 = dtype == PXS_F32 && nw == 4 && head_dim == 64 && value_dim == 64 && vec_ok && !row_map;
-    const int q_tile = fast32 ? kF32Queries : 32 * nw;
+    const bool split32 = fast32 && f32_split_grid(total_q, nseg, heads);
+    const int q_tile = split32 ? kSplitQueries : (fast32 ? kF32Queries : 32 * nw);
     int64_t * tile_start = nullptr;
     if (!self_tiles(total_q, nseg, q_tile, heads)) {
         tile_start = static_cast<int64_t *>(workspace);
@@ -1765,7 +2075,8 @@ int pxs_varlen_attention(int dtype, const void * q, int64_t ld_q, const void * k
         return nw == 4 ? launch_attn<uint16_t, 4>(a, total_q, heads, s)
                        : launch_attn<uint16_t, 1>(a, total_q, heads, s);
     }
-    if (fast32) return launch_attn_f32(a, total_q, heads, s);
+    if (split32) return launch_attn_f32<true>(a, total_q, heads, s);
+    if (fast32) return launch_attn_f32<false>(a, total_q, heads, s);
     return nw == 4 ? launch_attn<float, 4>(a, total_q, heads, s)
                    : launch_attn<float, 1>(a, total_q, heads, s);
 }

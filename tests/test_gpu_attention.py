@@ -6,6 +6,7 @@ from pathlib import Path
 
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 import workloads as W
@@ -62,16 +63,17 @@ def test_attention_fp32_random(px, orc, lens, heads, hd):
     assert_fp32(o, orc.varlen_attention(q, k, v, cu, cu, heads, hd, np.float32(scale)), what="attn")
 
 
-# fp32 segments of 256 queries and more on average, 64-wide heads: 64-query
-# workgroups whose two key groups take 32 keys each of every 64-key tile.  Key
-# counts at the edges of both (a group without keys, a ragged last tile, none at
-# all), query counts at the edges of the workgroup, scores up to +-40 that
-# come late.
+# fp32 segments of 256 queries and more on average, 64-wide heads.  Few heads: 64
+# query workgroups whose two key groups take 32 keys each of every 64-key tile;
+# many: 128-query workgroups with operands split into three bf16 terms.  Key
+# counts at the edges of a tile and of its halves, or none, query counts at the
+# edges of both workgroups, scores up to +-40 that come late.
+@pytest.mark.parametrize("heads", [3, 48])
 @pytest.mark.parametrize("q_lens,k_lens,gain", [
     ((256,), (1,), 1.0), ((257, 319, 320), (32, 33, 64), 1.0), ((300, 300), (0, 65), 1.0),
     ((511, 1, 640), (97, 1000, 31), 1.0), ((600,), (777,), 8.0)])
-def test_attention_fp32_tiled(px, orc, q_lens, k_lens, gain):
-    heads, hd = 3, 64
+def test_attention_fp32_tiled(px, orc, heads, q_lens, k_lens, gain):
+    hd = 64
     cu_q = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int64)
     cu_k = np.concatenate([[0], np.cumsum(k_lens)]).astype(np.int64)
     nq, nk, C = int(cu_q[-1]), int(cu_k[-1]), heads * hd
@@ -79,10 +81,47 @@ def test_attention_fp32_tiled(px, orc, q_lens, k_lens, gain):
     k = W.normal(67, nk * C, 2).reshape(nk, C)
     k[nk // 2:] *= gain
     v = W.normal(67, nk * C, 3).reshape(nk, C)
-    print(f"[attn fp32 tiled] q={q_lens} k={k_lens}", flush=True)
+    print(f"[attn fp32 tiled] heads={heads} q={q_lens} k={k_lens}", flush=True)
     o = host(px.varlen_attention(t32(q), t32(k), t32(v), ti64(cu_q), ti64(cu_k), heads, hd, 0.125))
     assert_fp32(o, orc.varlen_attention(q, k, v, cu_q, cu_k, heads, hd, np.float32(0.125)),
                 what="attn fp32 tiled")
+
+
+@pytest.mark.parametrize("what", ["inf_k", "nan_v", "huge_q", "tiny_v"])
+def test_attention_fp32_split_range(px, what):
+    """Values out of the split's range take a workgroup's queries again in fp32:
+    NaN where 64-bit attention has it (an infinite key gives infinite scores),
+    the other rows and heads as ever."""
+    dev, heads, hd, n = torch.device("cuda:0"), 32, 64, 520
+    g = torch.Generator(device=dev).manual_seed(70)
+    q, k, v = (torch.randn(n, heads * hd, generator=g, device=dev) for _ in range(3))
+    if what == "inf_k":
+        k[300, 5] = float("inf")
+    elif what == "nan_v":
+        v[77, 9] = float("nan")
+    elif what == "huge_q":
+        q[130, :hd] = 3e17 * q[130, :hd]
+    else:
+        v *= 1e-24
+    cu = torch.tensor([0, n], dtype=torch.int64, device=dev)
+    print(f"[attn fp32 range] {what}", flush=True)
+    o = px.varlen_attention(q, k, v, cu, cu, heads, hd, 0.125).double()
+    ref = torch.empty(n, heads * hd, dtype=torch.float64, device=dev)
+    for h in range(heads):
+        c = slice(h * hd, (h + 1) * hd)
+        ref[:, c] = torch.softmax(q[:, c].double() @ k[:, c].double().t().contiguous() * 0.125, 1) @ v[:, c].double()
+    if what == "inf_k":
+        # q of one sign gives the key all the weight (inf - inf: NaN), of the other none
+        assert torch.equal(torch.isnan(o[:, hd:]), torch.isnan(ref[:, hd:]))
+        bad = torch.isnan(ref).any(1)
+        assert bool(torch.isnan(o[bad, :hd]).all())
+        o, ref = o[~bad], ref[~bad]
+    else:
+        assert torch.equal(torch.isnan(o), torch.isnan(ref))
+    ok = torch.isfinite(ref)
+    # 1e-5 of the largest, as the fp32 tests; 3e17-fold scores pick one key whose
+    # value is passed on
+    assert float((o - ref).abs()[ok].max() / ref.abs()[ok].max()) <= 1e-5
 
 
 # Up to 64 segments the kernels find a tile's segment themselves, more take a
