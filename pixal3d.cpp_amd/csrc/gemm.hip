@@ -1690,21 +1690,22 @@ int launch_range_conv(const GemmArgs & args, hipStream_t stream) {
 
 // ---------------------------------------------------------------------------
 // fp32 split-K gather GEMM (SubMConv3d and linears in fp32).  A workgroup
-// owns 32 output rows x 32 CT output channels; its (offset, 32-channel chunk)
+// owns 32 TI output rows x 32 CT output channels; its (offset, 32-channel chunk)
 // steps are dealt round-robin to its 4 waves, so even a few hundred tiles
 // keep every CU busy.  Each wave loads its operands straight into VGPRs --
-// lane (h, r) takes the 64 contiguous bytes k = 16h .. 16h+15 of A row r and
-// of weight row r, the same K permutation on both sides of
+// lane (h, r) takes the 64 contiguous bytes k = 16h .. 16h+15 of A row r (of
+// each 32-row block) and of weight row r, the same K permutation on both sides of
 // v_mfma_f32_32x32x2_f32 -- with the next step's loads in flight during the
 // current step's MFMAs, and no barrier until the end, where waves 1 and up hand
 // their partial sums to wave 0 through LDS (a fixed summation order:
 // deterministic).  The operand loads return through the per-CU vector-memory
-// path, which bounds the kernel.
+// path, which bounds the kernel: TI = 2 reads each weight chunk once for 64
+// rows instead of 32.
 
-template <int EPI, int CT>
+template <int EPI, int TI, int CT>
 __global__ void __launch_bounds__(256)
 split_gemm_f32_kernel(GemmArgs a) {
-    constexpr int NW = 4, TI = 1, BM = 32 * TI, BN = 32 * CT;
+    constexpr int NW = 4, BM = 32 * TI, BN = 32 * CT;
     __shared__ float red[NW - 1][TI * CT][16][64];
     __shared__ int32_t idx_lds[32 * BM];
     __shared__ uint32_t tile_mask;
@@ -2019,13 +2020,13 @@ int launch_split_conv_f32(const GemmArgs & args, hipStream_t stream) {
     return check_launch("SubMConv3d (fp32 split)");
 }
 
-template <int EPI, int CT>
-int launch_split_f32_cols(const GemmArgs & args, hipStream_t stream) {
-    const int64_t tiles_m = (args.m + 31) / 32;
+template <int EPI, int TI, int CT>
+int launch_split_f32_tile(const GemmArgs & args, hipStream_t stream) {
+    const int64_t tiles_m = (args.m + 32 * TI - 1) / (32 * TI);
     const int64_t tiles_n = (args.cout + 32 * CT - 1) / (32 * CT);
     const int64_t blocks = tiles_m * tiles_n;
     if (blocks > INT32_MAX) return fail(PXS_ERR_ARG, "gather GEMM grid too large");
-    hipLaunchKernelGGL((split_gemm_f32_kernel<EPI, CT>), dim3(static_cast<unsigned>(blocks)),
+    hipLaunchKernelGGL((split_gemm_f32_kernel<EPI, TI, CT>), dim3(static_cast<unsigned>(blocks)),
                        dim3(256), 0, stream, args);
     return check_launch("gather GEMM (fp32 split-K)");
 }
@@ -2033,21 +2034,23 @@ int launch_split_f32_cols(const GemmArgs & args, hipStream_t stream) {
 template <int EPI>
 int launch_split_f32(const GemmArgs & args, hipStream_t stream) {
     const bool gather = (args.rowmap || args.grid) && args.noff >= 27;
-    // 64 x 64 tiles for nearly every CU: the split kernel.  Against this file's
-    // fp32 tiles (the whole call over a grid, us): 64 -> 64 at 22,032 rows (345
+    // More 64 x 64 tiles than CUs: the split kernel.  Against this file's fp32
+    // tiles (the whole call over a grid, us): 64 -> 64 at 22,032 rows (345
     // tiles) 83 against 103, 88,448 rows 227 against 277; 96 -> 192 at 8,912 rows
-    // (420) 118 against 138; 128 -> 128 at 8,912 rows (280) 153 against 166; 16 -> 36
-    // at 22,032 rows 46 against 69; at 140 tiles the same, below up to 1.7 times as
-    // long.  Errors against 64 bits are 0.45 to 0.65 of the fp32 tiles'.
+    // (420) 115 against 137; 128 -> 128 at 8,912 rows (280) 148 against 166; 16 -> 36
+    // at 22,032 rows 46 against 69.  Errors against 64 bits are 0.45 to 0.65 of the
+    // fp32 tiles'.  One round of 224 to 256 tiles is done sooner on 64-row fp32 tiles
+    // (64 -> 64 at 16,184 rows, 253 tiles: 57 against 66), fewer on 32-row ones.
     const int64_t squares = ((args.m + 63) / 64) * ((args.cout + 63) / 64);
-    if (EPI == kEpiStore && gather && args.noff < 32 && squares >= 224) return launch_split_conv_f32(args, stream);
+    if (EPI == kEpiStore && gather && args.noff < 32 && squares > 256) return launch_split_conv_f32(args, stream);
+    if (gather && squares >= 224) return launch_split_f32_tile<EPI, 2, 2>(args, stream);
     // Tiles of 32 columns where those still fit one per CU: a workgroup then
     // takes in two thirds of the operand bytes (32 -> 48 at up to 2,900 rows 14.2
     // against 20.8 us, 128 -> 128 at 1,592 rows 31 against 48; eight waves on the
     // 64-column tile 24 and 56).
     const int64_t narrow = ((args.m + 31) / 32) * ((args.cout + 31) / 32);
-    if (gather && narrow <= 256) return launch_split_f32_cols<EPI, 1>(args, stream);
-    return launch_split_f32_cols<EPI, 2>(args, stream);
+    if (gather && narrow <= 256) return launch_split_f32_tile<EPI, 1, 1>(args, stream);
+    return launch_split_f32_tile<EPI, 1, 2>(args, stream);
 }
 
 template <typename T, int BM, int BN, int EPI, int NSTAGE, int NW, int WAVES_M, int KSPLIT>
