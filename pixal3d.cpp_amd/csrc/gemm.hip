@@ -2392,9 +2392,69 @@ ordered_linear_rows_kernel(const float * __restrict__ x, int64_t rows, int cin,
     for (int o = 0; o < COUT; ++o) y[(row0 + t) * COUT + o] = acc[o];
 }
 
+// The same sums with one thread per (row, output), 8 lanes to a row, for 128 or
+// more inputs: with a thread per row few rows leave most SIMDs idle, each running
+// all outputs' chains one after the other, and the loads of a chunk wait for the
+// sums of the one before.  32 rows and the weights pass through LDS 128 inputs at
+// a time, the next chunk loaded into registers while one is summed; rows of LDS
+// are 132 floats apart, so the 8 rows (or outputs) a 16-byte read of a wave
+// covers lie on different banks.  8 outputs, us against the rows kernel: 500 x
+// 1024 15 / 115, 10,480 x 1024 18 / 200, 46,000 x 512 23 / 101, 174,000 x 256 34 /
+// 57, 662,000 x 128 73 / 101 (4.9 TB/s, about a copy's rate).
+constexpr int kLaneChunk = 128, kLanePitch = kLaneChunk + 4;
+__global__ void __launch_bounds__(256)
+ordered_linear_lanes_kernel(const float * __restrict__ x, int64_t rows, int cin,
+                            const float * __restrict__ weight, const float * __restrict__ bias, int cout,
+                            float * __restrict__ y) {
+#pragma clang fp contract(off)
+    __shared__ __align__(16) float x_lds[32 * kLanePitch], w_lds[8 * kLanePitch];
+    const int t = threadIdx.x;
+    const int64_t row0 = static_cast<int64_t>(blockIdx.x) * 32;
+    const int row = t >> 3, o = t & 7;
+    const int piece = (t & 31) * 4, line = t >> 5;  // this thread's 16-byte pieces: lines line + 8 q
+    float4 xv[4], wv;
+    auto load = [&](int k0) __attribute__((always_inline)) {
+        const bool in = k0 + piece < cin;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            xv[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (in && row0 + line + 8 * q < rows)
+                xv[q] = *reinterpret_cast<const float4 *>(x + (row0 + line + 8 * q) * cin + k0 + piece);
+        }
+        wv = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (in && line < cout) wv = *reinterpret_cast<const float4 *>(weight + static_cast<int64_t>(line) * cin + k0 + piece);
+    };
+    float value = bias && o < cout ? bias[o] : 0.0f;
+    load(0);
+    for (int k0 = 0; k0 < cin; k0 += kLaneChunk) {
+        __syncthreads();  // the previous chunk is consumed
+#pragma unroll
+        for (int q = 0; q < 4; ++q) *reinterpret_cast<float4 *>(x_lds + (line + 8 * q) * kLanePitch + piece) = xv[q];
+        *reinterpret_cast<float4 *>(w_lds + line * kLanePitch + piece) = wv;
+        if (k0 + kLaneChunk < cin) load(k0 + kLaneChunk);
+        __syncthreads();
+        const int kw = min(kLaneChunk, cin - k0);  // a multiple of 4
+#pragma unroll 8
+        for (int i = 0; i < kw; i += 4) {
+            const float4 a = *reinterpret_cast<const float4 *>(x_lds + row * kLanePitch + i);
+            const float4 b = *reinterpret_cast<const float4 *>(w_lds + o * kLanePitch + i);
+            value += b.x * a.x;
+            value += b.y * a.y;
+            value += b.z * a.z;
+            value += b.w * a.w;
+        }
+    }
+    if (o < cout && row0 + row < rows) y[(row0 + row) * cout + o] = value;
+}
+
 int launch_ordered_rows(const float * x, int64_t rows, int cin, const float * weight,
                         const float * bias, int cout, float * y, hipStream_t s) {
     const bool vec4 = cin % 4 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+    if (vec4 && aligned16(weight) && cin >= 128) {
+        hipLaunchKernelGGL(ordered_linear_lanes_kernel, dim3(static_cast<unsigned>((rows + 31) / 32)), dim3(256),
+                           0, s, x, rows, cin, weight, bias, cout, y);
+        return check_launch("ordered linear (lanes)");
+    }
     const dim3 grid(static_cast<unsigned>((rows + kOrderedRows - 1) / kOrderedRows));
     switch (cout) {
 #define PXS_ORDERED_ROWS(N)                                                                       \
@@ -2424,8 +2484,8 @@ int linear_rows(int dtype, const void * x, int64_t rows, int cin, const void * w
     if (rows == 0) return PXS_OK;
     PXS_CHECK(x && weight && y, PXS_ERR_ARG, "pxs_linear: null pointer");
     // A few fp32 outputs over narrow rows (the decoder's output layer, 64 -> 7
-    // over millions of rows): the reference's own operation order, one thread
-    // per row, HBM-bound, instead of MFMA tiles 7/8 empty.
+    // over millions of rows): the reference's own operation order,
+    // HBM-bound, instead of MFMA tiles 7/8 empty.
     if (dtype == PXS_F32 && act == PXS_ACT_NONE && cout <= kOrderedRowOut && cin <= 256)
         return launch_ordered_rows(static_cast<const float *>(x), rows, cin,
                                    static_cast<const float *>(weight), bias, cout,

@@ -238,6 +238,20 @@ def test_linear_ordered_bit_exact(px, orc, cin, cout, rows):
     np.testing.assert_array_equal(host(got), orc.linear(x, w, b))
 
 
+@pytest.mark.parametrize("cin", [128, 132, 260, 1024])
+@pytest.mark.parametrize("cout,rows", [(1, 1), (8, 31), (7, 33), (8, 500)])
+def test_linear_ordered_lanes_bit_exact(px, orc, cin, cout, rows):
+    """Few rows of 128 or more inputs take one thread per (row, output), 32
+    rows and 128 inputs at a time: whole and ragged last chunks (a single
+    4-input piece), one row, one row more or less than a workgroup, unused
+    output lanes, with and without a bias."""
+    x = W.normal(93, rows * cin, 1).reshape(rows, cin)
+    w = W.normal(93, cout * cin, 2, std=cin ** -0.5).reshape(cout, cin)
+    b = W.normal(93, cout, 3)
+    np.testing.assert_array_equal(host(px.linear_ordered(t32(x), t32(w), t32(b))), orc.linear(x, w, b))
+    np.testing.assert_array_equal(host(px.linear_ordered(t32(x), t32(w), None)), orc.linear(x, w, np.zeros_like(b)))
+
+
 @pytest.mark.parametrize("cin,cout", [(64, 7), (256, 8), (30, 2), (257, 8)])
 def test_linear_fp32_few_outputs(px, orc, cin, cout):
     """fp32 linears with at most 8 outputs and at most 256 inputs run in the
