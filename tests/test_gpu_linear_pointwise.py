@@ -163,6 +163,27 @@ def test_layer_norm_row_layouts(px, orc, channels, xd, yd):
         check(y, orc.layer_norm(xr, eps, gamma, beta), what=f"ln {channels} {xd}->{yd}")
 
 
+@pytest.mark.parametrize("rows", [1, 7, 1237])
+@pytest.mark.parametrize("xd,yd", [("f32", "f32"), ("bf16", "bf16"), ("f32", "bf16"), ("bf16", "f32")])
+def test_layer_norm_three_vectors_a_lane(px, orc, rows, xd, yd):
+    """Rows of 768 channels: 96 bf16 vectors on 32 lanes, 192 fp32 vectors on 64."""
+    import torch
+    x = (W.normal(58, rows * 768, 1) * 2 - 0.3).reshape(rows, 768)
+    g, b = W.normal(58, 768, 2), W.normal(58, 768, 3)
+    conv = t32 if xd == "f32" else tbf
+    xr = x if xd == "f32" else W.bf16_round(x)
+    out = torch.float32 if yd == "f32" else torch.bfloat16
+    check = assert_fp32 if yd == "f32" else assert_bf16
+    for gamma, beta, eps in ((g, b, 1e-6), (None, None, 1e-5)):
+        y = host(px.layer_norm(conv(x), eps, None if gamma is None else t32(gamma),
+                               None if beta is None else t32(beta), out_dtype=out))
+        check(y, orc.layer_norm(xr, eps, gamma, beta), what=f"ln 768 {xd}->{yd}")
+    coords = np.zeros((rows, 4), np.int32)
+    coords[rows // 2:, 0] = 1
+    bmod, tmod = W.normal(58, 6 * 768, 4, std=0.1), W.normal(58, 2 * 6 * 768, 5, std=0.1)
+    y = host(px.layer_norm_modulate(conv(x), 1e-6, ti32(coords), t32(bmod), t32(tmod), 3 * 768, out_dtype=out))
+    check(y, orc.modulate(coords, orc.layer_norm(xr, 1e-6), bmod, tmod, 3 * 768), what=f"ln mod 768 {xd}->{yd}")
+
 def test_layer_norm_small_channels_and_kat(px):
     import json
     from pathlib import Path
