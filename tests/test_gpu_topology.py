@@ -48,6 +48,19 @@ def test_neighbor_map_bit_exact(px, orc, case):
     assert px.validate(c, batch, shape) == (0, -1)
 
 
+@pytest.mark.parametrize("rows", [65_536, 65_537])
+def test_neighbor_map_hash_rows_limit(px, orc, rows):
+    """Up to 65,536 rows of unknown extents a lane looks up one neighbour, above
+    a thread several: the largest call of one kind and the smallest of the other."""
+    coords = np.ascontiguousarray(W.shell_coords(128, W.UNET_ITEMS, 2)[:rows])
+    assert coords.shape[0] == rows
+    nbr, masks = px.neighbor_map(ti32(coords))
+    ref = orc.neighbor_map(coords)
+    np.testing.assert_array_equal(nbr.cpu().numpy(), ref)
+    ref_masks = ((ref != rows).astype(np.int64) << np.arange(27)[:, None]).sum(0)
+    np.testing.assert_array_equal(masks.cpu().numpy().astype(np.int64) & 0x7FFFFFF, ref_masks)
+
+
 @pytest.mark.parametrize("case", list(coord_cases()) + ["edges"])
 def test_neighbor_map_grid_bit_exact(px, orc, case):
     """The dense-grid map equals the oracle's (and so the hash map's) bit for
