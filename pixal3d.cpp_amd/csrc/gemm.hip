@@ -2033,23 +2033,25 @@ int launch_split_f32_tile(const GemmArgs & args, hipStream_t stream) {
 
 template <int EPI>
 int launch_split_f32(const GemmArgs & args, hipStream_t stream) {
-    const bool gather = (args.rowmap || args.grid) && args.noff >= 27;
-    // More 64 x 64 tiles than CUs: the split kernel.  Against this file's fp32
-    // tiles (the whole call over a grid, us): 64 -> 64 at 22,032 rows (345
-    // tiles) 83 against 103, 88,448 rows 227 against 277; 96 -> 192 at 8,912 rows
-    // (420) 115 against 137; 128 -> 128 at 8,912 rows (280) 148 against 166; 16 -> 36
-    // at 22,032 rows 46 against 69.  Errors against 64 bits are 0.45 to 0.65 of the
-    // fp32 tiles'.  One round of 224 to 256 tiles is done sooner on 64-row fp32 tiles
-    // (64 -> 64 at 16,184 rows, 253 tiles: 57 against 66), fewer on 32-row ones.
-    const int64_t squares = ((args.m + 63) / 64) * ((args.cout + 63) / 64);
-    if (EPI == kEpiStore && gather && args.noff < 32 && squares > 256) return launch_split_conv_f32(args, stream);
-    if (gather && squares >= 224) return launch_split_f32_tile<EPI, 2, 2>(args, stream);
-    // Tiles of 32 columns where those still fit one per CU: a workgroup then
-    // takes in two thirds of the operand bytes (32 -> 48 at up to 2,900 rows 14.2
-    // against 20.8 us, 128 -> 128 at 1,592 rows 31 against 48; eight waves on the
-    // 64-column tile 24 and 56).
-    const int64_t narrow = ((args.m + 31) / 32) * ((args.cout + 31) / 32);
-    if (gather && narrow <= 256) return launch_split_f32_tile<EPI, 1, 1>(args, stream);
+    if constexpr (EPI == kEpiStore) {  // convolutions have no other epilogue
+        const bool gather = (args.rowmap || args.grid) && args.noff >= 27;
+        // More 64 x 64 tiles than CUs: the split kernel.  Against this file's fp32
+        // tiles (the whole call over a grid, us): 64 -> 64 at 22,032 rows (345
+        // tiles) 83 against 103, 88,448 rows 227 against 277; 96 -> 192 at 8,912 rows
+        // (420) 115 against 137; 128 -> 128 at 8,912 rows (280) 148 against 166; 16 -> 36
+        // at 22,032 rows 46 against 69.  Errors against 64 bits are 0.45 to 0.65 of the
+        // fp32 tiles'.  One round of 224 to 256 tiles is done sooner on 64-row fp32 tiles
+        // (64 -> 64 at 16,184 rows, 253 tiles: 57 against 66), fewer on 32-row ones.
+        const int64_t squares = ((args.m + 63) / 64) * ((args.cout + 63) / 64);
+        if (gather && args.noff < 32 && squares > 256) return launch_split_conv_f32(args, stream);
+        if (gather && squares >= 224) return launch_split_f32_tile<EPI, 2, 2>(args, stream);
+        // Tiles of 32 columns where those still fit one per CU: a workgroup then
+        // takes in two thirds of the operand bytes (32 -> 48 at up to 2,900 rows 14.2
+        // against 20.8 us, 128 -> 128 at 1,592 rows 31 against 48; eight waves on the
+        // 64-column tile 24 and 56).
+        const int64_t narrow = ((args.m + 31) / 32) * ((args.cout + 31) / 32);
+        if (gather && narrow <= 256) return launch_split_f32_tile<EPI, 1, 1>(args, stream);
+    }
     return launch_split_f32_tile<EPI, 1, 2>(args, stream);
 }
 
