@@ -174,9 +174,13 @@ SamplerBuffers carve_sampler(Carver & c, int dtype, const pxs_flow_config & f, i
     b.x0 = static_cast<float *>(c.take(static_cast<size_t>(rows) * f.out_channels * sizeof(float)));
     b.status = static_cast<int64_t *>(c.take(sizeof(int64_t)));
     b.guide_ws = c.take(pxs_flow_guidance_workspace_bytes(batch));
-    b.flow_ws = c.take(pxs_slat_flow_workspace_bytes(dtype, &f, 2 * rows,
-                                                     std::max<int64_t>(cond_tokens + uncond_tokens, 1),
-                                                     2 * batch));
+    // A guided step's forward takes twice the rows, an unguided one the rows
+    // alone with either context; a forward over fewer rows can need more.
+    const size_t both = pxs_slat_flow_workspace_bytes(dtype, &f, 2 * rows, cond_tokens + uncond_tokens,
+                                                      2 * batch);
+    const size_t cond = pxs_slat_flow_workspace_bytes(dtype, &f, rows, cond_tokens, batch);
+    const size_t uncond = pxs_slat_flow_workspace_bytes(dtype, &f, rows, uncond_tokens, batch);
+    b.flow_ws = c.take(std::max(both, std::max(cond, uncond)));
     return b;
 }
 

@@ -1,0 +1,49 @@
+"""Workspace sizes (host functions of libpxs.so, no GPU): each query covers
+every layout that the call it sizes can carve."""
+
+import ctypes as C
+
+import pytest
+
+import pxs
+
+LIB = pxs.load_library()
+
+
+def up(nbytes):
+    return (nbytes + 255) // 256 * 256  # each buffer is 256-byte aligned
+
+
+def flow_config(channels, heads, blocks, cond_channels, latent=32, mlp_ratio=4):
+    return pxs.FlowConfig(latent, latent, channels, cond_channels, blocks, heads, 0,
+                          mlp_ratio * channels, 1e-6, 1.0, 10000.0, 1, 1, 0)
+
+
+def flow_bytes(dtype, cfg, rows, tokens, batch):
+    return LIB.pxs_slat_flow_workspace_bytes(dtype, C.byref(cfg), rows, tokens, batch)
+
+
+def sampler_bytes(dtype, cfg, rows, cond, uncond, batch):
+    return LIB.pxs_flow_euler_sample_workspace_bytes(dtype, C.byref(cfg), rows, cond, uncond, batch)
+
+
+@pytest.mark.parametrize("dtype", [pxs.PXS_BF16, pxs.PXS_F32])
+@pytest.mark.parametrize("channels,heads,blocks", [(1024, 16, 24), (1536, 24, 30), (256, 4, 2)])
+@pytest.mark.parametrize("cond,uncond", [(1370, 1370), (5000, 1), (1, 9000), (2621, 2622)])
+def test_sampler_workspace_holds_every_step(dtype, channels, heads, blocks, cond, uncond):
+    """A guided step runs the forward over twice the rows, an unguided one over
+    the rows alone with either context, all in the workspace's last buffer."""
+    cfg = flow_config(channels, heads, blocks, 1024)
+    e = 2 if dtype == pxs.PXS_BF16 else 4
+    for batch in (1, 3):
+        for rows in (3, 700, 1344, 1345, 2688, 2689, 4095, 4096, 4097, 4600, 5000, 8192, 8193):
+            front = (up(2 * rows * 16) + 2 * up((2 * batch + 1) * 8) + up(2 * rows * 32 * 4) +
+                     up(2 * batch * 4) + up((cond + uncond) * 1024 * e) + up(2 * rows * 32 * 4) +
+                     2 * up(rows * 32 * 4) + up(8) +
+                     up(LIB.pxs_flow_guidance_workspace_bytes(batch)))
+            have = sampler_bytes(dtype, cfg, rows, cond, uncond, batch) - front
+            for r, tokens, b in ((2 * rows, cond + uncond, 2 * batch), (rows, cond, batch),
+                                 (rows, uncond, batch)):
+                need = flow_bytes(dtype, cfg, r, tokens, b)
+                assert need <= have, (f"rows {rows}, batch {batch}: a step over {r} rows and {tokens} "
+                                      f"tokens uses {need} of {have} bytes")
