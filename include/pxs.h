@@ -10,7 +10,9 @@
  *   - Calls are asynchronous on `stream` unless stated; none of them allocate
  *     device memory: scratch comes from a caller-provided workspace sized by
  *     the matching *_workspace_bytes query, 256-byte aligned (as hipMalloc
- *     returns; a misaligned one is an argument error).  (A pack's first
+ *     returns; a misaligned one is an argument error).  The sizes never fall
+ *     as a call's rows, context tokens or items grow, so one workspace of the
+ *     largest call's size serves every smaller call.  (A pack's first
  *     upload allocates its 32 MiB of pinned host staging, freed by
  *     pxs_pack_close.)
  *   - Coordinates are int32 rows (batch, x, y, z), read as 16-byte rows, so

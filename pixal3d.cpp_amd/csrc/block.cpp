@@ -38,6 +38,10 @@ int residual_splits(int dtype, int64_t rows, int cin, int channels) {
     return residual_norm_takes(channels) ? dense_splits(dtype, rows, cin, channels) : 0;
 }
 
+int64_t residual_split_rows(int dtype, int64_t rows, int cin, int channels) {
+    return residual_norm_takes(channels) ? dense_split_rows(dtype, rows, cin, channels) : 0;
+}
+
 BlockBuffers carve_block(Carver & c, int dtype, const pxs_block_config & cfg, int64_t rows,
                          int64_t tokens, int batch_size) {
     const size_t e = dtype_bytes(dtype);
@@ -55,11 +59,13 @@ BlockBuffers carve_block(Carver & c, int dtype, const pxs_block_config & cfg, in
     b.ckv = c.take(t * 2 * C * e);
     b.ck = c.take(t * C * e);
     b.attn_ws = c.take(pxs_attention_workspace_bytes(batch_size));
-    int splits = std::max(residual_splits(dtype, rows, cfg.channels, cfg.channels),
-                                residual_splits(dtype, rows, cfg.mlp_hidden, cfg.channels));
+    // Of the most partial sums that this many rows or fewer make, so that a
+    // workspace serves every smaller call.
+    int64_t partial = std::max(residual_split_rows(dtype, rows, cfg.channels, cfg.channels),
+                               residual_split_rows(dtype, rows, cfg.mlp_hidden, cfg.channels));
     if (cfg.use_projection)
-        splits = std::max(splits, residual_splits(dtype, rows, cfg.proj_in_channels, cfg.channels));
-    b.partial = static_cast<float *>(c.take(static_cast<size_t>(splits) * r * C * 4));
+        partial = std::max(partial, residual_split_rows(dtype, rows, cfg.proj_in_channels, cfg.channels));
+    b.partial = static_cast<float *>(c.take(static_cast<size_t>(partial) * C * 4));
     return b;
 }
 
@@ -225,10 +231,12 @@ struct FlowBuffers {
 // rows those launches are a small part, and the buffer is bounded.
 constexpr int64_t kContextAheadRows = 8192;
 constexpr int64_t kContextAheadBytes = int64_t{1} << 29;
+int64_t context_ahead_tokens(const pxs_flow_config & f) {
+    return kContextAheadBytes / (int64_t{4} * std::max(f.model_channels, 1) * std::max(f.num_blocks, 1));
+}
 bool context_ahead(int dtype, const pxs_flow_config & f, int64_t rows, int64_t tokens) {
     return dtype == PXS_BF16 && f.num_blocks > 1 && rows <= kContextAheadRows && tokens > 0 &&
-           dense_group_takes(f.cond_channels, 2 * f.model_channels) &&
-           tokens <= kContextAheadBytes / (int64_t{4} * f.model_channels * f.num_blocks);
+           dense_group_takes(f.cond_channels, 2 * f.model_channels) && tokens <= context_ahead_tokens(f);
 }
 
 constexpr int kTimestepFreqDim = 256;  // src/slat_flow.cpp:209
@@ -297,7 +305,12 @@ size_t pxs_slat_flow_workspace_bytes(int dtype, const pxs_flow_config * cfg, int
     if (!cfg) return 0;
     Carver c(nullptr);
     carve_flow(c, dtype, *cfg, rows, context_tokens, batch_size);
-    return c.used();
+    // Every buffer but context_kv grows with rows and tokens; this is the
+    // largest of the smaller calls that have one.
+    Carver ahead(nullptr);
+    carve_flow(ahead, dtype, *cfg, std::min(rows, kContextAheadRows),
+               std::min(context_tokens, context_ahead_tokens(*cfg)), batch_size);
+    return std::max(c.used(), ahead.used());
 }
 
 int pxs_slat_flow_forward(int dtype, const pxs_flow_config * cfg, const pxs_flow_weights * w,

@@ -879,14 +879,25 @@ int dense_linear_group(const void * x, int64_t rows, int cin, const void * const
 // 1,288 rows 1,632 against 1,500, 1,515, 1,508, 1,539; 2,600 rows (168 tiles) 2,118
 // against 2,037, 2,077, 2,202, 2,229; 4,064 rows (256 tiles) 2,503 against 2,522,
 // 2,698, 2,736, 2,863.
+constexpr int64_t kSplitTiles = 170;
 int dense_splits(int dtype, int64_t rows, int cin, int cout) {
     const int vec = dtype == PXS_BF16 ? 8 : 4, chunk = 8 * vec;
     if (rows <= 0 || cin % vec != 0 || cout % 4 != 0 || cout <= 64) return 0;
     const int64_t tiles = ((rows + 127) / 128) * ((cout + 127) / 128);
-    if (tiles > 170) return 0;
+    if (tiles > kSplitTiles) return 0;
     const int64_t most = std::min<int64_t>(4, cin / (4 * chunk));  // 4 stages of K each
     const int64_t splits = std::min(most, std::max<int64_t>(2, 256 / tiles));
     return splits >= 2 ? static_cast<int>(splits) : 0;
+}
+
+int64_t dense_split_rows(int dtype, int64_t rows, int cin, int cout) {
+    int64_t most = 0;
+    const int64_t row_tiles = std::min((rows + 127) / 128, kSplitTiles / ((cout + 127) / 128));
+    for (int64_t t = 1; t <= row_tiles; ++t) {  // the splits depend on the row tiles only
+        const int64_t r = std::min(rows, 128 * t);
+        most = std::max(most, dense_splits(dtype, r, cin, cout) * r);
+    }
+    return most;
 }
 
 int dense_partial(int dtype, const void * x, int64_t rows, int cin, const void * w, int cout,

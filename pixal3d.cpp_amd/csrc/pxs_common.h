@@ -48,6 +48,8 @@ int dense_linear_group(const void * x, int64_t rows, int cin, const void * const
 // its result (csrc/dense.hip, csrc/pointwise.hip).
 //   dense_splits: splits of K for this shape (rows of x and w 16-byte
 //     aligned), 0 when one pass is better.
+//   dense_split_rows: rows of partial sums (splits * rows) that a call of up to
+//     this many rows makes at most.
 //   dense_partial: partial[s] [rows, cout] fp32 = split s of x w^T.
 //   residual_norm: residual += (sum of the partials in order + bias) [* gate],
 //     then y = layer norm of the row with gamma and beta, or the adaLN modulate
@@ -67,6 +69,7 @@ struct ResidualNorm {
     void * y;
 };
 int dense_splits(int dtype, int64_t rows, int cin, int cout);
+int64_t dense_split_rows(int dtype, int64_t rows, int cin, int cout);
 int dense_partial(int dtype, const void * x, int64_t rows, int cin, const void * w, int cout,
                   int splits, float * partial, hipStream_t s);
 bool residual_norm_takes(int channels);

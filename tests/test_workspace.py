@@ -47,3 +47,44 @@ def test_sampler_workspace_holds_every_step(dtype, channels, heads, blocks, cond
                 need = flow_bytes(dtype, cfg, r, tokens, b)
                 assert need <= have, (f"rows {rows}, batch {batch}: a step over {r} rows and {tokens} "
                                       f"tokens uses {need} of {have} bytes")
+
+
+def never_shrinks(sizes, what):
+    worst = max(zip(sizes, sizes[1:]), key=lambda p: p[0] - p[1])
+    assert worst[0] <= worst[1], f"{what}: {worst[0]} bytes, then {worst[1]} for a larger call"
+
+
+ROWS = sorted({1, 7, 100, *(k + d for k in (128, 1344, 2688, 4096, 8192, 10752, 21760, 43520)
+                            for d in (-1, 0, 1))})
+
+
+@pytest.mark.parametrize("dtype", [pxs.PXS_BF16, pxs.PXS_F32])
+@pytest.mark.parametrize("channels,heads,blocks", [(1024, 16, 24), (1536, 24, 30), (256, 4, 2)])
+def test_flow_and_block_workspaces_serve_every_smaller_call(dtype, channels, heads, blocks):
+    """One workspace of the largest call's size serves calls of fewer rows,
+    context tokens and items: the sizes never fall as any of them grows."""
+    cfg = flow_config(channels, heads, blocks, 1024)
+    block = pxs.BlockConfig(channels, heads, 4 * channels, 1024, 512, 1e-6, 1.0, 10000.0, 1, 1, 1, 1)
+    cap = (1 << 29) // (4 * channels * blocks)  # tokens whose keys and values of all blocks are 512 MB
+    tokens = sorted({0, 1, 1370, cap - 1, cap, cap + 1, 2 * cap, 40000})
+    sizes = {
+        "flow": lambda r, t, b: flow_bytes(dtype, cfg, r, t, b),
+        "block": lambda r, t, b: LIB.pxs_transformer_block_workspace_bytes(dtype, C.byref(block), r, t, b),
+        "sampler": lambda r, t, b: sampler_bytes(dtype, cfg, r, t, t, b),
+    }
+    for name, size in sizes.items():
+        for b in (1, 2, 5):
+            for t in tokens:
+                never_shrinks([size(r, t, b) for r in ROWS], f"{name}, {t} tokens, growing rows")
+            for r in ROWS:
+                never_shrinks([size(r, t, b) for t in tokens], f"{name}, {r} rows, growing tokens")
+        never_shrinks([size(3000, 1370, b) for b in range(1, 70)], f"{name}, growing items")
+
+
+def test_decoder_workspaces_serve_every_smaller_call():
+    for dtype in (pxs.PXS_BF16, pxs.PXS_F32):
+        for ch in (64, 256, 1024):
+            never_shrinks([LIB.pxs_convnext_block_workspace_bytes(dtype, r, ch, 4 * ch, 1) for r in ROWS],
+                          "ConvNeXt block, growing rows")
+            never_shrinks([LIB.pxs_resblock_c2s_workspace_bytes(dtype, r, ch, ch // 2) for r in ROWS],
+                          "up-block, growing rows")
