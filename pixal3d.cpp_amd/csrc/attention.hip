@@ -1830,7 +1830,9 @@ int launch_attn_bf16(const AttnArgs & args, int64_t total_q, int heads, hipStrea
 // fp32 attention that a grid of 64-query workgroups does not spread over more
 // than the CUs once: flash_attn_f32_kernel, whose workgroups are done sooner (300
 // x 1,370 x 16 heads 61 against 80 us, 256 x 256 x 4 16 against 20); otherwise the
-// split kernel (1,000 x 1,000 x 16, 288 workgroups, 61 against 85 us).
+// split kernel (1,000 x 1,000 x 16, 288 workgroups, 61 against 85 us).  The grid is
+// one branch's (Branches): a guided step of 129 to 256 workgroups per branch takes up
+// to 1.2 times the other kernel's time, as each forward alone would with a lower line.
 bool f32_split_grid(int64_t total_q, int nseg, int heads) {
     return (total_q / kF32Queries + nseg + 1) * heads > 256;
 }
@@ -1970,23 +1972,12 @@ attn_wide_kernel(AttnArgs a, int64_t total_q, float scale) {
 }
 
 } // namespace
-} // namespace pxs
 
-using namespace pxs;
-
-extern "C" {
-
-size_t pxs_attention_workspace_bytes(int nseg) {
-    const int64_t n = std::max(nseg, 1);
-    return static_cast<size_t>(n + 1) * sizeof(int64_t) + static_cast<size_t>(n) * sizeof(int32_t) +
-           scan_workspace_bytes(n) + 64;
-}
-
-int pxs_varlen_attention(int dtype, const void * q, int64_t ld_q, const void * k, int64_t ld_k,
-                         const void * v, int64_t ld_v, const int64_t * cu_q,
-                         const int64_t * cu_k, int nseg, int64_t total_q,
-                         const int32_t * row_map, int heads, int head_dim, int value_dim,
-                         float scale, void * o, int64_t ld_o, void * workspace, void * stream) {
+int varlen_attention(int dtype, const void * q, int64_t ld_q, const void * k, int64_t ld_k,
+                     const void * v, int64_t ld_v, const int64_t * cu_q, const int64_t * cu_k,
+                     int nseg, int64_t total_q, const int32_t * row_map, int heads, int head_dim,
+                     int value_dim, float scale, void * o, int64_t ld_o, void * workspace,
+                     int branches, void * stream) {
     PXS_CHECK_WORKSPACE(workspace, "pxs_varlen_attention");
     PXS_CHECK(dtype == PXS_F32 || dtype == PXS_BF16, PXS_ERR_ARG, "pxs_varlen_attention: bad dtype");
     PXS_CHECK(heads > 0 && head_dim > 0 && head_dim <= kWideMaxDim && value_dim > 0 &&
@@ -2050,7 +2041,7 @@ int pxs_varlen_attention(int dtype, const void * q, int64_t ld_q, const void * k
     const bool vec_ok = (head_dim % vec == 0) && (value_dim % vec == 0) && (ld_q % vec == 0) &&
                         (ld_k % vec == 0) && (ld_v % vec == 0) && aligned16(q) && aligned16(k) && aligned16(v);
     const bool fast32 = dtype == PXS_F32 && nw == 4 && head_dim == 64 && value_dim == 64 && vec_ok && !row_map;
-    const bool split32 = fast32 && f32_split_grid(total_q, nseg, heads);
+    const bool split32 = fast32 && f32_split_grid(total_q / branches, nseg / branches, heads);
     const int q_tile = split32 ? kSplitQueries : (fast32 ? kF32Queries : 32 * nw);
     int64_t * tile_start = nullptr;
     if (!self_tiles(total_q, nseg, q_tile, heads)) {
@@ -2079,6 +2070,27 @@ int pxs_varlen_attention(int dtype, const void * q, int64_t ld_q, const void * k
     if (fast32) return launch_attn_f32<false>(a, total_q, heads, s);
     return nw == 4 ? launch_attn<float, 4>(a, total_q, heads, s)
                    : launch_attn<float, 1>(a, total_q, heads, s);
+}
+
+} // namespace pxs
+
+using namespace pxs;
+
+extern "C" {
+
+size_t pxs_attention_workspace_bytes(int nseg) {
+    const int64_t n = std::max(nseg, 1);
+    return static_cast<size_t>(n + 1) * sizeof(int64_t) + static_cast<size_t>(n) * sizeof(int32_t) +
+           scan_workspace_bytes(n) + 64;
+}
+
+int pxs_varlen_attention(int dtype, const void * q, int64_t ld_q, const void * k, int64_t ld_k,
+                         const void * v, int64_t ld_v, const int64_t * cu_q,
+                         const int64_t * cu_k, int nseg, int64_t total_q,
+                         const int32_t * row_map, int heads, int head_dim, int value_dim,
+                         float scale, void * o, int64_t ld_o, void * workspace, void * stream) {
+    return varlen_attention(dtype, q, ld_q, k, ld_k, v, ld_v, cu_q, cu_k, nseg, total_q, row_map,
+                            heads, head_dim, value_dim, scale, o, ld_o, workspace, 1, stream);
 }
 
 int pxs_varlen_attention_noalloc(int dtype, const void * q, int64_t ld_q, const void * k,

@@ -700,7 +700,7 @@ int launch_dense(const DenseArgs & a, hipStream_t stream, int count = 1, const G
 // fp32 linears of 1 to kFewRows rows (a flow's timestep embedding and its
 // modulation): one wave per output channel reads its weight row once, 16 bytes
 // per lane, and a tile of 64 rows would have run nearly empty: 1 x 1024 -> 6144
-// (25 MB of weights) 39 us on 64 x 64 tiles.
+// (25 MB of weights) 39 us on 64 x 64 tiles.  blockIdx.y: each kFewRows rows.
 constexpr int kFewRows = 4;
 __global__ void __launch_bounds__(256)
 few_rows_f32_kernel(DenseArgs a) {
@@ -708,14 +708,15 @@ few_rows_f32_kernel(DenseArgs a) {
     const int n = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (n >= a.n) return;
     const float * w = static_cast<const float *>(a.w) + static_cast<int64_t>(n) * a.k;
-    const float * x = static_cast<const float *>(a.x);
+    const int m0 = blockIdx.y * kFewRows, rows = min(static_cast<int>(a.m) - m0, kFewRows);
+    const float * x = static_cast<const float *>(a.x) + static_cast<int64_t>(m0) * a.k;
     float sum[kFewRows] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll 4
     for (int k = lane * 4; k < a.k; k += 256) {
         const float4 f = *reinterpret_cast<const float4 *>(w + k);
 #pragma unroll
         for (int m = 0; m < kFewRows; ++m) {
-            if (m >= a.m) break;
+            if (m >= rows) break;
             const float4 v = *reinterpret_cast<const float4 *>(x + static_cast<int64_t>(m) * a.k + k);
             sum[m] = fmaf(f.x, v.x, sum[m]);
             sum[m] = fmaf(f.y, v.y, sum[m]);
@@ -725,14 +726,14 @@ few_rows_f32_kernel(DenseArgs a) {
     }
 #pragma unroll
     for (int m = 0; m < kFewRows; ++m) {
-        if (m >= a.m) break;
+        if (m >= rows) break;
         float v = sum[m];
 #pragma unroll
         for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
         v += a.bias ? a.bias[n] : 0.0f;
         if (a.act == PXS_ACT_GELU_TANH) v = gelu_tanh_f(v);
         else if (a.act == PXS_ACT_SILU) v = silu_f(v);
-        if (lane == 0) static_cast<float *>(a.y)[static_cast<int64_t>(m) * a.n + n] = v;
+        if (lane == 0) static_cast<float *>(a.y)[static_cast<int64_t>(m0 + m) * a.n + n] = v;
     }
 }
 
@@ -805,7 +806,8 @@ int run_dense(int dtype, const DenseArgs & a, hipStream_t s) {
 } // namespace
 
 int dense_linear(int dtype, const void * x, int64_t rows, int cin, const void * w,
-                 const float * bias, int cout, int act, void * y, hipStream_t s, bool * done) {
+                 const float * bias, int cout, int act, void * y, int64_t plan_rows, hipStream_t s,
+                 bool * done) {
     *done = false;
     if (!dense_takes(dtype, x, cin, w)) return PXS_OK;
     DenseArgs a{};
@@ -815,8 +817,9 @@ int dense_linear(int dtype, const void * x, int64_t rows, int cin, const void * 
     // Whole 16-byte pieces of output rows: the store goes through LDS.
     if (a.vec_out && cout % (dtype == PXS_BF16 ? 8 : 4) == 0 && aligned_to(y, 16)) a.vec_out = 2;
     *done = true;
-    if (dtype == PXS_F32 && rows > 0 && rows <= kFewRows) {
-        hipLaunchKernelGGL(few_rows_f32_kernel, dim3(grid_for(cout, 4)), dim3(256), 0, s, a);
+    if (dtype == PXS_F32 && rows > 0 && plan_rows <= kFewRows) {
+        hipLaunchKernelGGL(few_rows_f32_kernel, dim3(grid_for(cout, 4), grid_for(rows, kFewRows)), dim3(256), 0,
+                           s, a);
         return check_launch("linear of few rows");
     }
     return run_dense<kDenseStore>(dtype, a, s);
@@ -873,20 +876,26 @@ int dense_linear_group(const void * x, int64_t rows, int cin, const void * const
 // more operand bytes per product through each CU (about 40 GB/s, the bound
 // here: 1,000 x 4096 -> 1024 in bf16 takes 38 us on 128 x 64 tiles and 28 us on
 // 64 x 64 tiles, with two stages in flight or six).  K is then split so that
-// the tiles come near to one per CU, two splits still paying at 170 tiles.
+// the tiles come near to one per CU.
 // Six blocks of width 1024 with their three residual linears in one pass
 // against 2, 3, 4, 5 splits: 248 rows 1,775 us against 1,628, 1,596, 1,586, 1,590;
 // 1,288 rows 1,632 against 1,500, 1,515, 1,508, 1,539; 2,600 rows (168 tiles) 2,118
 // against 2,037, 2,077, 2,202, 2,229; 4,064 rows (256 tiles) 2,503 against 2,522,
 // 2,698, 2,736, 2,863.
-constexpr int64_t kSplitTiles = 170;
+// A guided step runs the rows of a call twice with the splits of the call alone
+// (Branches), so up to four splits come with a quarter and more of the CUs idle
+// and none past 104 tiles, where twice as many still gain from two: at width
+// 1024, two forwards of 1,600 rows (104 tiles) in one 2,964 us against 3,060 in
+// one pass; of 2,600 rows 3,956 against 4,160 with two splits, though one forward
+// takes 1,258 against 1,210.
+constexpr int64_t kSplitTiles = 104;
 int dense_splits(int dtype, int64_t rows, int cin, int cout) {
     const int vec = dtype == PXS_BF16 ? 8 : 4, chunk = 8 * vec;
     if (rows <= 0 || cin % vec != 0 || cout % 4 != 0 || cout <= 64) return 0;
     const int64_t tiles = ((rows + 127) / 128) * ((cout + 127) / 128);
     if (tiles > kSplitTiles) return 0;
     const int64_t most = std::min<int64_t>(4, cin / (4 * chunk));  // 4 stages of K each
-    const int64_t splits = std::min(most, std::max<int64_t>(2, 256 / tiles));
+    const int64_t splits = std::min(most, std::max<int64_t>(2, 192 / tiles));
     return splits >= 2 ? static_cast<int>(splits) : 0;
 }
 

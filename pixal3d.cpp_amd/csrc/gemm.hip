@@ -2478,7 +2478,7 @@ int launch_ordered_rows(const float * x, int64_t rows, int cin, const float * we
 // whole 16-byte pieces, the gather-GEMM kernels (one offset, no row map)
 // otherwise.
 int linear_rows(int dtype, const void * x, int64_t rows, int cin, const void * weight,
-                const float * bias, int cout, int act, void * y, hipStream_t s) {
+                const float * bias, int cout, int act, void * y, int64_t plan_rows, hipStream_t s) {
     if (int rc = check_dtype(dtype, "pxs_linear")) return rc;
     PXS_CHECK(rows >= 0 && cin > 0 && cout > 0, PXS_ERR_ARG, "pxs_linear: bad shape");
     PXS_CHECK(act == PXS_ACT_NONE || act == PXS_ACT_GELU_TANH || act == PXS_ACT_SILU,
@@ -2493,7 +2493,8 @@ int linear_rows(int dtype, const void * x, int64_t rows, int cin, const void * w
                                    static_cast<const float *>(weight), bias, cout,
                                    static_cast<float *>(y), s);
     bool done = false;
-    if (int rc = dense_linear(dtype, x, rows, cin, weight, bias, cout, act, y, s, &done)) return rc;
+    if (int rc = dense_linear(dtype, x, rows, cin, weight, bias, cout, act, y, plan_rows, s, &done))
+        return rc;
     if (done) return PXS_OK;
     GemmArgs a{};
     a.x = x; a.rows_in = rows; a.ldx = cin; a.cin = cin; a.w = weight; a.bias = bias;
@@ -2736,7 +2737,7 @@ int pxs_sparse_conv3d_s2(int dtype, const void * x, int64_t n_in, int cin, const
 
 int pxs_linear(int dtype, const void * x, int64_t rows, int cin, const void * weight,
                const float * bias, int cout, int act, void * y, void * stream) {
-    return linear_rows(dtype, x, rows, cin, weight, bias, cout, act, y, as_stream(stream));
+    return linear_rows(dtype, x, rows, cin, weight, bias, cout, act, y, rows, as_stream(stream));
 }
 
 int pxs_linear_gate_residual(int dtype, const void * x, int64_t rows, int cin,

@@ -26,8 +26,11 @@ int check_launch(const char * what);
 //   dense_linear:          y (dtype) = act(x w^T + bias)
 //   dense_linear_residual: residual (fp32) += x w^T + bias
 //   dense_linear_gate:     residual += (x w^T + bias) * (block_mod[o + c] + time_mod[b, o + c])
+// (plan_rows: the rows that a kernel whose sums are taken in another order is
+// chosen by; see Branches.)
 int dense_linear(int dtype, const void * x, int64_t rows, int cin, const void * w,
-                 const float * bias, int cout, int act, void * y, hipStream_t s, bool * done);
+                 const float * bias, int cout, int act, void * y, int64_t plan_rows, hipStream_t s,
+                 bool * done);
 int dense_linear_residual(int dtype, const void * x, int64_t rows, int cin, const void * w,
                           const float * bias, int cout, float * residual, hipStream_t s,
                           bool * done);
@@ -35,6 +38,32 @@ int dense_linear_gate(int dtype, const void * x, int64_t rows, int cin, const vo
                       const float * bias, int cout, const int32_t * coords,
                       const float * block_mod, const float * time_mod, int gate_offset,
                       float * residual, hipStream_t s, bool * done);
+
+// Branches.  A guided sampler step runs two branches (twice the rows, items and
+// segments) in one forward, and its velocities equal those of two forwards bit
+// for bit.  Where a kernel that takes its sums in another order is chosen by the
+// size of a call, these internal forms choose it by the size of one branch; the
+// public calls have one.  Other kernels give a row the same bits in any call.
+//   linear_rows:          pxs_linear, chosen for plan_rows rows (kAnyRows: the
+//     kernel of many rows, for inputs whose rows are not split evenly).
+//   varlen_attention:     pxs_varlen_attention.
+//   slat_flow_forward and slat_flow_workspace_bytes: pxs_slat_flow_*.
+constexpr int64_t kAnyRows = INT64_MAX;
+int linear_rows(int dtype, const void * x, int64_t rows, int cin, const void * weight,
+                const float * bias, int cout, int act, void * y, int64_t plan_rows, hipStream_t s);
+int varlen_attention(int dtype, const void * q, int64_t ld_q, const void * k, int64_t ld_k,
+                     const void * v, int64_t ld_v, const int64_t * cu_q, const int64_t * cu_k,
+                     int nseg, int64_t total_q, const int32_t * row_map, int heads, int head_dim,
+                     int value_dim, float scale, void * o, int64_t ld_o, void * workspace,
+                     int branches, void * stream);
+int slat_flow_forward(int dtype, const pxs_flow_config * cfg, const pxs_flow_weights * w,
+                      const int32_t * coords, int64_t rows, int batch_size, const int64_t * cu_rows,
+                      const float * x, const float * timesteps, const void * context,
+                      const int64_t * context_offsets, int64_t context_tokens,
+                      const void * projected, float * out, void * workspace, int branches,
+                      void * stream);
+size_t slat_flow_workspace_bytes(int dtype, const pxs_flow_config * cfg, int64_t rows,
+                                 int64_t context_tokens, int batch_size, int branches);
 
 // bf16 linears of one input with up to kDenseGroup weights [cout, cin] and fp32
 // biases, in one launch: y [count, rows, cout] (csrc/dense.hip).  x, y, weights and biases

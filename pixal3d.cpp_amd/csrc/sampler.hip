@@ -176,8 +176,8 @@ SamplerBuffers carve_sampler(Carver & c, int dtype, const pxs_flow_config & f, i
     b.guide_ws = c.take(pxs_flow_guidance_workspace_bytes(batch));
     // A guided step's forward takes twice the rows, an unguided one the rows
     // alone with either context; a forward over fewer rows can need more.
-    const size_t both = pxs_slat_flow_workspace_bytes(dtype, &f, 2 * rows, cond_tokens + uncond_tokens,
-                                                      2 * batch);
+    const size_t both = slat_flow_workspace_bytes(dtype, &f, 2 * rows, cond_tokens + uncond_tokens,
+                                                  2 * batch, 2);
     const size_t cond = pxs_slat_flow_workspace_bytes(dtype, &f, rows, cond_tokens, batch);
     const size_t uncond = pxs_slat_flow_workspace_bytes(dtype, &f, rows, uncond_tokens, batch);
     b.flow_ws = c.take(std::max(both, std::max(cond, uncond)));
@@ -374,10 +374,10 @@ int pxs_flow_euler_sample(int dtype, const pxs_flow_config * cfg, const pxs_flow
                               "pxs_flow_euler_sample: state copy"));
             hipLaunchKernelGGL(fill_f32_kernel, dim3(grid_for(2 * batch_size, 64)), dim3(64), 0, s,
                                b.t2, 2 * batch_size, model_t);
-            PXS_TRY(pxs_slat_flow_forward(dtype, cfg, w, b.coords2, 2 * rows, 2 * batch_size, b.cu2,
-                                          b.x2, b.t2, b.ctx2, b.ctx_off2,
-                                          cond_tokens + uncond_tokens, nullptr, b.velocity,
-                                          b.flow_ws, stream));
+            PXS_TRY(slat_flow_forward(dtype, cfg, w, b.coords2, 2 * rows, 2 * batch_size, b.cu2,
+                                      b.x2, b.t2, b.ctx2, b.ctx_off2,
+                                      cond_tokens + uncond_tokens, nullptr, b.velocity,
+                                      b.flow_ws, 2, stream));
             PXS_TRY(pxs_check_finite(PXS_F32, b.velocity, 2 * rows, C, C, b.status, stream));
             if (scfg->guidance_rescale > 0.0f) {
                 // x0 of the conditional prediction, then of the plain CFG blend.

@@ -132,6 +132,72 @@ def test_device_sampler_batched_cfg_equals_separate_forwards(px):
     torch.cuda.synchronize()
     np.testing.assert_array_equal(host(got), host(state))
 
+# Rows per item, and context tokens of the two branches; each crosses a line at
+# which a kernel that sums in another order is taken: the K splits of residual
+# linears (bf16 width 256 and 1024, fp32), one pass instead (10,000 rows), the
+# fp32 attention of more workgroups than CUs (2,100 rows x 4 heads), the fp32
+# linears of up to 4 rows (3 items; 3 rows, 3 and 2 tokens), and the context
+# keys and values of all blocks ahead (4,600 rows).
+BRANCH_CASES = {
+    "bf16_1024_700": (torch.bfloat16, 1024, 1, [700], 50, 3),
+    "bf16_256_5000": (torch.bfloat16, 256, 2, [5000], 7, 130),
+    "bf16_256_6000": (torch.bfloat16, 256, 2, [6000], 40, 40),
+    "bf16_512_4600": (torch.bfloat16, 512, 2, [2300, 2300], 60, 9),
+    "bf16_256_33blocks": (torch.bfloat16, 256, 33, [140], 9, 12),
+    "f32_256_2100": (torch.float32, 256, 1, [2100], 20, 33),
+    "f32_256_700x3": (torch.float32, 256, 1, [700, 650, 750], 5, 6),
+    "f32_256_3": (torch.float32, 256, 1, [3], 3, 2),
+}
+
+
+@pytest.mark.parametrize("name", list(BRANCH_CASES))
+def test_device_sampler_equals_separate_forwards_at_size(px, name):
+    """The sampler's guided and unguided steps against separate forwards of its
+    two branches, bit for bit, where the doubled batch is larger than a line
+    that a branch is not."""
+    dtype, ch, nb, items, cond_tokens, unc_tokens = BRANCH_CASES[name]
+    print(f"[device sampler] {name}", flush=True)
+    lat, batch, rows = 16, len(items), sum(items)
+    idx = np.concatenate([np.arange(n) for n in items])
+    coords = ti32(np.stack([np.repeat(np.arange(batch), items), idx // 1024, idx // 32 % 32, idx % 32], 1))
+    cu = px.batch_cu_seqlens(coords, batch)
+    gen = torch.Generator(device="cuda").manual_seed(17)
+    rand = lambda *s, std=1.0: torch.randn(*s, device="cuda", generator=gen) * std  # noqa: E731
+    cfg = pxs.FlowConfig(lat, lat, ch, ch, nb, ch // 64, 0, 4 * ch, 1e-6, 1.0, 10000.0, 1, 1, 0)
+    fw = [rand(ch, lat, std=0.2), rand(ch), rand(ch, 256, std=0.02), rand(ch), rand(ch, ch, std=0.02),
+          rand(ch), rand(6 * ch, ch, std=0.02), rand(6 * ch, std=0.1), rand(lat, ch, std=0.03), rand(lat)]
+    sizes = [6 * ch, 3 * ch * ch, 3 * ch, ch, ch, ch * ch, ch, ch, ch, ch * ch, ch, 2 * ch * ch, 2 * ch,
+             ch, ch, ch * ch, ch, 0, 0, 4 * ch * ch, 4 * ch, 4 * ch * ch, ch]
+    blocks = []
+    for _ in range(nb):
+        ws = [rand(n, std=0.03) if n else None for n in sizes]
+        for i in (3, 4, 7, 13, 14):
+            ws[i] = ws[i] + 1.0
+        blocks.append([w.to(dtype) if w is not None and i in pxs.BLOCK_LINEAR_WEIGHTS else w
+                       for i, w in enumerate(ws)])
+    arr = (pxs.BlockWeights * nb)(*[pxs.block_weights(b) for b in blocks])
+    weights = pxs.FlowWeights(*[a.data_ptr() for a in fw], arr)
+    ctx, unc = rand(batch * cond_tokens, ch).to(dtype), rand(batch * unc_tokens, ch).to(dtype)
+    ctx_off = ti64(np.arange(batch + 1) * cond_tokens)
+    unc_off = ti64(np.arange(batch + 1) * unc_tokens)
+    noise = rand(rows, lat)
+    scfg = pxs.SamplerConfig(3, 1e-5, 1.0, 5.0, 0.0, 0.5, 1.0)  # the last step is unguided
+    got = px.flow_euler_sample(cfg, weights, scfg, coords, batch, cu, noise, ctx, ctx_off, unc, unc_off)
+    state, guided = noise.clone(), []
+    for step in range(3):
+        t, tn, g = px.flow_sampler_schedule(scfg, step)
+        guided.append(g != 1.0)
+        tt = torch.full((batch,), float(np.float32(1000.0) * np.float32(t)), device="cuda")
+        pred = px.slat_flow_forward(cfg, weights, coords, batch, cu, state, tt, ctx, ctx_off)
+        if guided[-1]:
+            neg = px.slat_flow_forward(cfg, weights, coords, batch, cu, state, tt, unc, unc_off)
+            pred = px.flow_guidance(state, pred, neg, coords, cu, batch, t, 1e-5, g, 0.0)
+        px.flow_euler_update(state, pred, float(np.float32(t) - np.float32(tn)))
+    torch.cuda.synchronize()
+    assert guided == [True, True, False]
+    assert torch.isfinite(state).all()
+    assert torch.equal(got, state), f"{name}: max difference {(got - state).abs().max().item():.3e}"
+
 
 def test_device_sampler_matches_oracle(px, orc):
     """pxs_flow_euler_sample against orc_flow_euler_sample whose velocity is
