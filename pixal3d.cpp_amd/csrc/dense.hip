@@ -884,10 +884,10 @@ int dense_linear_group(const void * x, int64_t rows, int cin, const void * const
 // 2,698, 2,736, 2,863.
 // A guided step runs the rows of a call twice with the splits of the call alone
 // (Branches), so up to four splits come with a quarter and more of the CUs idle
-// and none past 104 tiles, where twice as many still gain from two: at width
-// 1024, two forwards of 1,600 rows (104 tiles) in one 2,964 us against 3,060 in
-// one pass; of 2,600 rows 3,956 against 4,160 with two splits, though one forward
-// takes 1,258 against 1,210.
+// and none past 104 tiles, where twice as many still gain from two.  Two guided
+// steps of four blocks of width 1024 with two splits against one pass: 1,600 rows
+// (104 tiles) 2,872 us against 2,964; 2,600 rows (168) 4,160 against 3,956, though
+// one forward alone takes 1,258 against 1,302.
 constexpr int64_t kSplitTiles = 104;
 int dense_splits(int dtype, int64_t rows, int cin, int cout) {
     const int vec = dtype == PXS_BF16 ? 8 : 4, chunk = 8 * vec;
