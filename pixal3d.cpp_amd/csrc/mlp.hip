@@ -264,9 +264,16 @@ int convnext_mlp(const void * y, int64_t rows, int channels, float eps, const fl
                     static_cast<const uint16_t *>(w0), b0, static_cast<const uint16_t *>(w2), b2, hidden,
                     x_in, x_out};
     *done = true;
-    if (channels == 64) return launch_mlp<64>(a, s);
-    if (channels == 128) return launch_mlp<128>(a, s);
-    if (channels == 256) return launch_mlp<256>(a, s);
+    // A workgroup walks the whole hidden width for its 256 rows, so a call of few
+    // rows takes as long as one that fills the CUs, and the separate launches, which
+    // split the columns too, are done sooner.  The whole block, us, in one kernel
+    // against the separate launches, M = 4 C: 64 channels at 300 rows 38 / 45 (M =
+    // 1024 54 / 52); 128 at 1,000 rows 78 / 71, 4,096 78 / 75, 8,000 81 / 84, 20,000 85 /
+    // 101; 256 at 1,000 rows 232 / 153, 20,000 248 / 203, 32,768 (half the CUs) 265 /
+    // 250, 35,000 373 / 380, 50,000 397 / 436.
+    if (channels == 64 && (hidden <= 512 || rows >= 4096)) return launch_mlp<64>(a, s);
+    if (channels == 128 && rows >= 8192) return launch_mlp<128>(a, s);
+    if (channels == 256 && rows > 32768) return launch_mlp<256>(a, s);
     *done = false;
     return PXS_OK;
 }

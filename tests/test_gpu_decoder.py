@@ -112,6 +112,39 @@ def test_convnext_block_bf16_mlp(px, C, M, rows):
     assert_bf16(host(y - x), host(ref), tol=2.0 ** -8, what="convnext mlp")
 
 
+# Both sides of the row counts from which the one-kernel MLP is taken, one of
+# them ragged over its 256-row workgroups.
+@pytest.mark.parametrize("C,M,rows", [(128, 512, 300), (128, 512, 8191), (128, 512, 8192),
+                                      (256, 1024, 500), (256, 1024, 32768), (256, 1024, 32769),
+                                      (256, 192, 33001)])
+def test_convnext_block_bf16_mlp_of_few_rows(px, C, M, rows):
+    """Below the line the block is its single ops, bit for bit; from it on,
+    within the one-kernel MLP's rounding of the norm and the hidden tensor."""
+    dev = torch.device("cuda:0")
+    i = torch.arange(rows, device=dev)
+    coords = torch.stack([0 * i, i // 400, i // 2 % 200, i % 2], 1).to(torch.int32)
+    g = torch.Generator(device=dev).manual_seed(rows + C)
+    rnd = lambda *s, std=1.0: torch.randn(*s, generator=g, device=dev) * std  # noqa: E731
+    bf = torch.bfloat16
+    w = {"norm_weight": 1.0 + rnd(C, std=0.1), "norm_bias": rnd(C, std=0.1),
+         "conv1_weight": rnd(27, C, C, std=(27 * C) ** -0.5).to(bf), "conv1_bias": rnd(C, std=0.1),
+         "mlp0_weight": rnd(M, C, std=C ** -0.5).to(bf), "mlp0_bias": rnd(M, std=0.1),
+         "mlp2_weight": rnd(C, M, std=M ** -0.5).to(bf), "mlp2_bias": rnd(C, std=0.1)}
+    x = rnd(rows, C)
+    print(f"convnext mlp rows={rows} C={C} M={M}", flush=True)
+    nbr, masks = px.neighbor_map(coords)
+    y = px.convnext_block(coords, x, M, 1e-6, pxs.decoder_block_weights(w), pxs.PXS_BF16, nbr, masks)
+    c = px.subm_conv3d(x.to(bf), w["conv1_weight"], w["conv1_bias"], nbr, masks)
+    n = px.layer_norm(c, 1e-6, w["norm_weight"], w["norm_bias"])
+    ref = x.clone()
+    px.linear_residual(px.linear(n, w["mlp0_weight"], w["mlp0_bias"], act=2), w["mlp2_weight"],
+                       w["mlp2_bias"], ref)
+    if rows < {128: 8192, 256: 32769}[C]:
+        assert torch.equal(y, ref)
+    else:
+        assert_bf16(host(y - x), host(ref - x), tol=2.0 ** -8, what="convnext mlp")
+
+
 def test_convnext_block_in_place_with_given_map(px, orc):
     """y aliasing x and a caller-built neighbor map give the same result."""
     C, M = 32, 128
