@@ -1476,8 +1476,9 @@ flash_attn_f32_kernel(AttnArgs a, int heads, int64_t tiles_bound) {
 // registers; each 64-key K and V tile, loaded into registers while the one
 // before is multiplied, is split by the workgroup's threads on its way into
 // three bf16 planes each in LDS, laid out and read as the bf16 kernel's tiles;
-// and a wave splits its own probabilities.  A workgroup whose operands or results leave the split's range
-// takes its queries again on v_mfma_f32_32x32x2_f32 (flash_f32_queries).
+// and a wave splits its own probabilities.  A workgroup whose operands or results
+// leave the split's range takes its queries again on v_mfma_f32_32x32x2_f32
+// (flash_f32_queries).
 // Bound by the vector instructions of the splits and the softmax: 4,560 x 4,560
 // x 16 heads in 613 us against 850 of flash_attn_f32_kernel and 1,106 of the
 // generic kernel, errors 1.07e-6 against 8.8e-7 (its two key groups are two
@@ -1740,17 +1741,39 @@ flash_attn_f32_split_kernel(AttnArgs a, int heads, int64_t tiles_bound) {
             }
     }
 
+    // The rules of split3.h for the sums over the keys, whose probabilities are at
+    // most 1; the scores' own losses are below 2^-36 (f32_split_scale).
     l_run += __shfl_xor(l_run, 32, 64);
+    const int keys = static_cast<int>(min<int64_t>(k_end - k_begin, INT32_MAX));
     bool odd = hi > kSplitHigh || !(l_run < INFINITY);
+    const float low = split_low(kSplitHigh, keys);
 #pragma unroll
     for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) odd |= split_sum_odd(oacc[dt][v]);
-    if (__syncthreads_or(odd)) {
-        f32x4 qv[8];
+        for (int v = 0; v < 16; ++v) odd |= split_sum_odd(oacc[dt][v], low);
+    if (__builtin_expect(__syncthreads_or(odd), 0)) {
+        hi = split_block_max(hi, reinterpret_cast<uint32_t *>(k_lds));
+        const float tile_low = split_low(hi, keys);
+        bool again = hi > kSplitHigh || !(l_run < INFINITY), zero = false;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) qv[u] = *reinterpret_cast<const f32x4 *>(q + 4 * u);
-        flash_f32_queries(a, kp, vp, qv, k_begin, k_end, h, r, oacc, l_run);
+        for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                zero |= oacc[dt][v] == 0.0f;
+                again |= oacc[dt][v] != 0.0f && split_sum_odd(oacc[dt][v], tile_low);
+            }
+        if (__syncthreads_or(zero))
+            for (int j = 0; j < ntiles; ++j) {
+                load(j);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) again |= split_small(vr[i]);
+            }
+        if (__syncthreads_or(again)) {
+            f32x4 qv[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) qv[u] = *reinterpret_cast<const f32x4 *>(q + 4 * u);
+            flash_f32_queries(a, kp, vp, qv, k_begin, k_end, h, r, oacc, l_run);
+        }
     }
 
     if (!q_valid) return;
@@ -1836,6 +1859,9 @@ int launch_attn_bf16(const AttnArgs & args, int64_t total_q, int heads, hipStrea
 bool f32_split_grid(int64_t total_q, int nseg, int heads) {
     return (total_q / kF32Queries + nseg + 1) * heads > 256;
 }
+// The split may move a score before its scale by 128 x 2^50 x 2^-134: scales up to
+// 2^41 keep that below 2^-36, far under a score's rounding.
+bool f32_split_scale(float scale) { return scale <= 0x1p41f; }
 
 template <bool SPLIT>
 int launch_attn_f32(const AttnArgs & args, int64_t total_q, int heads, hipStream_t stream) {
@@ -2041,7 +2067,8 @@ int varlen_attention(int dtype, const void * q, int64_t ld_q, const void * k, in
     const bool vec_ok = (head_dim % vec == 0) && (value_dim % vec == 0) && (ld_q % vec == 0) &&
                         (ld_k % vec == 0) && (ld_v % vec == 0) && aligned16(q) && aligned16(k) && aligned16(v);
     const bool fast32 = dtype == PXS_F32 && nw == 4 && head_dim == 64 && value_dim == 64 && vec_ok && !row_map;
-    const bool split32 = fast32 && f32_split_grid(total_q / branches, nseg / branches, heads);
+    const bool split32 = fast32 && f32_split_grid(total_q / branches, nseg / branches, heads) &&
+                         f32_split_scale(scale);
     const int q_tile = split32 ? kSplitQueries : (fast32 ? kF32Queries : 32 * nw);
     int64_t * tile_start = nullptr;
     if (!self_tiles(total_q, nseg, q_tile, heads)) {

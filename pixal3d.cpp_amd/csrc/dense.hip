@@ -595,41 +595,133 @@ dense_split_kernel(DenseArgs a) {
             }
         }
     }
+    // A split's share of K has the whole K's bound: the rule then is one of rows and
+    // channels, whatever the split.
     bool odd = hi > kSplitHigh;
+    const float low = split_low(kSplitHigh, a.k);
+    float sum[TI][TJ][16];
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
         for (int j = 0; j < TJ; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) odd |= split_sum_odd(acc[i][j][v]);
-    if (__syncthreads_or(odd)) {
-        // rare: the whole tile again in fp32
+            for (int v = 0; v < 16; ++v) {
+                sum[i][j][v] = acc[i][j][v];
+                asm("" : "+v"(sum[i][j][v]));  // scalars from here on: vectors would be copied whole, and spill
+                odd |= split_sum_odd(sum[i][j][v], low);
+            }
+    if (__builtin_expect(__syncthreads_or(odd), 0)) {
+        hi = split_block_max(hi, reinterpret_cast<uint32_t *>(smem));
+        const float tile_low = split_low(hi, a.k);
+        bool again = hi > kSplitHigh, zero = false;
 #pragma unroll
         for (int i = 0; i < TI; ++i)
 #pragma unroll
             for (int j = 0; j < TJ; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-        const float * xr[TI];
-        const float * wr[TJ];
-#pragma unroll
-        for (int i = 0; i < TI; ++i) {
-            const int64_t m = p0 + wm * WM + i * 32 + r;
-            xr[i] = x + (m < a.m ? m : a.m - 1) * a.k;
-        }
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) {
-            const int n = n0 + wn * WN + j * 32 + r;
-            wr[j] = w + static_cast<int64_t>(n < a.n ? n : a.n - 1) * a.k;
-        }
+                for (int v = 0; v < 16; ++v) {
+                    zero |= sum[i][j][v] == 0.0f;
+                    again |= sum[i][j][v] != 0.0f && split_sum_odd(sum[i][j][v], tile_low);
+                }
         const int k_end = min(a.k, (chunk0 + chunks) * 32);  // a multiple of 4, as chunk0 * 32 is
-        for (int k = chunk0 * 32 + h; k < k_end; k += 2)
+        if (__syncthreads_or(zero)) {
+            // Which rows and channels hold a zero; the fewer of them are looked through
+            // first: zeros of zero rows (or of zero weights) are what they should be.
+            uint32_t * flags = reinterpret_cast<uint32_t *>(smem);  // BM rows, then BN channels
+            for (int i = tid; i < (BM + BN) / 32; i += NT) flags[i] = 0u;
+            __syncthreads();
 #pragma unroll
             for (int i = 0; i < TI; ++i)
 #pragma unroll
-                for (int j = 0; j < TJ; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(wr[j][k], xr[i][k], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < TJ; ++j) {
+                    bool any = false;
+                    uint32_t channels = 0;
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const bool z = sum[i][j][v] == 0.0f;
+                        any |= z;
+                        const uint64_t lanes = __ballot(z);
+                        channels |= (static_cast<uint32_t>(lanes) ? 1u : 0u) << (8 * (v >> 2) + (v & 3));
+                        channels |= (lanes >> 32 ? 1u : 0u) << (8 * (v >> 2) + 4 + (v & 3));
+                    }
+                    const uint64_t rows = __ballot(any);
+                    if (lane == 0) {
+                        atomicOr(flags + (wm * WM) / 32 + i, static_cast<uint32_t>(rows | rows >> 32));
+                        atomicOr(flags + (BM + wn * WN) / 32 + j, channels);
+                    }
+                }
+            __syncthreads();
+            int in_x = 0, in_w = 0;
+            for (int i = 0; i < BM / 32; ++i) in_x += __popc(flags[i]);
+            for (int i = BM / 32; i < (BM + BN) / 32; ++i) in_w += __popc(flags[i]);
+            const int first = in_x <= in_w ? 0 : BM, count = in_x <= in_w ? BM : BN;
+            bool nonzero = false;
+            for (int i = 0; i < count; ++i) {
+                if (!(flags[(first + i) / 32] >> (i & 31) & 1u)) continue;
+                const float * p = first == 0 ? x + (p0 + (i < last_x ? i : last_x)) * a.k
+                                             : w + static_cast<int64_t>(n0 + (i < last_w ? i : last_w)) * a.k;
+                for (int k = chunk0 * 32 + tid * 4; k < k_end; k += NT * 4)
+                    nonzero |= max_abs(*reinterpret_cast<const float4 *>(p + k)) != 0.0f;
+            }
+            if (__syncthreads_or(nonzero))
+#pragma unroll 1
+                for (int i = 0; i < XI + WI; ++i) {
+                    const int m = row + RS * (i < XI ? i : i - XI);
+                    const float * p = i < XI ? x + (p0 + (m < last_x ? m : last_x)) * a.k
+                                             : w + static_cast<int64_t>(n0 + (m < last_w ? m : last_w)) * a.k;
+                    for (int k = chunk0 * 32 + piece * 4; k < k_end; k += 32)
+                        again |= split_small(*reinterpret_cast<const float4 *>(p + k));
+                }
+        }
+        if (__syncthreads_or(again)) {
+            // One 32 x 32 block at a time, its sums picked out and put back by number:
+            // with the blocks' loops written out one after the other registers spilled.
+#pragma unroll 1
+            for (int b = 0; b < TI * TJ; ++b) {
+                const int64_t m = p0 + wm * WM + b / TJ * 32 + r;
+                const int n = n0 + wn * WN + b % TJ * 32 + r;
+                const float * xr = x + (m < a.m ? m : a.m - 1) * a.k;
+                const float * wr = w + static_cast<int64_t>(n < a.n ? n : a.n - 1) * a.k;
+                f32x16 second = {};
+                float hi_x = 0.0f, hi_w = 0.0f;
+                bool small_x = false, small_w = false;
+                for (int k = chunk0 * 32 + 4 * h; k - 4 * h < k_end; k += 8) {
+                    float4 fx = make_float4(0.0f, 0.0f, 0.0f, 0.0f), fw = fx;
+                    if (k < k_end) {
+                        fx = *reinterpret_cast<const float4 *>(xr + k);
+                        fw = *reinterpret_cast<const float4 *>(wr + k);
+                    }
+                    hi_x = fmaxf(hi_x, max_abs(fx));
+                    hi_w = fmaxf(hi_w, max_abs(fw));
+                    small_x |= split_small(fx);
+                    small_w |= split_small(fw);
+                    second = __builtin_amdgcn_mfma_f32_32x32x2f32(fw.x, fx.x, second, 0, 0, 0);
+                    second = __builtin_amdgcn_mfma_f32_32x32x2f32(fw.y, fx.y, second, 0, 0, 0);
+                    second = __builtin_amdgcn_mfma_f32_32x32x2f32(fw.z, fx.z, second, 0, 0, 0);
+                    second = __builtin_amdgcn_mfma_f32_32x32x2f32(fw.w, fx.w, second, 0, 0, 0);
+                }
+                float block[16];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) block[v] = sum[0][0][v];
+#pragma unroll
+                for (int q = 1; q < TI * TJ; ++q)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) block[v] = q == b ? sum[q / TJ][q % TJ][v] : block[v];
+                split_select(block, second, hi_w, hi_x, small_w, small_x, a.k, h);
+#pragma unroll
+                for (int q = 0; q < TI * TJ; ++q)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) sum[q / TJ][q % TJ][v] = q == b ? block[v] : sum[q / TJ][q % TJ][v];
+            }
+        }
+        __syncthreads();  // the words in smem have been read
     }
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = sum[i][j][v];
     if constexpr (EPI == kDenseStore) {
         if (a.vec_out == 2) {
             // 32 rows of each wave's block at a time through the idle planes

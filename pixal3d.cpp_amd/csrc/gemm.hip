@@ -1989,28 +1989,94 @@ split_conv_f32_kernel(GemmArgs a) {
         step(even);
         if (s + 1 < steps) step(odd_step);
     }
-    f32x16 sum[1][1];
+    float sum[16];
+    const int terms = a.noff * a.cin;
     bool odd = hi > kSplitHigh;
+    const float low = split_low(kSplitHigh, terms);
+    // Outputs of this lane: rows 8 (v / 4) + v % 4 < live of channel n.
+    const int n = n0 + wn * 32 + r;
+    const int live = n < a.cout ? static_cast<int>(min<int64_t>(a.m - p0, BM)) - wm * 32 - 4 * h : 0;
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-        sum[0][0][v] = (lead[0][v] + lead[1][v]) + (rest[0][v] + rest[1][v]);
-        odd |= split_sum_odd(sum[0][0][v]);
+        sum[v] = (lead[0][v] + lead[1][v]) + (rest[0][v] + rest[1][v]);
+        odd |= 8 * (v >> 2) + (v & 3) < live && split_sum_odd(sum[v], low);
     }
-    if (__syncthreads_or(odd)) {
-        // rare: the tile again on the fp32 matrix instruction
+    if (__builtin_expect(__syncthreads_or(odd), 0)) {
+        hi = split_block_max(hi, &tile_mask);
+        const float tile_low = split_low(hi, terms);
+        bool again = hi > kSplitHigh, zero = false;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) sum[0][0][v] = 0.0f;
-        const int n = n0 + wn * 32 + r;
-        for (int i = 0; i < kcount; ++i) {
-            const int k = koff[i];
-            const int32_t src = idx_lds[k * BM + wm * 32 + r];
-            const float * xr = x + static_cast<int64_t>(src < 0 ? 0 : src) * a.ldx;
-            const float * wr = w + (static_cast<int64_t>(k) * a.cout + (n < a.cout ? n : 0)) * a.cin;
-            for (int c = h; c < a.cin; c += 2)  // cin is a multiple of 4
-                sum[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(src < 0 ? 0.0f : xr[c], wr[c], sum[0][0], 0, 0, 0);
+        for (int v = 0; v < 16; ++v) {
+            if (8 * (v >> 2) + (v & 3) >= live) continue;
+            zero |= sum[v] == 0.0f;
+            again |= sum[v] != 0.0f && split_sum_odd(sum[v], tile_low);
+        }
+        if (__syncthreads_or(zero)) {
+            // Zeros whose gathered rows are all zero are what they should be.
+            uint32_t * flags = reinterpret_cast<uint32_t *>(sx);  // BM rows
+            if (tid < BM / 32) flags[tid] = 0u;
+            __syncthreads();
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int at_row = 8 * (v >> 2) + (v & 3);
+                const uint64_t lanes = __ballot(at_row < live && sum[v] == 0.0f);
+                if (lane == 0)
+                    atomicOr(flags + wm, (static_cast<uint32_t>(lanes) ? 1u << at_row : 0u) |
+                                             (lanes >> 32 ? 16u << at_row : 0u));
+            }
+            __syncthreads();
+            bool nonzero = false;
+            for (int m = tid >> 4; m < BM; m += NT / 16) {
+                if (!(flags[m / 32] >> (m & 31) & 1u)) continue;
+#pragma unroll 4
+                for (int i = 0; i < kcount; ++i) {
+                    const int32_t src = idx_lds[koff[i] * BM + m];
+                    const float * xr = x + static_cast<int64_t>(src < 0 ? 0 : src) * a.ldx;
+                    for (int c = (tid & 15) * 4; c < (src >= 0 ? a.cin : 0); c += 64)
+                        nonzero |= max_abs(*reinterpret_cast<const float4 *>(xr + c)) != 0.0f;
+                }
+            }
+            if (__syncthreads_or(nonzero)) {
+                next = next_i = next_chunk = 0;
+                for (int s = 0; s < steps; ++s) {
+                    load(even);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) again |= split_small(even.x[q]) | split_small(even.w[q]);
+                }
+            }
+        }
+        if (__syncthreads_or(again)) {
+            f32x16 second = {};
+            float hi_x = 0.0f, hi_w = 0.0f;
+            bool small_x = false, small_w = false;
+            for (int i = 0; i < kcount; ++i) {
+                const int k = koff[i];
+                const int32_t src = idx_lds[k * BM + wm * 32 + r];
+                const float * xr = x + static_cast<int64_t>(src < 0 ? 0 : src) * a.ldx;
+                const float * wr = w + (static_cast<int64_t>(k) * a.cout + (n < a.cout ? n : 0)) * a.cin;
+                for (int c = 4 * h; c - 4 * h < a.cin; c += 8) {  // cin is a multiple of 4
+                    float4 fx = make_float4(0.0f, 0.0f, 0.0f, 0.0f), fw = fx;
+                    if (c < a.cin) {
+                        if (src >= 0) fx = *reinterpret_cast<const float4 *>(xr + c);
+                        fw = *reinterpret_cast<const float4 *>(wr + c);
+                    }
+                    hi_x = fmaxf(hi_x, max_abs(fx));
+                    hi_w = fmaxf(hi_w, max_abs(fw));
+                    small_x |= split_small(fx);
+                    small_w |= split_small(fw);
+                    second = __builtin_amdgcn_mfma_f32_32x32x2f32(fx.x, fw.x, second, 0, 0, 0);
+                    second = __builtin_amdgcn_mfma_f32_32x32x2f32(fx.y, fw.y, second, 0, 0, 0);
+                    second = __builtin_amdgcn_mfma_f32_32x32x2f32(fx.z, fw.z, second, 0, 0, 0);
+                    second = __builtin_amdgcn_mfma_f32_32x32x2f32(fx.w, fw.w, second, 0, 0, 0);
+                }
+            }
+            split_select(sum, second, hi_x, hi_w, small_x, small_w, terms, h);
         }
     }
-    gemm_epilogue<float, 1, 1, 32, 32, kEpiStore>(a, sum, p0, n0, wm, wn, h, r);
+    f32x16 out[1][1];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) out[0][0][v] = sum[v];
+    gemm_epilogue<float, 1, 1, 32, 32, kEpiStore>(a, out, p0, n0, wm, wn, h, r);
 }
 
 int launch_split_conv_f32(const GemmArgs & args, hipStream_t stream) {
