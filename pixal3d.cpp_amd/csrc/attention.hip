@@ -1287,11 +1287,11 @@ window_attn_bf16_kernel(AttnArgs a, int heads, int heads_per_group, int groups) 
 // once at the end.  Rows stay row-major, 16-byte pieces XOR-swizzled: f32_kswz
 // spreads the 16 key rows one 16-byte K read covers over all banks, f32_vswz
 // the two key rows (4 apart) one 4-byte V read covers.
-// Bound by the fp32 matrix cores and the softmax's vector work beside them:
-// 4,600 x 4,600 keys x 16 heads in 0.90 ms, 96 TFLOP/s (1.04 ms with 128
-// queries per workgroup and unsplit keys, whose 592 workgroups leave the CUs
-// 2 or 3 each; the generic kernel, which stages each tile through registers
-// with nothing in flight, took the block it is in from 2.50 to 2.85 ms).
+// Bound by a workgroup's chain of tiles: taken where 64-query workgroups do not fill
+// the CUs (f32_split_grid), 300 x 1,370 keys x 16 heads 61 us, 256 x 256 x 4 16 us
+// (the generic kernel stages each tile through registers with nothing in flight: 4,560
+// x 4,560 x 16 1,106 us where this one took 850), and for scales that
+// flash_attn_f32_split_kernel does not take.
 __device__ __forceinline__ int f32_kswz(int row) { return row & 15; }
 __device__ __forceinline__ int f32_vswz(int row) { return ((row >> 2) & 1) << 3; }
 

@@ -942,7 +942,8 @@ __device__ __forceinline__ void gemm_lds_tile(const GemmArgs & a, int logical, c
     constexpr bool kStageable =
         EPI == kEpiStore && sizeof(T) == 2 && BM * kStagedPitch <= lds_gemm_bytes<BM, BN, NSTAGE>(27);
     // (A 256 x 256 tile reaches into the source table of 27 offsets, which no
-    // wave reads any more.)
+    // wave reads any more: 768 -> 1536 at 33,220 rows 2,252 us against 2,298 stored
+    // two bytes at a time, at 29,704 rows 1,722 against 1,749.)
     const bool staged = kStageable && BM * kStagedPitch <= NSTAGE * kStageBytes + a.noff * BM * 4 &&
                         a.cout % 8 == 0 && a.ldy % 8 == 0 &&
                         (reinterpret_cast<uintptr_t>(a.y) & 15) == 0;
@@ -1689,7 +1690,7 @@ int launch_range_conv(const GemmArgs & args, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------
-// fp32 split-K gather GEMM (SubMConv3d and linears in fp32).  A workgroup
+// fp32 split-K gather GEMM (SubMConv3d and stride-2 convolutions in fp32).  A workgroup
 // owns 32 TI output rows x 32 CT output channels; its (offset, 32-channel chunk)
 // steps are dealt round-robin to its 4 waves, so even a few hundred tiles
 // keep every CU busy.  Each wave loads its operands straight into VGPRs --
@@ -1702,7 +1703,7 @@ int launch_range_conv(const GemmArgs & args, hipStream_t stream) {
 // path, which bounds the kernel: TI = 2 reads each weight chunk once for 64
 // rows instead of 32.
 
-template <int EPI, int TI, int CT>
+template <int TI, int CT>
 __global__ void __launch_bounds__(256)
 split_gemm_f32_kernel(GemmArgs a) {
     constexpr int NW = 4, BM = 32 * TI, BN = 32 * CT;
@@ -1855,7 +1856,7 @@ split_gemm_f32_kernel(GemmArgs a) {
             for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
                 for (int v = 0; v < 16; ++v) acc[ti][ct][v] += red[wv][ti * CT + ct][v][lane];
-    gemm_epilogue<float, TI, CT, 32 * TI, BN, EPI>(a, acc, p0, n0, 0, 0, h, r);
+    gemm_epilogue<float, TI, CT, 32 * TI, BN, kEpiStore>(a, acc, p0, n0, 0, 0, h, r);
 }
 
 #ifndef PXS_SPLIT_F32
@@ -2086,39 +2087,40 @@ int launch_split_conv_f32(const GemmArgs & args, hipStream_t stream) {
     return check_launch("SubMConv3d (fp32 split)");
 }
 
-template <int EPI, int TI, int CT>
+template <int TI, int CT>
 int launch_split_f32_tile(const GemmArgs & args, hipStream_t stream) {
     const int64_t tiles_m = (args.m + 32 * TI - 1) / (32 * TI);
     const int64_t tiles_n = (args.cout + 32 * CT - 1) / (32 * CT);
     const int64_t blocks = tiles_m * tiles_n;
     if (blocks > INT32_MAX) return fail(PXS_ERR_ARG, "gather GEMM grid too large");
-    hipLaunchKernelGGL((split_gemm_f32_kernel<EPI, TI, CT>), dim3(static_cast<unsigned>(blocks)),
+    hipLaunchKernelGGL((split_gemm_f32_kernel<TI, CT>), dim3(static_cast<unsigned>(blocks)),
                        dim3(256), 0, stream, args);
     return check_launch("gather GEMM (fp32 split-K)");
 }
 
-template <int EPI>
 int launch_split_f32(const GemmArgs & args, hipStream_t stream) {
-    if constexpr (EPI == kEpiStore) {  // convolutions have no other epilogue
-        const bool gather = (args.rowmap || args.grid) && args.noff >= 27;
-        // More 64 x 64 tiles than CUs: the split kernel.  Against this file's fp32
-        // tiles (the whole call over a grid, us): 64 -> 64 at 22,032 rows (345
-        // tiles) 83 against 103, 88,448 rows 227 against 277; 96 -> 192 at 8,912 rows
-        // (420) 115 against 137; 128 -> 128 at 8,912 rows (280) 148 against 166; 16 -> 36
-        // at 22,032 rows 46 against 69.  Errors against 64 bits are 0.45 to 0.65 of the
-        // fp32 tiles'.  One round of 224 to 256 tiles is done sooner on 64-row fp32 tiles
-        // (64 -> 64 at 16,184 rows, 253 tiles: 57 against 66), fewer on 32-row ones.
-        const int64_t squares = ((args.m + 63) / 64) * ((args.cout + 63) / 64);
-        if (gather && args.noff < 32 && squares > 256) return launch_split_conv_f32(args, stream);
-        if (gather && squares >= 224) return launch_split_f32_tile<EPI, 2, 2>(args, stream);
-        // Tiles of 32 columns where those still fit one per CU: a workgroup then
-        // takes in two thirds of the operand bytes (32 -> 48 at up to 2,900 rows 14.2
-        // against 20.8 us, 128 -> 128 at 1,592 rows 31 against 48; eight waves on the
-        // 64-column tile 24 and 56).
-        const int64_t narrow = ((args.m + 31) / 32) * ((args.cout + 31) / 32);
-        if (gather && narrow <= 256) return launch_split_f32_tile<EPI, 1, 1>(args, stream);
-    }
-    return launch_split_f32_tile<EPI, 1, 2>(args, stream);
+    const bool gather = (args.rowmap || args.grid) && args.noff >= 27;
+    // More 64 x 64 tiles than CUs: the split kernel.  Against this file's fp32
+    // tiles (the whole call over a grid, us): 64 -> 64 at 22,032 rows (345
+    // tiles) 83 against 103, 88,448 rows 227 against 277; 96 -> 192 at 8,912 rows
+    // (420) 115 against 137; 128 -> 128 at 8,912 rows (280) 148 against 166; 16 -> 36
+    // at 22,032 rows 46 against 69.  Errors against 64 bits are 0.45 to 0.65 of the
+    // fp32 tiles'.  One round of 224 to 256 tiles is done sooner on 64-row fp32 tiles
+    // (64 -> 64 at 16,184 rows, 253 tiles: 57 against 66), fewer on 32-row ones.
+    // Inputs wider than 128 channels in the third round of 256 tiles, and wider than
+    // 256 in the first four, would be done sooner on fp32 tiles too (256 -> 256 at 12,027
+    // rows 443 against 476, 512 -> 256 at 8,315 831 against 927, at 6,395 555 against 570), at
+    // twice the error (6.1e-7 against 2.9e-7): they stay here.
+    const int64_t squares = ((args.m + 63) / 64) * ((args.cout + 63) / 64);
+    if (gather && args.noff < 32 && squares > 256) return launch_split_conv_f32(args, stream);
+    if (gather && squares >= 224) return launch_split_f32_tile<2, 2>(args, stream);
+    // Tiles of 32 columns where those still fit one per CU: a workgroup then
+    // takes in two thirds of the operand bytes (32 -> 48 at up to 2,900 rows 14.2
+    // against 20.8 us, 128 -> 128 at 1,592 rows 31 against 48; eight waves on the
+    // 64-column tile 24 and 56).
+    const int64_t narrow = ((args.m + 31) / 32) * ((args.cout + 31) / 32);
+    if (gather && narrow <= 256) return launch_split_f32_tile<1, 1>(args, stream);
+    return launch_split_f32_tile<1, 2>(args, stream);
 }
 
 template <typename T, int BM, int BN, int EPI, int NSTAGE, int NW, int WAVES_M, int KSPLIT>
@@ -2231,9 +2233,12 @@ int dispatch(const GemmArgs & args, hipStream_t stream) {
             // Short ones (the 8-offset stride-2 conv, 16 K stages) lose 6%:
             // with one workgroup per CU nothing hides a tile's prologue.
             const int64_t kstages = static_cast<int64_t>(args.noff) * ((args.cin + 63) / 64);
-            // (192-row tiles, which put SubMConv3d 256->256 on ~40k rows in
-            // one round of tiles instead of 1.2, measured the same: the
-            // chip-wide operand rate bounds it, not the last round.)
+            // One workgroup per CU: the last round of tiles counts.  192-row tiles
+            // of 8 waves take fewer rounds at some sizes (rows in two layers, us, 128-
+            // against 192-row tiles: 256 -> 256 at 39,000 rows, 305 and 204 tiles, 226 /
+            // 151; 512 -> 512 at 21,000, 330 and 220, 429 / 291; 1024 -> 1024 at 10,480,
+            // 328 and 220, 840 / 591) and more time where both take as many (256 -> 256
+            // at 8,900, 70 and 47, 112 / 150); child_conv chooses between them.
             // Long gathers of at least 512 output channels, with two or more
             // rounds of 256x256 tiles: each stage's 64 KB feed 2x the MACs
             // of a 128x256 stage's 48 KB (one workgroup per CU either way;
@@ -2300,11 +2305,10 @@ int run_gemm(int dtype, GemmArgs & args, int epi, hipStream_t stream) {
     const int vec = dtype == PXS_BF16 ? 8 : 4;
     args.vec_ok = (args.cin % vec == 0) && (args.ldx % vec == 0) && aligned16(args.x) &&
                   aligned16(args.w);
-    if (dtype == PXS_F32 && args.vec_ok && PXS_SPLIT_F32 && args.m > 0 && args.cout > 0 &&
-        args.noff <= 32 && (args.ldx % 4 == 0)) {
-        if (epi == kEpiStore) return launch_split_f32<kEpiStore>(args, stream);
-        if (epi == kEpiAddResidual) return launch_split_f32<kEpiAddResidual>(args, stream);
-        return launch_split_f32<kEpiGateResidual>(args, stream);
+    // (Plain fp32 linears of whole 16-byte pieces run in csrc/dense.hip.)
+    if (dtype == PXS_F32 && epi == kEpiStore && args.vec_ok && PXS_SPLIT_F32 && args.m > 0 &&
+        args.cout > 0 && args.noff <= 32 && (args.ldx % 4 == 0)) {
+        return launch_split_f32(args, stream);
     }
     if (dtype == PXS_BF16) {
         // SubMConv3d over a voxel grid: neighbourhood ranges, 128-column
