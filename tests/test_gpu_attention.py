@@ -124,6 +124,34 @@ def test_attention_fp32_split_range(px, what):
     assert float((o - ref).abs()[ok].max() / ref.abs()[ok].max()) <= 1e-5
 
 
+# The fp32 kernels with a segment table: more than 64 segments, or more than 2,048
+# workgroups; on split operands, and (scales above 2^41) on the fp32 instruction.
+@pytest.mark.parametrize("heads,lens,big", [(2, [256 + 3 * i for i in range(65)], False), (16, [8600, 8100], False),
+                                            (2, [257] * 65, True), (16, [8600, 8100], True)])
+def test_attention_fp32_segment_table(px, heads, lens, big):
+    dev = torch.device("cuda:0")
+    g = torch.Generator(device=dev).manual_seed(len(lens) + heads)
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    n = int(cu[-1])
+    q, k, v = (torch.randn(n, heads * 64, generator=g, device=dev) for _ in range(3))
+    scale = 2.0 ** 43 if big else 0.125
+    if big:
+        q *= 2.0 ** -46
+    print(f"[attn fp32 table] heads={heads} segments={len(lens)} scale={scale:g}", flush=True)
+    b = torch.tensor(cu, dtype=torch.int64, device=dev)
+    o = px.varlen_attention(q, k, v, b, b, heads, 64, scale)
+    for s in sorted({0, 1, len(lens) // 2, len(lens) - 1}):
+        rows = torch.arange(int(cu[s]), int(cu[s + 1]), device=dev)
+        some = torch.unique(torch.cat([rows[:3], rows[-3:], rows[::97]]))
+        for h in sorted({0, heads - 1}):
+            c = slice(64 * h, 64 * h + 64)
+            p = torch.softmax(q[some][:, c].double() @ k[rows][:, c].double().t().contiguous() * scale, 1)
+            ref = p @ v[rows][:, c].double()
+            err = float((o[some][:, c] - ref).norm() / ref.norm())
+            print(f"[attn fp32 table] segment {s} head {h} relative L2 {err:.2e}", flush=True)
+            assert err <= 3e-6, (s, h, err)
+
+
 # Up to 64 segments the kernels find a tile's segment themselves, more take a
 # table: counts on both sides, with empty segments first, last and between.
 @pytest.mark.parametrize("nseg", [2, 63, 64, 65])

@@ -189,3 +189,64 @@ def test_block_residual_linears_split_over_k(px, orc, C, rows, M, PC):
     ref = orc.transformer_block(coords, 2, x, tmod, ctx, off, [C, H, M, CC, PC, 1, 1, 1, int(PC > 0)],
                                 [1e-6, 1.0, 10000.0], ws, projected=proj)
     assert_fp32(host(hidden), ref, what="block split")
+
+
+# Rows on both sides of the one-pass line (104 tiles of 128 x 128), ragged ones,
+# and each split count (4, 3, 2 at width 256: 48, 64 and 104 tiles).
+@pytest.mark.parametrize("C,rows,M,PC", [(1024, 130, 1024, 0), (256, 1, 1024, 1024), (256, 3000, 1024, 0),
+                                         (256, 4096, 1024, 1024), (256, 6656, 1024, 0), (256, 6657, 1024, 0),
+                                         (512, 700, 2048, 2048)])
+@pytest.mark.parametrize("part", ["self", "cross", "projection", "mlp"])
+def test_block_bf16_residual_linears_split_over_k(px, C, rows, M, PC, part):
+    """One residual linear of a bf16 block at a time (the others' weights zero),
+    against the block made of single ops, whose linears run in one pass: the
+    fp32 update differs by the order of its sums only."""
+    if part == "projection" and not PC:
+        pytest.skip("no projection in this block")
+    H, T, bf = C // 64, 12, torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(rows + C)
+    rand = lambda *s, std=1.0: torch.randn(*s, device="cuda", generator=g) * std  # noqa: E731
+    i = torch.arange(rows, device="cuda")
+    batch = 2 if rows > 1 else 1
+    c = torch.stack([i * batch // rows, i // 256, i // 16 % 16, i % 16], 1).to(torch.int32)
+    cu = px.batch_cu_seqlens(c, batch)
+    sizes = [6 * C, 3 * C * C, 3 * C, C, C, C * C, C, C, C, C * C, C, 2 * C * C, 2 * C, C, C, C * C, C,
+             C * PC, C if PC else 0, M * C, M, C * M, C]
+    ws = [rand(n, std=0.03) if n else None for n in sizes]
+    for k in (3, 4, 7, 13, 14):
+        ws[k] = ws[k] + 1.0
+    for name, (wi, bi) in {"self": (5, 6), "cross": (15, 16), "projection": (17, 18), "mlp": (21, 22)}.items():
+        if name != part and ws[wi] is not None:
+            ws[wi], ws[bi] = ws[wi] * 0, ws[bi] * 0
+    ws = [w.to(bf) if w is not None and k in pxs.BLOCK_LINEAR_WEIGHTS else w for k, w in enumerate(ws)]
+    x, tm = rand(rows, C), rand(batch, 6 * C, std=0.3)
+    ctx, off = rand(batch * T, C).to(bf), ti64(np.arange(batch + 1) * T)
+    proj = rand(rows, PC).to(bf) if PC else None
+    print(f"[block bf16 split] rows={rows} C={C} M={M} PC={PC} {part}", flush=True)
+    got = x.clone()
+    px.transformer_block(block_cfg(C, H, M, C, PC, PC > 0), pxs.block_weights(ws), c, batch, cu, got, tm,
+                         ctx, off, projected=proj)
+    ref, w2 = x.clone(), lambda k, n: ws[k].view(n, -1)  # noqa: E731
+    if part == "self":
+        xm = px.layer_norm_modulate(ref, 1e-6, c, ws[0], tm, 0, out_dtype=bf)
+        q, k, v = px.qkv_prepare(px.linear(xm, w2(1, 3 * C), ws[2]), H, 64, ws[3], ws[4], c)
+        att = px.varlen_attention(q, k, v, cu, cu, H, 64, 0.125)
+        px.linear_gate_residual(att, w2(5, C), ws[6], c, ws[0], tm, 2 * C, ref)
+    elif part == "cross":
+        xm = px.layer_norm(ref, 1e-6, ws[7], ws[8], out_dtype=bf)
+        q = px.mh_rms_norm(px.linear(xm, w2(9, C), ws[10]), H, 64, ws[13])
+        kv = px.linear(ctx, w2(11, 2 * C), ws[12])
+        k = px.mh_rms_norm(kv[:, :C].contiguous(), H, 64, ws[14])
+        att = px.varlen_attention(q, k, kv[:, C:].contiguous(), cu, off, H, 64, 0.125)
+        px.linear_residual(att, w2(15, C), ws[16], ref)
+    elif part == "projection":
+        px.linear_residual(proj, w2(17, C), ws[18], ref)
+    else:
+        xm = px.layer_norm_modulate(ref, 1e-6, c, ws[0], tm, 3 * C, out_dtype=bf)
+        px.linear_gate_residual(px.linear(xm, w2(19, M), ws[20], act=1), w2(21, C), ws[22], c, ws[0], tm,
+                                5 * C, ref)
+    err = float((got - ref).norm() / (ref - x).norm())
+    print(f"[block bf16 split] relative L2 of the update {err:.2e}", flush=True)
+    # sums of K products in other orders, and the update's rounding at the residual's
+    # size: a few 2^-24 each
+    assert err <= 2e-6

@@ -163,6 +163,29 @@ def test_layer_norm_row_layouts(px, orc, channels, xd, yd):
         check(y, orc.layer_norm(xr, eps, gamma, beta), what=f"ln {channels} {xd}->{yd}")
 
 
+@pytest.mark.parametrize("xd,channels", [("f32", 384), ("bf16", 1536)])
+@pytest.mark.parametrize("yd", ["f32", "bf16"])
+@pytest.mark.parametrize("rows", [1, 1237])
+def test_layer_norm_three_vectors_of_other_widths(px, orc, xd, channels, yd, rows):
+    """The widths that the other dtype's 96 and 192 vectors also make: 384 fp32
+    channels on 32 lanes, 1,536 bf16 channels on 64."""
+    import torch
+    x = (W.normal(59, rows * channels, 1) * 2 - 0.3).reshape(rows, channels)
+    g, b = W.normal(59, channels, 2), W.normal(59, channels, 3)
+    conv = t32 if xd == "f32" else tbf
+    xr = x if xd == "f32" else W.bf16_round(x)
+    out = torch.float32 if yd == "f32" else torch.bfloat16
+    check = assert_fp32 if yd == "f32" else assert_bf16
+    y = host(px.layer_norm(conv(x), 1e-6, t32(g), t32(b), out_dtype=out))
+    check(y, orc.layer_norm(xr, 1e-6, g, b), what=f"ln {channels} {xd}->{yd}")
+    coords = np.zeros((rows, 4), np.int32)
+    coords[rows // 2:, 0] = 1
+    bmod, tmod = W.normal(59, 6 * channels, 4, std=0.1), W.normal(59, 2 * 6 * channels, 5, std=0.1)
+    y = host(px.layer_norm_modulate(conv(x), 1e-6, ti32(coords), t32(bmod), t32(tmod), 3 * channels, out_dtype=out))
+    check(y, orc.modulate(coords, orc.layer_norm(xr, 1e-6), bmod, tmod, 3 * channels),
+          what=f"ln mod {channels} {xd}->{yd}")
+
+
 @pytest.mark.parametrize("rows", [1, 7, 1237])
 @pytest.mark.parametrize("xd,yd", [("f32", "f32"), ("bf16", "bf16"), ("f32", "bf16"), ("bf16", "f32")])
 def test_layer_norm_three_vectors_a_lane(px, orc, rows, xd, yd):

@@ -16,7 +16,7 @@ import torch
 
 import oracle as O
 import pxs
-from gpu_common import FP32_TOL, host, max_rel, t32, ti32, ti64
+from gpu_common import FP32_TOL, host, max_rel, random_flow, t32, ti32, ti64
 from test_gpu_block import device_weights
 from test_oracle import SAMPLER_CASES, sampler_inputs
 
@@ -162,21 +162,8 @@ def test_device_sampler_equals_separate_forwards_at_size(px, name):
     coords = ti32(np.stack([np.repeat(np.arange(batch), items), idx // 1024, idx // 32 % 32, idx % 32], 1))
     cu = px.batch_cu_seqlens(coords, batch)
     gen = torch.Generator(device="cuda").manual_seed(17)
-    rand = lambda *s, std=1.0: torch.randn(*s, device="cuda", generator=gen) * std  # noqa: E731
-    cfg = pxs.FlowConfig(lat, lat, ch, ch, nb, ch // 64, 0, 4 * ch, 1e-6, 1.0, 10000.0, 1, 1, 0)
-    fw = [rand(ch, lat, std=0.2), rand(ch), rand(ch, 256, std=0.02), rand(ch), rand(ch, ch, std=0.02),
-          rand(ch), rand(6 * ch, ch, std=0.02), rand(6 * ch, std=0.1), rand(lat, ch, std=0.03), rand(lat)]
-    sizes = [6 * ch, 3 * ch * ch, 3 * ch, ch, ch, ch * ch, ch, ch, ch, ch * ch, ch, 2 * ch * ch, 2 * ch,
-             ch, ch, ch * ch, ch, 0, 0, 4 * ch * ch, 4 * ch, 4 * ch * ch, ch]
-    blocks = []
-    for _ in range(nb):
-        ws = [rand(n, std=0.03) if n else None for n in sizes]
-        for i in (3, 4, 7, 13, 14):
-            ws[i] = ws[i] + 1.0
-        blocks.append([w.to(dtype) if w is not None and i in pxs.BLOCK_LINEAR_WEIGHTS else w
-                       for i, w in enumerate(ws)])
-    arr = (pxs.BlockWeights * nb)(*[pxs.block_weights(b) for b in blocks])
-    weights = pxs.FlowWeights(*[a.data_ptr() for a in fw], arr)
+    rand = lambda *s: torch.randn(*s, device="cuda", generator=gen)  # noqa: E731
+    cfg, weights, tensors, keep = random_flow(dtype, ch, nb, lat, 18)
     ctx, unc = rand(batch * cond_tokens, ch).to(dtype), rand(batch * unc_tokens, ch).to(dtype)
     ctx_off = ti64(np.arange(batch + 1) * cond_tokens)
     unc_off = ti64(np.arange(batch + 1) * unc_tokens)
@@ -197,6 +184,30 @@ def test_device_sampler_equals_separate_forwards_at_size(px, name):
     assert guided == [True, True, False]
     assert torch.isfinite(state).all()
     assert torch.equal(got, state), f"{name}: max difference {(got - state).abs().max().item():.3e}"
+
+
+@pytest.mark.parametrize("blocks,tokens", [(2, 130), (32, 7), (33, 131)])
+def test_context_ahead_of_the_blocks(px, blocks, tokens):
+    """The context keys and values of all blocks in one launch per 32 blocks
+    give the forward's bits of a launch per block, which a key bias off its 16
+    bytes asks for; every block has weights of its own."""
+    ch, rows = 256, 140
+    cfg, weights, tensors, keep = random_flow(torch.bfloat16, ch, blocks, 16, blocks)
+    i = torch.arange(rows, device="cuda")
+    coords = torch.stack([0 * i, i // 64, i // 8 % 8, i % 8], 1).to(torch.int32)
+    cu = px.batch_cu_seqlens(coords, 1)
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    x, t = torch.randn(rows, 16, device="cuda", generator=g), torch.full((1,), 500.0, device="cuda")
+    ctx = torch.randn(tokens, ch, device="cuda", generator=g).to(torch.bfloat16)
+    off = ti64(np.array([0, tokens]))
+    print(f"[context ahead] {blocks} blocks, {tokens} tokens", flush=True)
+    ahead = px.slat_flow_forward(cfg, weights, coords, 1, cu, x, t, ctx, off)
+    odd = torch.empty(2 * ch + 1, device="cuda")[1:]
+    odd.copy_(tensors[blocks - 1][12])
+    tensors[blocks - 1][12] = odd
+    arr = (pxs.BlockWeights * blocks)(*[pxs.block_weights(b) for b in tensors])
+    single = pxs.FlowWeights(*[a.data_ptr() for a in keep[0]], arr)
+    assert torch.equal(px.slat_flow_forward(cfg, single, coords, 1, cu, x, t, ctx, off), ahead)
 
 
 def test_device_sampler_matches_oracle(px, orc):

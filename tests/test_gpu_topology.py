@@ -227,6 +227,22 @@ def test_window_partition_unsorted_rows(px, orc, window, shift):
     np.testing.assert_array_equal(cu.cpu().numpy(), rcu)
 
 
+@pytest.mark.parametrize("window", [8, 10, 12])
+def test_window_partition_full_windows(px, orc, window):
+    """A filled 24^3 grid in random row order: windows of 512, 1,000 and 1,728
+    rows, whose ranks are taken two and four rows a thread and in chunks."""
+    coords = np.stack(np.meshgrid([0], *[np.arange(24)] * 3, indexing="ij"), -1).reshape(-1, 4)
+    coords = coords[np.random.default_rng(window).permutation(coords.shape[0])].astype(np.int32)
+    print(f"[window_partition full] window={window}", flush=True)
+    for shift in (0, window // 2):
+        fwd, bwd, cu, nwin = px.window_partition(ti32(coords), 1, (24, 24, 24), window, shift)
+        rfwd, rbwd, rcu = orc.window_partition(coords, (24, 24, 24), window, shift)
+        assert nwin == len(rcu) - 1
+        np.testing.assert_array_equal(fwd.cpu().numpy(), rfwd)
+        np.testing.assert_array_equal(bwd.cpu().numpy(), rbwd)
+        np.testing.assert_array_equal(cu.cpu().numpy(), rcu)
+
+
 def test_window_partition_padded_segments(px, orc):
     """Without reading the window count, cu_seqlens up to min(n, windows) ends
     in empty segments, and attention over that bound equals attention over
