@@ -1762,12 +1762,31 @@ flash_attn_f32_split_kernel(AttnArgs a, int heads, int64_t tiles_bound) {
                 zero |= oacc[dt][v] == 0.0f;
                 again |= oacc[dt][v] != 0.0f && split_sum_odd(oacc[dt][v], tile_low);
             }
-        if (__syncthreads_or(zero))
-            for (int j = 0; j < ntiles; ++j) {
-                load(j);
+        if (__syncthreads_or(zero)) {
+            // Small values in the dims that hold a zero, 4 dims at a time over all threads.
+            uint32_t * flags = reinterpret_cast<uint32_t *>(v_lds);
+            if (tid < 2) flags[tid] = 0u;
+            __syncthreads();
 #pragma unroll
-                for (int i = 0; i < 4; ++i) again |= split_small(vr[i]);
+            for (int dt = 0; dt < 2; ++dt) {
+                uint32_t dims = 0;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const uint64_t lanes = __ballot(oacc[dt][v] == 0.0f);
+                    dims |= (static_cast<uint32_t>(lanes) ? 1u : 0u) << (8 * (v >> 2) + (v & 3));
+                    dims |= (lanes >> 32 ? 1u : 0u) << (8 * (v >> 2) + 4 + (v & 3));
+                }
+                if (lane == 0) atomicOr(flags + dt, dims);
             }
+            __syncthreads();
+#pragma unroll 1
+            for (int d = 0; d < 64; d += 4) {
+                if (!(flags[d / 32] >> (d & 31) & 15u)) continue;
+#pragma unroll 4
+                for (int64_t key = k_begin + tid; key < k_end; key += 256)
+                    again |= split_small(*reinterpret_cast<const float4 *>(vp + key * a.ldv + d));
+            }
+        }
         if (__syncthreads_or(again)) {
             f32x4 qv[8];
 #pragma unroll

@@ -625,8 +625,9 @@ dense_split_kernel(DenseArgs a) {
                 }
         const int k_end = min(a.k, (chunk0 + chunks) * 32);  // a multiple of 4, as chunk0 * 32 is
         if (__syncthreads_or(zero)) {
-            // Which rows and channels hold a zero; the fewer of them are looked through
-            // first: zeros of zero rows (or of zero weights) are what they should be.
+            // Zeros of zero rows, or of zero channels, are what they should be, and of the
+            // others (of sums that cancel, about one output in 2^28) those without small operands.
+            // So only the rows and channels that hold a zero are looked through.
             uint32_t * flags = reinterpret_cast<uint32_t *>(smem);  // BM rows, then BN channels
             for (int i = tid; i < (BM + BN) / 32; i += NT) flags[i] = 0u;
             __syncthreads();
@@ -654,24 +655,58 @@ dense_split_kernel(DenseArgs a) {
             int in_x = 0, in_w = 0;
             for (int i = 0; i < BM / 32; ++i) in_x += __popc(flags[i]);
             for (int i = BM / 32; i < (BM + BN) / 32; ++i) in_w += __popc(flags[i]);
-            const int first = in_x <= in_w ? 0 : BM, count = in_x <= in_w ? BM : BN;
-            bool nonzero = false;
-            for (int i = 0; i < count; ++i) {
-                if (!(flags[(first + i) / 32] >> (i & 31) & 1u)) continue;
-                const float * p = first == 0 ? x + (p0 + (i < last_x ? i : last_x)) * a.k
-                                             : w + static_cast<int64_t>(n0 + (i < last_w ? i : last_w)) * a.k;
-                for (int k = chunk0 * 32 + tid * 4; k < k_end; k += NT * 4)
-                    nonzero |= max_abs(*reinterpret_cast<const float4 *>(p + k)) != 0.0f;
-            }
-            if (__syncthreads_or(nonzero))
-#pragma unroll 1
-                for (int i = 0; i < XI + WI; ++i) {
-                    const int m = row + RS * (i < XI ? i : i - XI);
-                    const float * p = i < XI ? x + (p0 + (m < last_x ? m : last_x)) * a.k
-                                             : w + static_cast<int64_t>(n0 + (m < last_w ? m : last_w)) * a.k;
-                    for (int k = chunk0 * 32 + piece * 4; k < k_end; k += 32)
-                        again |= split_small(*reinterpret_cast<const float4 *>(p + k));
+            // The marked lines of X or W: whether one is not all zero, whether one holds a
+            // small operand.  Few lines: each over all threads; many: 256 inputs of all lines
+            // at a time, and with `first` only up to the first operand that is not zero.
+            auto look = [&](bool of_x, bool few, bool first, bool & nonzero, bool & small) {
+                const int base = of_x ? 0 : BM, count = of_x ? BM : BN;
+                auto line = [&](int i) -> const float * {
+                    return of_x ? x + (p0 + (i < last_x ? i : last_x)) * a.k
+                                : w + static_cast<int64_t>(n0 + (i < last_w ? i : last_w)) * a.k;
+                };
+                auto marked = [&](int i) { return (flags[(base + i) / 32] >> (i & 31) & 1u) != 0; };
+                if (few) {
+                    for (int i0 = 0; i0 < count; i0 += 32)
+                        for (uint32_t left = flags[(base + i0) / 32]; left != 0; left &= left - 1) {
+                            const float * p = line(i0 + __ffs(left) - 1);
+                            for (int k = chunk0 * 32 + tid * 4; k < k_end; k += NT * 4) {
+                                const float4 f = *reinterpret_cast<const float4 *>(p + k);
+                                nonzero |= max_abs(f) != 0.0f;
+                                small |= split_small(f);
+                            }
+                        }
+                    return;
                 }
+                for (int k0 = chunk0 * 32; k0 < k_end; k0 += 256) {
+                    for (int i = row; i < count; i += RS) {
+                        if (!marked(i)) continue;
+                        const float * p = line(i);
+#pragma unroll 4
+                        for (int k = k0 + piece * 4; k < min(k0 + 256, k_end); k += 32) {
+                            const float4 f = *reinterpret_cast<const float4 *>(p + k);
+                            nonzero |= max_abs(f) != 0.0f;
+                            small |= split_small(f);
+                        }
+                    }
+                    if (first && __syncthreads_or(nonzero)) return;
+                }
+            };
+            const bool few_x = in_x <= 16, few_w = in_w <= 16;
+            bool clean = false, small = false;
+#pragma unroll 1
+            for (int pass = 0; pass < 2 && !clean; ++pass) {
+                const bool of_x = (in_x <= in_w) == (pass == 0);
+                bool nonzero = false, found = false;
+                look(of_x, of_x ? few_x : few_w, true, nonzero, found);
+                clean = !__syncthreads_or(nonzero);
+                small |= found;
+            }
+            if (!clean) {
+                bool unused = false;
+                if (!few_x) look(true, false, false, unused, small);
+                if (!few_w) look(false, false, false, unused, small);
+                again |= small;
+            }
         }
         if (__syncthreads_or(again)) {
             // One 32 x 32 block at a time, its sums picked out and put back by number:

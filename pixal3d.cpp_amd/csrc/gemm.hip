@@ -2013,36 +2013,50 @@ split_conv_f32_kernel(GemmArgs a) {
             again |= sum[v] != 0.0f && split_sum_odd(sum[v], tile_low);
         }
         if (__syncthreads_or(zero)) {
-            // Zeros whose gathered rows are all zero are what they should be.
-            uint32_t * flags = reinterpret_cast<uint32_t *>(sx);  // BM rows
-            if (tid < BM / 32) flags[tid] = 0u;
+            // Zeros whose gathered rows are all zero are what they should be, and of the
+            // others those without small operands: the rows and channels that hold a zero
+            // are looked through.
+            uint32_t * flags = reinterpret_cast<uint32_t *>(sx);  // BM rows, BN channels
+            if (tid < (BM + BN) / 32) flags[tid] = 0u;
             __syncthreads();
+            bool any = false;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int at_row = 8 * (v >> 2) + (v & 3);
-                const uint64_t lanes = __ballot(at_row < live && sum[v] == 0.0f);
+                const bool z = at_row < live && sum[v] == 0.0f;
+                any |= z;
+                const uint64_t lanes = __ballot(z);
                 if (lane == 0)
                     atomicOr(flags + wm, (static_cast<uint32_t>(lanes) ? 1u << at_row : 0u) |
                                              (lanes >> 32 ? 16u << at_row : 0u));
             }
+            const uint64_t columns = __ballot(any);
+            if (lane == 0) atomicOr(flags + BM / 32 + wn, static_cast<uint32_t>(columns | columns >> 32));
             __syncthreads();
-            bool nonzero = false;
+            bool nonzero = false, small = false;
             for (int m = tid >> 4; m < BM; m += NT / 16) {
                 if (!(flags[m / 32] >> (m & 31) & 1u)) continue;
 #pragma unroll 4
                 for (int i = 0; i < kcount; ++i) {
                     const int32_t src = idx_lds[koff[i] * BM + m];
                     const float * xr = x + static_cast<int64_t>(src < 0 ? 0 : src) * a.ldx;
-                    for (int c = (tid & 15) * 4; c < (src >= 0 ? a.cin : 0); c += 64)
-                        nonzero |= max_abs(*reinterpret_cast<const float4 *>(xr + c)) != 0.0f;
+                    for (int c = (tid & 15) * 4; c < (src >= 0 ? a.cin : 0); c += 64) {
+                        const float4 f = *reinterpret_cast<const float4 *>(xr + c);
+                        nonzero |= max_abs(f) != 0.0f;
+                        small |= split_small(f);
+                    }
                 }
             }
             if (__syncthreads_or(nonzero)) {
-                next = next_i = next_chunk = 0;
-                for (int s = 0; s < steps; ++s) {
-                    load(even);
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) again |= split_small(even.x[q]) | split_small(even.w[q]);
+                again |= small;
+                for (int m = tid >> 4; m < BN; m += NT / 16) {
+                    if (!(flags[BM / 32 + m / 32] >> (m & 31) & 1u)) continue;
+#pragma unroll 4
+                    for (int i = 0; i < kcount; ++i) {
+                        const float * wr = w + (static_cast<int64_t>(koff[i]) * a.cout + n0 + m) * a.cin;
+                        for (int c = (tid & 15) * 4; c < a.cin; c += 64)
+                            again |= split_small(*reinterpret_cast<const float4 *>(wr + c));
+                    }
                 }
             }
         }

@@ -16,10 +16,11 @@
 // tiles pay for one comparison per sum with the bound of hi = 2^50; a tile with
 // smaller sums takes its own hi, and looks for small operands where sums are zero.
 // Measured, us, ordinary inputs first: linear 20,000 x 1024 -> 1024 242, scaled by
-// 1e-20 243, by 1e-26 (some sums near zero in most tiles) 699, an infinity in every
-// tile 987, a row of zeros in every tile 259; convolution of 30,000 rows 64 -> 64 80,
-// by 1e-20 86, an infinity in every tile 221, half the rows zero 110; attention of
-// 4,000 x 16 heads 369, values by 1e-20 370, an infinite value 1,795, zero columns 402.
+// 1e-20 243, by 1e-26 (some sums near zero in most tiles) 690, an infinity in every
+// tile 970, a row of zeros in every tile 253, zero weights 350; convolution of 30,000
+// rows 64 -> 64 80, by 1e-20 85, an infinity in every tile 220, half the rows zero 120;
+// attention of 4,000 x 16 heads 370, values by 1e-20 371, an infinite value 1,795, zero
+// columns 378.
 #pragma once
 
 #include "pxs_common.h"

@@ -273,3 +273,49 @@ def test_conv_rows_do_not_touch_each_other(px, what):
     y2 = px.subm_conv3d(x2, w, None, nbr, masks)
     far = ~(nbr == 5000).any(0)
     assert torch.equal(y2[far], y[far])
+
+
+# Zeros of zero rows, of zero channels, of both, and of operands so small that no
+# plane holds them; few zero rows (looked through by row) and few zero channels.
+@pytest.mark.parametrize("rows,k,n", [(700, 64, 130), (3000, 512, 260), (200, 36, 68)])
+@pytest.mark.parametrize("zero_rows,zero_channels", [(3, 0), (0, 3), (2, 2), (97, 1)])
+@pytest.mark.parametrize("tiny", [False, True])
+def test_linear_zeros(px, rows, k, n, zero_rows, zero_channels, tiny):
+    g = gen(rows + zero_rows)
+    x, w = normal(g, rows, k), normal(g, n, k)
+    if zero_rows:
+        x[::zero_rows + 7] = 0.0
+    if zero_channels:
+        w[::zero_channels + 5] = 0.0
+    if tiny:
+        x[11::50] = 2.0 ** -140
+        x[12::50] *= 2.0 ** -142
+        w[7::40] *= 2.0 ** -141
+    print(f"[split zeros] {rows}x{k}->{n} zero rows {zero_rows} channels {zero_channels} tiny {tiny}", flush=True)
+    y = px.linear(x, w).double()
+    ref = x.double() @ w.double().t()
+    room = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t()) + k * 2.0 ** -149
+    assert ((y - ref).abs() <= room).all()
+    assert (y[(x == 0).all(1)] == 0).all() and (y[:, (w == 0).all(1)] == 0).all()
+    if tiny:  # fp32 keeps them
+        assert (y[11::50].abs().sum(1) > 0).all()
+
+
+@pytest.mark.parametrize("tiny", [False, True])
+def test_conv_zeros(px, tiny):
+    n, c = 17000, 64
+    g = gen(5)
+    nbr, masks = px.neighbor_map(slab(n))
+    x, w = normal(g, n, c), normal(g, 27, c, c)
+    x[2000:6000] = 0.0
+    w[:, 9] = 0.0
+    if tiny:
+        x[3000:3400] = 2.0 ** -140
+    print(f"[split zeros] conv tiny {tiny}", flush=True)
+    y = px.subm_conv3d(x, w, None, nbr, masks).double()
+    rows = torch.arange(1500, 6500, 3, device="cuda")
+    ref, room = conv64(x, w, nbr, rows), conv64(x.abs(), w.abs(), nbr, rows)
+    assert ((y[rows] - ref).abs() <= 27 * c * (2.0 ** -24 * room + 2.0 ** -149)).all()
+    assert (y[:, 9] == 0).all() and (y[2600:2790] == 0).all()
+    if tiny:
+        assert (y[3200].abs().sum() > 0).item()
