@@ -1009,20 +1009,20 @@ int dense_linear_group(const void * x, int64_t rows, int cin, const void * const
 // 1,288 rows 1,632 against 1,500, 1,515, 1,508, 1,539; 2,600 rows (168 tiles) 2,118
 // against 2,037, 2,077, 2,202, 2,229; 4,064 rows (256 tiles) 2,503 against 2,522,
 // 2,698, 2,736, 2,863.
-// A guided step runs the rows of a call twice with the splits of the call alone
-// (Branches), so up to four splits come with a quarter and more of the CUs idle
-// and none past 104 tiles, where twice as many still gain from two.  Two guided
-// steps of four blocks of width 1024 with two splits against one pass: 1,600 rows
-// (104 tiles) 2,872 us against 2,964; 2,600 rows (168) 4,160 against 3,956, though
-// one forward alone takes 1,258 against 1,302.
-constexpr int64_t kSplitTiles = 104;
+// So up to 170 tiles, by the call alone.  A guided step runs the rows of a call twice
+// with the splits of one branch (Branches) where those of the doubled batch would
+// suit it better past 104 tiles: two guided steps of four blocks of width 1024, 1,600
+// rows (104 tiles) 2,870 us against 2,956 in one pass, 2,600 rows (168) 4,160 against
+// 3,956.  A line at 104 would cost one forward alone as much (2,100 rows 1,255 us
+// against 1,171).
+constexpr int64_t kSplitTiles = 170;
 int dense_splits(int dtype, int64_t rows, int cin, int cout) {
     const int vec = dtype == PXS_BF16 ? 8 : 4, chunk = 8 * vec;
     if (rows <= 0 || cin % vec != 0 || cout % 4 != 0 || cout <= 64) return 0;
     const int64_t tiles = ((rows + 127) / 128) * ((cout + 127) / 128);
     if (tiles > kSplitTiles) return 0;
     const int64_t most = std::min<int64_t>(4, cin / (4 * chunk));  // 4 stages of K each
-    const int64_t splits = std::min(most, std::max<int64_t>(2, 192 / tiles));
+    const int64_t splits = std::min(most, std::max<int64_t>(2, 256 / tiles));
     return splits >= 2 ? static_cast<int>(splits) : 0;
 }
 

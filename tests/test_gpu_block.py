@@ -191,10 +191,10 @@ def test_block_residual_linears_split_over_k(px, orc, C, rows, M, PC):
     assert_fp32(host(hidden), ref, what="block split")
 
 
-# Rows on both sides of the one-pass line (104 tiles of 128 x 128), ragged ones,
-# and each split count (4, 3, 2 at width 256: 48, 64 and 104 tiles).
+# Rows on both sides of the one-pass line (170 tiles of 128 x 128), ragged ones,
+# and each split count (4, 3, 2 at width 256: 48, 80 and 170 tiles).
 @pytest.mark.parametrize("C,rows,M,PC", [(1024, 130, 1024, 0), (256, 1, 1024, 1024), (256, 3000, 1024, 0),
-                                         (256, 4096, 1024, 1024), (256, 6656, 1024, 0), (256, 6657, 1024, 0),
+                                         (256, 5120, 1024, 1024), (256, 10880, 1024, 0), (256, 10881, 1024, 0),
                                          (512, 700, 2048, 2048)])
 @pytest.mark.parametrize("part", ["self", "cross", "projection", "mlp"])
 def test_block_bf16_residual_linears_split_over_k(px, C, rows, M, PC, part):

@@ -134,7 +134,7 @@ def test_device_sampler_batched_cfg_equals_separate_forwards(px):
 
 # Rows per item, and context tokens of the two branches; each crosses a line at
 # which a kernel that sums in another order is taken: the K splits of residual
-# linears (bf16 width 256 and 1024, fp32), one pass instead (10,000 rows), the
+# linears (bf16 width 256 and 1024, fp32), one pass instead (9,200 and 12,000 rows), the
 # fp32 attention of more workgroups than CUs (2,100 rows x 4 heads), the fp32
 # linears of up to 4 rows (3 items; 3 rows, 3 and 2 tokens), and the context
 # keys and values of all blocks ahead (4,600 rows).

@@ -54,7 +54,7 @@ def never_shrinks(sizes, what):
     assert worst[0] <= worst[1], f"{what}: {worst[0]} bytes, then {worst[1]} for a larger call"
 
 
-ROWS = sorted({1, 7, 100, *(k + d for k in (128, 1344, 1664, 2688, 3328, 4096, 6656, 8192, 10752, 21760, 43520)
+ROWS = sorted({1, 7, 100, *(k + d for k in (128, 1344, 1664, 2688, 3328, 4096, 6656, 10880, 8192, 10752, 21760, 43520)
                             for d in (-1, 0, 1))})
 
 
