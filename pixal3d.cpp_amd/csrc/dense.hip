@@ -1028,6 +1028,7 @@ int dense_splits(int dtype, int64_t rows, int cin, int cout) {
 
 int64_t dense_split_rows(int dtype, int64_t rows, int cin, int cout) {
     int64_t most = 0;
+    if (cout <= 0) return 0;  // (a size query takes any configuration)
     const int64_t row_tiles = std::min((rows + 127) / 128, kSplitTiles / ((cout + 127) / 128));
     for (int64_t t = 1; t <= row_tiles; ++t) {  // the splits depend on the row tiles only
         const int64_t r = std::min(rows, 128 * t);

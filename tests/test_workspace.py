@@ -88,3 +88,16 @@ def test_decoder_workspaces_serve_every_smaller_call():
                           "ConvNeXt block, growing rows")
             never_shrinks([LIB.pxs_resblock_c2s_workspace_bytes(dtype, r, ch, ch // 2) for r in ROWS],
                           "up-block, growing rows")
+
+
+def test_sizes_of_refused_configurations():
+    """A size query answers for configurations that the call then refuses."""
+    for ch in (0, -256):
+        cfg = flow_config(ch, 4, 2, 64)
+        block = pxs.BlockConfig(ch, 4, 256, 64, 0, 1e-6, 1.0, 10000.0, 1, 1, 1, 0)
+        for dtype in (pxs.PXS_BF16, pxs.PXS_F32):
+            for rows in (0, 100):
+                flow_bytes(dtype, cfg, rows, 10, 1)
+                LIB.pxs_transformer_block_workspace_bytes(dtype, C.byref(block), rows, 10, 1)
+    assert LIB.pxs_slat_flow_workspace_bytes(pxs.PXS_BF16, None, 100, 10, 1) == 0
+    assert LIB.pxs_transformer_block_workspace_bytes(pxs.PXS_BF16, None, 100, 10, 1) == 0
